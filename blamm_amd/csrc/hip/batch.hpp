@@ -186,18 +186,18 @@ bool dma_setup(DmaReadback& d, const void* device_ptr)
 }
 
 // Gathered fragments per column block of a batch (uint4 elements of frag_a,
-// and of frag_b in the split-BF16 forms).
-size_t batch_frag_elems(bool bf)
+// and of frag_b in the split-BF16 form).
+size_t batch_frag_elems(int precision)
 {
-    return bf ? (size_t)kMaxChunks * 64 : (size_t)kMaxLen * 16;
+    return prec_screen(precision) ? kScreenBlock / 2 : prec_bf(precision) ? (size_t)kMaxChunks * 64 : (size_t)kMaxLen * 16;
 }
 
 // Device bytes of one column block of a batch: its fragments and the
 // per-slot threshold, slot map and band tables.
 uint64_t batch_block_bytes(const blamm_hip_ctx* c)
 {
-    const bool bf = prec_bf(c->precision);
-    return (bf ? 2 : 1) * batch_frag_elems(bf) * sizeof(uint4) + (uint64_t)c->cols_per_blk * (4 + 4 + 8 + 8);
+    return (c->precision == BLAMM_PREC_BF16X2_LO ? 2 : 1) * batch_frag_elems(c->precision) * sizeof(uint4) +
+           (uint64_t)c->cols_per_blk * (4 + 4 + 8 + 8);
 }
 
 // Host-written tables of a batch live in one device arena laid out like their
@@ -238,10 +238,11 @@ struct blamm_hip_batch {
     MetaView<uint32_t> groups;      // column groups (group_pack)
     MetaView<uint4> chunks;         // (t0, t1, request, 0)
     MetaView<uint64_t> runs;        // run starts of the batch stream
-    MetaView<uint2> items;          // (chunk, group), per XCD sub-queue
+    MetaView<uint2> items;          // (chunk, group), per queue
     // device-written
     DevBuf<uint4> frag_a, frag_b;   // gathered fragments (fp32 weights in frag_a)
     DevBuf<double> band, band_hi;   // per batch slot
+    DevBuf<double2> bound;          // per batch slot (screen)
     DevBuf<uint32_t> req_count;
     DevBuf<unsigned long long> req_off, cursor;
     DevBuf<uint4> cand;
@@ -341,6 +342,13 @@ int meta_fit(blamm_hip_batch* b, const size_t (&need)[kMetaTables])
     return BLAMM_OK;
 }
 
+// Workgroups of the batch's persistent filter.
+uint32_t batch_grid(const blamm_hip_batch* b, bool mask)
+{
+    const int wgs = persistent_wgs_per_cu(b->ctx->precision, mask, true);
+    return (uint32_t)b->ctx->num_cu * (uint32_t)std::max(1, wgs - (b->leave_room ? 1 : 0));
+}
+
 int batch_enqueue_kernels(blamm_hip_batch* b, bool mask, uint32_t grid)
 {
     blamm_hip_ctx* c = b->ctx;
@@ -366,37 +374,59 @@ int batch_enqueue_kernels(blamm_hip_batch* b, bool mask, uint32_t grid)
                        (const uint64_t*)b->runs.p, 0u, 0u, (const BatchDesc*)b->desc.p);
     HIP_TRY(hipGetLastError());
     // the batch's column blocks from the library's fragments
-    GatherArgs ga;
-    ga.desc = b->desc.p;
-    ga.slot_map = b->slot_map.p;
-    ga.lib_a = (const uint4*)c->frag_a.p;
-    ga.lib_b = (const uint4*)c->frag_b.p;
-    ga.lib_w = (const float*)c->frag_a.p;
-    ga.lib_band = c->slot_band_any.p;
-    ga.lib_band_hi = c->slot_band_hi_any.p;
-    ga.out_a = b->frag_a.p;
-    ga.out_b = b->frag_b.p;
-    ga.out_w = (float*)b->frag_a.p;
-    ga.out_band = b->band.p;
-    ga.out_band_hi = b->band_hi.p;
-    if (bf) hipLaunchKernelGGL(gather_kernel<true>, dim3((uint32_t)c->num_cu * 4), dim3(256), 0, b->stream, ga);
-    else hipLaunchKernelGGL(gather_kernel<false>, dim3((uint32_t)c->num_cu * 4), dim3(256), 0, b->stream, ga);
+    FilterArgs a{};
+    ScreenArgs sa{};
+    if (prec_screen(c->precision)) {
+        ScreenGatherArgs ga;
+        ga.desc = b->desc.p;
+        ga.slot_map = b->slot_map.p;
+        ga.lib_frag = c->screen_frag[mask ? 1 : 0].p;
+        ga.lib_bound = c->screen_bound[mask ? 1 : 0].p;
+        ga.out_frag = (uint2*)b->frag_a.p;
+        ga.out_bound = b->bound.p;
+        hipLaunchKernelGGL(screen_gather_kernel, dim3((uint32_t)c->num_cu * 4), dim3(256), 0, b->stream, ga);
+        sa.packed = b->packed.p;
+        sa.lcmask = mask ? b->lcmask.p : nullptr;
+        sa.frag = (const uint2*)b->frag_a.p;
+        sa.thr = b->thr.p;
+        sa.bound = b->bound.p;
+        sa.groups = b->groups.p;
+        sa.cand = b->cand.p;
+        sa.counters = b->counters.p;
+        sa.cand_cap = b->cand.n;
+    } else {
+        GatherArgs ga;
+        ga.desc = b->desc.p;
+        ga.slot_map = b->slot_map.p;
+        ga.lib_a = (const uint4*)c->frag_a.p;
+        ga.lib_b = (const uint4*)c->frag_b.p;
+        ga.lib_w = (const float*)c->frag_a.p;
+        ga.lib_band = c->slot_band_any.p;
+        ga.lib_band_hi = c->slot_band_hi_any.p;
+        ga.out_a = b->frag_a.p;
+        ga.out_b = b->frag_b.p;
+        ga.out_w = (float*)b->frag_a.p;
+        ga.out_band = b->band.p;
+        ga.out_band_hi = b->band_hi.p;
+        const dim3 gg((uint32_t)c->num_cu * 4);
+        if (bf) hipLaunchKernelGGL(gather_kernel<true>, gg, dim3(256), 0, b->stream, ga);
+        else hipLaunchKernelGGL(gather_kernel<false>, gg, dim3(256), 0, b->stream, ga);
+        a.packed = b->packed.p;
+        a.lcmask = mask ? b->lcmask.p : nullptr;
+        a.frag_a = b->frag_a.p;
+        a.frag_b = b->frag_b.p;
+        a.thr = b->thr.p;
+        a.band = b->band.p;
+        a.band_hi = b->band_hi.p;
+        a.groups = b->groups.p;
+        a.cand = b->cand.p;
+        a.counters = b->counters.p;
+        a.cand_cap = b->cand.n;
+    }
     HIP_TRY(hipGetLastError());
-    FilterArgs a;
-    a.packed = b->packed.p;
-    a.lcmask = mask ? b->lcmask.p : nullptr;
-    a.frag_a = b->frag_a.p;
-    a.frag_b = b->frag_b.p;
-    a.thr = b->thr.p;
-    a.band = b->band.p;
-    a.band_hi = b->band_hi.p;
-    a.groups = b->groups.p;
-    a.cand = b->cand.p;
-    a.counters = b->counters.p;
-    a.cand_cap = b->cand.n;
     const WorkQueue q{0, 0, 1, 1};
     const ListArgs l{b->desc.p, b->items.p, b->chunks.p};
-    hipError_t e = launch_filter(bf, prec_lo(c->precision), mask, true, a, q, l, grid, b->stream);
+    hipError_t e = launch_filter(c->precision, mask, true, sa, a, q, l, grid, b->stream);
     if (e != hipSuccess) return fail(BLAMM_ERR_DEVICE, std::string("batch filter launch: ") + hipGetErrorString(e));
     FinalizeArgs f = finalize_args(c, b->cand.p, b->cand.n, b->counters.p, b->packed.p, mask ? b->lcmask.p : nullptr,
                                    b->runs.p);
@@ -430,7 +460,7 @@ __global__ __launch_bounds__(256) void export_counts_kernel(const unsigned long 
                                                             const unsigned long long* req_off, uint32_t nreq,
                                                             unsigned long long* cnt_out, unsigned long long* off_out)
 {
-    for (uint32_t i = threadIdx.x; i < (uint32_t)kCntSlots; i += blockDim.x) cnt_out[i] = counters[i];
+    for (uint32_t i = threadIdx.x; i < (uint32_t)kCntStats; i += blockDim.x) cnt_out[i] = counters[i];
     for (uint32_t i = threadIdx.x; i <= nreq; i += blockDim.x) off_out[i] = req_off[i];
 }
 
@@ -443,9 +473,7 @@ int batch_launch(blamm_hip_batch* b)
     if (!b->exec[v] || b->exec_buf_gen[v] != b->buf_gen || b->exec_lib_gen[v] != c->lib_gen) {
         if (b->exec[v]) (void)hipGraphExecDestroy(b->exec[v]);
         b->exec[v] = nullptr;
-        const bool bf = prec_bf(c->precision);
-        const int wgs = persistent_wgs_per_cu(bf, prec_lo(c->precision), b->mask, true);
-        const uint32_t grid = (uint32_t)c->num_cu * (uint32_t)std::max(1, wgs - (b->leave_room ? 1 : 0));
+        const uint32_t grid = batch_grid(b, b->mask);
         HIP_TRY(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
         const int rc = batch_enqueue_kernels(b, b->mask, grid);
         hipGraph_t g = nullptr;
@@ -467,7 +495,7 @@ int batch_launch(blamm_hip_batch* b)
     HIP_TRY(hipEventRecord(b->ev_start, b->stream));
     HIP_TRY(hipGraphLaunch(b->exec[v], b->stream));
     HIP_TRY(hipEventRecord(b->ev_end, b->stream));
-    if (b->off_h.n < (size_t)b->nreq + 1 || b->req_off.n < (size_t)b->nreq + 1 || b->cnt_h.n < (size_t)kCntSlots)
+    if (b->off_h.n < (size_t)b->nreq + 1 || b->req_off.n < (size_t)b->nreq + 1 || b->cnt_h.n < (size_t)kCntStats)
         return fail(BLAMM_ERR_STATE, "batch launch: counter buffers smaller than the batch");
     hipLaunchKernelGGL(export_counts_kernel, dim3(1), dim3(256), 0, b->stream, b->counters.p, b->req_off.p, b->nreq,
                        b->cnt_h.p, b->off_h.p);
@@ -608,7 +636,7 @@ int blamm_hip_batch_create(blamm_hip_ctx* c, uint64_t max_bases, uint32_t max_re
     if (e == hipSuccess) e = hipEventCreateWithFlags(&b->ev_done, hipEventDisableTiming);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&b->ev_copy, hipEventDisableTiming);
     if (e == hipSuccess) e = b->counters.reserve(kCntSlots);
-    if (e == hipSuccess) e = b->cnt_h.reserve(kCntSlots);
+    if (e == hipSuccess) e = b->cnt_h.reserve(kCntStats);
     const uint64_t nb = std::min<uint64_t>(max_bases, kBatchMaxBases);
     const uint64_t nr = std::max<uint32_t>(max_requests, 1);
     if (e == hipSuccess) e = b->packed.reserve(nb / 32 + nr * 2 + 16);
@@ -635,7 +663,7 @@ int blamm_hip_batch_destroy(blamm_hip_batch* b)
     drop_graphs(b);
     b->packed.release(); b->lcmask.release(); b->run_bits.release(); b->meta.release();
     b->frag_a.release(); b->frag_b.release(); b->band.release();
-    b->band_hi.release();
+    b->band_hi.release(); b->bound.release();
     b->req_count.release(); b->req_off.release(); b->cursor.release();
     b->cand.release(); b->counters.release();
     b->hits.release(); b->grouped.release();
@@ -655,7 +683,7 @@ uint64_t blamm_hip_batch_device_bytes(const blamm_hip_batch* b)
 {
     if (!b) return 0;
     return (b->packed.n + b->lcmask.n + b->run_bits.n) * 8 + b->meta.n + (b->frag_a.n + b->frag_b.n) * 16 +
-           (b->band.n + b->band_hi.n) * 8 + b->req_count.n * 4 + (b->req_off.n + b->cursor.n) * 8 + b->cand.n * 16 +
+           (b->band.n + b->band_hi.n) * 8 + b->bound.n * sizeof(double2) + b->req_count.n * 4 + (b->req_off.n + b->cursor.n) * 8 + b->cand.n * 16 +
            b->hits.n * sizeof(DevHit) + b->grouped.n * sizeof(GroupedHit) + kCntSlots * 8;
 }
 
@@ -696,8 +724,7 @@ int blamm_hip_batch_submit(blamm_hip_batch* b, const blamm_request* reqs, uint32
     const uint64_t pw = total / 32 + 16, mw = mask ? total / 64 + 16 : 0;
     const size_t nslots = (size_t)c->nslots;
     const uint32_t cpb = (uint32_t)c->cols_per_blk;
-    const uint32_t ct = std::max<uint32_t>(1, c->tuning.chunk_tiles);
-    const bool bf = prec_bf(c->precision);
+    const bool bf = prec_bf(c->precision), screen = prec_screen(c->precision);
     const uint32_t nbmax = std::min<uint32_t>(c->tuning.blocks_per_wave, bf ? kNbMaxBf16 : kNbMaxFp32);
     const int kstep = (int)c->tuning.kpad_positions / 4;
 
@@ -715,7 +742,7 @@ int blamm_hip_batch_submit(blamm_hip_batch* b, const blamm_request* reqs, uint32
         }
         if (sel.empty() || b->n_h[r] == 0) continue;
         const uint32_t blk_first = (uint32_t)breq.size();
-        std::vector<int> nchs;
+        std::vector<int> nchs, lens;
         for (size_t i = 0; i < sel.size(); i += cpb) {
             int lm = 0;
             for (uint32_t k = 0; k < cpb; ++k) {
@@ -733,10 +760,12 @@ int blamm_hip_batch_submit(blamm_hip_batch* b, const blamm_request* reqs, uint32
             int nch = (lm + 3) / 4;
             nch = std::min(kMaxChunks, (nch + kstep - 1) / kstep * kstep);
             nchs.push_back(nch);
+            lens.push_back(lm);
             breq.push_back(r);
         }
         std::vector<GroupInfo> gr;
-        for (size_t i = 0; i < nchs.size();) {
+        if (screen) gr = screen_groups(lens, blk_first, c->tuning.blocks_per_wave);
+        else for (size_t i = 0; i < nchs.size();) {
             size_t e = i;
             while (e < nchs.size() && nchs[e] == nchs[i]) ++e;
             size_t bb = i;
@@ -756,9 +785,12 @@ int blamm_hip_batch_submit(blamm_hip_batch* b, const blamm_request* reqs, uint32
     }
     const uint32_t nblk = (uint32_t)breq.size();
     if (nblk >= (1u << 20)) return fail(BLAMM_ERR_ARG, "batch_submit: too many column blocks in one batch");
-    // Chunks and items, chunk k to sub-queue k % kXcds, chunk-major.
+    // Chunks and items, chunk k to queue k % kQueues, chunk-major.
+    uint64_t work = 0;
+    for (uint32_t r = 0; r < nreq; ++r) work += (b->n_h[r] + kBf16Tile - 1) / kBf16Tile * rgroups[r].size();
+    const uint32_t ct = item_tiles(work, batch_grid(b, mask) * kWavesPerBlock, c->tuning.chunk_tiles);
     std::vector<uint4> chunks;
-    std::vector<std::vector<uint2>> sub(kXcds);
+    uint64_t sub[kQueues] = {};
     for (uint32_t r = 0; r < nreq; ++r) {
         if (b->n_h[r] == 0 || rgroups[r].empty()) continue;
         const uint32_t tb = (uint32_t)(b->start_h[r] / kBf16Tile);
@@ -766,16 +798,16 @@ int blamm_hip_batch_submit(blamm_hip_batch* b, const blamm_request* reqs, uint32
         for (uint32_t t = tb; t < te; t += ct) {
             const uint32_t k = (uint32_t)chunks.size();
             chunks.push_back(make_uint4(t, std::min(te, t + ct), r, 0));
-            for (uint32_t g : rgroups[r]) sub[k % kXcds].push_back(make_uint2(k, g));
+            sub[k % kQueues] += rgroups[r].size();
         }
     }
     BatchDesc d{};
     size_t nitems = 0;
-    for (int x = 0; x < kXcds; ++x) {
+    for (int x = 0; x < kQueues; ++x) {
         d.sub_begin[x] = (uint32_t)nitems;
-        nitems += sub[x].size();
+        nitems += sub[x];
     }
-    d.sub_begin[kXcds] = (uint32_t)nitems;
+    d.sub_begin[kQueues] = (uint32_t)nitems;
     if (nitems >= (1ull << 32)) return fail(BLAMM_ERR_ARG, "batch_submit: work list too long");
     d.nreq = nreq;
     d.nbases = (uint32_t)total;
@@ -797,12 +829,15 @@ int blamm_hip_batch_submit(blamm_hip_batch* b, const blamm_request* reqs, uint32
     need[kMetaRuns] = nruns + 1;
     need[kMetaItems] = std::max<size_t>(nitems, 1);
     BLAMM_TRY(meta_fit(b, need));
-    BLAMM_TRY(batch_grow(b, b->band, nbs));
-    BLAMM_TRY(batch_grow(b, b->band_hi, nbs));
-    const size_t fr = (size_t)std::max<uint32_t>(nblk, 1) * batch_frag_elems(bf);
+    const size_t fr = (size_t)std::max<uint32_t>(nblk, 1) * batch_frag_elems(c->precision);
     BLAMM_TRY(batch_grow(b, b->frag_a, fr));
-    if (bf) BLAMM_TRY(batch_grow(b, b->frag_b, fr));
-    else BLAMM_TRY(batch_grow(b, b->frag_b, 1));
+    if (screen) {
+        BLAMM_TRY(batch_grow(b, b->bound, nbs));
+    } else {
+        BLAMM_TRY(batch_grow(b, b->band, nbs));
+        BLAMM_TRY(batch_grow(b, b->band_hi, nbs));
+        BLAMM_TRY(batch_grow(b, b->frag_b, bf ? fr : 1));
+    }
     BLAMM_TRY(batch_grow(b, b->req_count, nreq));
     BLAMM_TRY(batch_grow(b, b->req_off, (size_t)nreq + 1));
     BLAMM_TRY(batch_grow(b, b->cursor, nreq));
@@ -861,11 +896,11 @@ int blamm_hip_batch_submit(blamm_hip_batch* b, const blamm_request* reqs, uint32
     std::memcpy(table(kMetaBlkReq), breq.data(), (size_t)nblk * 4);
     std::memcpy(table(kMetaGroups), gpk.data(), gpk.size() * 4);
     std::memcpy(table(kMetaChunks), chunks.data(), chunks.size() * 16);
-    size_t at = 0;
-    for (int x = 0; x < kXcds; ++x) {
-        std::memcpy(table(kMetaItems) + at * 8, sub[x].data(), sub[x].size() * 8);
-        at += sub[x].size();
-    }
+    uint2* items = (uint2*)table(kMetaItems);
+    size_t at[kQueues];
+    for (int x = 0; x < kQueues; ++x) at[x] = d.sub_begin[x];
+    for (size_t k = 0; k < chunks.size(); ++k)
+        for (uint32_t g : rgroups[chunks[k].z]) items[at[k % kQueues]++] = make_uint2((uint32_t)k, g);
     std::memcpy(table(kMetaDesc), &d, sizeof(d));
 
     hipStream_t s = b->stream;

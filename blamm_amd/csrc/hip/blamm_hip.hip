@@ -120,14 +120,14 @@ struct GroupInfo {
 
 }  // namespace
 
-// Scratch of blamm_hip_scan_device_noalloc: the scan counters (first 256
+// Scratch of blamm_hip_scan_device_noalloc: the scan counters (first 8,448
 // bytes) and BLAMM_NOALLOC_MAX_RECORDS filter records of 16 bytes, 64 MiB in
 // all.  Every GPU the library runs on holds its own copy until the process
 // ends; all contexts on one GPU share it, so no-alloc scans that overlap on
 // one GPU race.  Host code never uses the array's name as an address: the
 // device address of each GPU's copy comes from hipGetSymbolAddress, taken
 // once per device in blamm_hip_create with that device current.
-constexpr uint64_t kNoAllocHeader = 256;
+constexpr uint64_t kNoAllocHeader = 8448;
 static_assert(kCntSlots * sizeof(unsigned long long) <= kNoAllocHeader, "counters exceed the scratch header");
 static __device__ __align__(256) uint8_t scratch[kNoAllocHeader + (uint64_t)BLAMM_NOALLOC_MAX_RECORDS * 16];
 
@@ -178,6 +178,7 @@ struct blamm_hip_ctx {
     int nslots = 0;
     int cols_per_blk = 32;
     std::vector<GroupInfo> groups;             // longest motifs first
+    uint32_t nscan_groups = 0;                 // groups of the scan in scan_groups_d
     std::vector<int> slot_col_h;               // -1 = empty slot
     std::vector<double> band_h, seq_h;         // per slot
     double max_filter_band = 0.0, max_score_error = 0.0;
@@ -186,7 +187,11 @@ struct blamm_hip_ctx {
     DevBuf<double> slot_band, slot_band_any, slot_seq;   // band_any: valid in a block of any length
     DevBuf<double> slot_band_hi, slot_band_hi_any;      // hi-only stage of the bf16 filter
     DevBuf<int> slot_len;
-    DevBuf<uint32_t> slot_col, groups_d;
+    DevBuf<uint32_t> slot_col, scan_groups_d;
+    // screen layout (default form): fragments and bounds for streams without
+    // [0] and with [1] a lowercase mask
+    DevBuf<uint2> screen_frag[2];
+    DevBuf<double2> screen_bound[2];
 
     // empirical histograms
     DevBuf<HistSlot> hist_slots;
@@ -215,58 +220,55 @@ struct blamm_hip_ctx {
 
 namespace {
 
-// Precision modes: FP32, or bf16 with the filter in its hi-only or lazy-lo
-// form (both keep the PWM split into hi and lo terms on the device).
+// Precision modes: FP32, split bf16 with the lo products on the matrix cores,
+// or (default) split bf16 behind the screen.  Both bf16 modes keep the hi and
+// lo terms on the device (histograms use them).
 inline bool prec_bf(int p) { return p == BLAMM_PREC_BF16X2 || p == BLAMM_PREC_BF16X2_LO; }
-inline bool prec_lo(int p) { return p == BLAMM_PREC_BF16X2_LO; }
+inline bool prec_screen(int p) { return p == BLAMM_PREC_BF16X2; }
 
-template <bool BF, bool MASK, bool LIST>
-const void* filter_kernel_ptr()
+template <bool MASK, bool LIST>
+const void* filter_kernel_ptr(int precision)
 {
-    return (const void*)filter_persistent_kernel<BF, MASK, LIST>;
+    return precision == BLAMM_PREC_BF16X2      ? (const void*)screen_kernel<MASK, LIST>
+           : precision == BLAMM_PREC_BF16X2_LO ? (const void*)filter_lo_kernel<MASK, LIST>
+                                               : (const void*)filter_fp32_kernel<MASK, LIST>;
 }
 
-const void* filter_kernel(bool bf, bool lo, bool mask, bool list)
+const void* filter_kernel(int precision, bool mask, bool list)
 {
-    if (bf && lo) {
-        if (mask) return list ? (const void*)filter_lo_kernel<true, true> : (const void*)filter_lo_kernel<true, false>;
-        return list ? (const void*)filter_lo_kernel<false, true> : (const void*)filter_lo_kernel<false, false>;
-    }
-    if (bf) {
-        if (mask) return list ? filter_kernel_ptr<true, true, true>() : filter_kernel_ptr<true, true, false>();
-        return list ? filter_kernel_ptr<true, false, true>() : filter_kernel_ptr<true, false, false>();
-    }
-    if (mask) return list ? filter_kernel_ptr<false, true, true>() : filter_kernel_ptr<false, true, false>();
-    return list ? filter_kernel_ptr<false, false, true>() : filter_kernel_ptr<false, false, false>();
+    if (mask) return list ? filter_kernel_ptr<true, true>(precision) : filter_kernel_ptr<true, false>(precision);
+    return list ? filter_kernel_ptr<false, true>(precision) : filter_kernel_ptr<false, false>(precision);
 }
 
 // Workgroups of the persistent filter resident per CU (register/LDS limits).
-int persistent_wgs_per_cu(bool bf, bool lo, bool mask, bool list)
+int persistent_wgs_per_cu(int precision, bool mask, bool list)
 {
     int n = 0;
-    hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, filter_kernel(bf, lo, mask, list), kThreads, 0);
+    hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, filter_kernel(precision, mask, list), kThreads, 0);
     return (e == hipSuccess && n > 0) ? n : 1;
 }
 
-hipError_t launch_filter(bool bf, bool lo, bool mask, bool list, const FilterArgs& a, const WorkQueue& q,
-                         const ListArgs& l, uint32_t grid, hipStream_t s)
+// Window tiles per work item for `work` tiles x groups on `waves` resident
+// waves: about 24 items per wave, so that the last ones end together, but not
+// below 16 tiles, where loading a group's fragments shows, unless there is not
+// even one such item per wave.  `most` is the tuned window tile.
+uint32_t item_tiles(uint64_t work, uint32_t waves, uint32_t most)
 {
-#define BLAMM_LAUNCH(B, M, L) \
-    hipLaunchKernelGGL((filter_persistent_kernel<B, M, L>), dim3(grid), dim3(kThreads), 0, s, a, q, l)
-#define BLAMM_LAUNCH_LO(M, L) hipLaunchKernelGGL((filter_lo_kernel<M, L>), dim3(grid), dim3(kThreads), 0, s, a, q, l)
-    if (bf && lo) {
-        if (mask) { if (list) BLAMM_LAUNCH_LO(true, true); else BLAMM_LAUNCH_LO(true, false); }
-        else { if (list) BLAMM_LAUNCH_LO(false, true); else BLAMM_LAUNCH_LO(false, false); }
-    } else if (bf) {
-        if (mask) { if (list) BLAMM_LAUNCH(true, true, true); else BLAMM_LAUNCH(true, true, false); }
-        else { if (list) BLAMM_LAUNCH(true, false, true); else BLAMM_LAUNCH(true, false, false); }
-    } else {
-        if (mask) { if (list) BLAMM_LAUNCH(false, true, true); else BLAMM_LAUNCH(false, true, false); }
-        else { if (list) BLAMM_LAUNCH(false, false, true); else BLAMM_LAUNCH(false, false, false); }
-    }
-#undef BLAMM_LAUNCH
-#undef BLAMM_LAUNCH_LO
-    return hipGetLastError();
+    const uint64_t w = std::max<uint32_t>(waves, 1);
+    const uint64_t fine = std::min<uint64_t>(16, std::max<uint64_t>(2, work / w));
+    return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(most, std::max<uint64_t>(work / (24 * w), fine)));
+}
+
+// Launch the precision's filter: `a` for the screen, `f` for the others.
+hipError_t launch_filter(int precision, bool mask, bool list, const ScreenArgs& a, const FilterArgs& f,
+                         const WorkQueue& q, const ListArgs& l, uint32_t grid, hipStream_t s)
+{
+    WorkQueue qa = q;
+    ListArgs la = l;
+    ScreenArgs sa = a;
+    FilterArgs fa = f;
+    void* args[] = {prec_screen(precision) ? (void*)&sa : (void*)&fa, &qa, &la};
+    return hipLaunchKernel(filter_kernel(precision, mask, list), dim3(grid), dim3(kThreads), args, 0, s);
 }
 
 hipError_t launch_finalize(bool bf, bool list, const FinalizeArgs& f, uint32_t grid, hipStream_t s)
@@ -297,6 +299,28 @@ int check_tuning(const blamm_tuning& t, int precision)
     if (t.kpad_positions != 4 && t.kpad_positions != 8)
         return fail(BLAMM_ERR_ARG, "tuning: kpad_positions must be 4 or 8");
     return BLAMM_OK;
+}
+
+// Column groups of the screen for consecutive blocks blk0, blk0 + 1, ... whose
+// longest motifs are blk_len (non-decreasing): runs of blocks with the same
+// number of MFMAs cut into groups of screen_blocks(), the remainder into
+// smaller powers of two, so no padding block is scored.  Longest first.
+std::vector<GroupInfo> screen_groups(const std::vector<int>& blk_len, uint32_t blk0, uint32_t unit)
+{
+    std::vector<GroupInfo> out;
+    auto steps = [&](size_t i) { return (blk_len[i] + kScreenPos - 1) / kScreenPos; };
+    for (size_t i = 0; i < blk_len.size();) {
+        size_t e = i;
+        while (e < blk_len.size() && steps(e) == steps(i)) ++e;
+        const int ks = steps(i);
+        for (uint32_t nb = (uint32_t)screen_blocks(ks, (int)unit); nb >= 1; nb /= 2)
+            while (e - i >= nb) {
+                out.push_back({blk0 + (uint32_t)i, (uint32_t)ks, nb});
+                i += nb;
+            }
+    }
+    std::stable_sort(out.begin(), out.end(), [](const GroupInfo& x, const GroupInfo& y) { return x.nch > y.nch; });
+    return out;
 }
 
 // Lay the stored library out for the kernels under the context's tuning and
@@ -352,6 +376,15 @@ int relayout(blamm_hip_ctx* c)
     std::stable_sort(groups.begin(), groups.end(), [](const GroupInfo& x, const GroupInfo& y) { return x.nch > y.nch; });
     const int nblk = (int)blocks.size();
     const int nslots = nblk * cols_per_blk;
+    // The scan's groups: those of the screen in the default form.
+    std::vector<GroupInfo> scan_groups = groups;
+    if (prec_screen(c->precision)) {
+        std::vector<int> blk_len(nblk, 1);
+        for (int i = 0; i < nblk; ++i)
+            for (int col : blocks[i])
+                if (col >= 0) blk_len[i] = std::max(blk_len[i], lengths[col]);
+        scan_groups = screen_groups(blk_len, 0, c->tuning.blocks_per_wave);
+    }
     if (nblk >= (1 << 20)) return fail(BLAMM_ERR_ARG, "set_library: too many columns");
 
     std::vector<float> s_thr(nslots, INFINITY), s_w((size_t)nslots * kMaxLen * 4, 0.f);
@@ -461,8 +494,9 @@ int relayout(blamm_hip_ctx* c)
                 }
         fb.assign(16, 0);
     }
-    std::vector<uint32_t> gpk(groups.size());
-    for (size_t g = 0; g < groups.size(); ++g) gpk[g] = group_pack(groups[g].blk0, groups[g].nch, groups[g].nb);
+    std::vector<uint32_t> gpk(scan_groups.size());
+    for (size_t g = 0; g < scan_groups.size(); ++g)
+        gpk[g] = group_pack(scan_groups[g].blk0, scan_groups[g].nch, scan_groups[g].nb);
 
     c->have_lib = false;
     HIP_TRY(hipStreamSynchronize(c->stream));
@@ -488,7 +522,7 @@ int relayout(blamm_hip_ctx* c)
     HIP_TRY(hipMemcpy(c->slot_w2.p, s_w2.data(), s_w2.size() * sizeof(float), hipMemcpyHostToDevice));
     HIP_TRY(c->slot_len.reserve(nslots));
     HIP_TRY(c->slot_col.reserve(nslots));
-    HIP_TRY(c->groups_d.reserve(gpk.size()));
+    HIP_TRY(c->scan_groups_d.reserve(gpk.size()));
     HIP_TRY(hipMemcpy(c->frag_a.p, fa.data(), fa.size(), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(c->frag_b.p, fb.data(), fb.size(), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(c->slot_thr.p, s_thr.data(), nslots * sizeof(float), hipMemcpyHostToDevice));
@@ -501,10 +535,27 @@ int relayout(blamm_hip_ctx* c)
     HIP_TRY(hipMemcpy(c->slot_w.p, s_w.data(), s_w.size() * sizeof(float), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(c->slot_len.p, s_len.data(), nslots * sizeof(int), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(c->slot_col.p, s_col.data(), nslots * sizeof(uint32_t), hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(c->groups_d.p, gpk.data(), gpk.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(c->scan_groups_d.p, gpk.data(), gpk.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+    if (prec_screen(c->precision)) {
+        ScreenLayoutArgs a;
+        a.slot_w = c->slot_w.p;
+        a.slot_len = c->slot_len.p;
+        a.nslots = (uint32_t)nslots;
+        for (int m = 0; m < 2; ++m) {
+            HIP_TRY(c->screen_frag[m].reserve((size_t)nblk * kScreenBlock));
+            HIP_TRY(c->screen_bound[m].reserve(nslots));
+            a.frag[m] = c->screen_frag[m].p;
+            a.bound[m] = c->screen_bound[m].p;
+        }
+        hipLaunchKernelGGL(screen_layout_kernel, dim3((nslots + kWavesPerBlock - 1) / kWavesPerBlock), dim3(kThreads),
+                           0, c->stream, a);
+        HIP_TRY(hipGetLastError());
+        HIP_TRY(hipStreamSynchronize(c->stream));   // scans may run on other streams
+    }
     c->nslots = nslots;
     c->cols_per_blk = cols_per_blk;
     c->groups = groups;
+    c->nscan_groups = (uint32_t)gpk.size();
     c->slot_col_h = s_colh;
     c->band_h = s_band;
     c->seq_h = s_seq;
@@ -526,7 +577,24 @@ FilterArgs filter_args(const blamm_hip_ctx* c, const uint64_t* packed, const uin
     a.thr = thr;
     a.band = c->slot_band.p;
     a.band_hi = c->slot_band_hi.p;
-    a.groups = c->groups_d.p;
+    a.groups = c->scan_groups_d.p;
+    a.cand = cand;
+    a.counters = counters;
+    a.cand_cap = cand_cap;
+    return a;
+}
+
+ScreenArgs screen_args(const blamm_hip_ctx* c, const uint64_t* packed, const uint64_t* lcmask, const float* thr,
+                       uint4* cand, uint64_t cand_cap, unsigned long long* counters)
+{
+    const int m = lcmask ? 1 : 0;
+    ScreenArgs a;
+    a.packed = packed;
+    a.lcmask = lcmask;
+    a.frag = c->screen_frag[m].p;
+    a.thr = thr;
+    a.bound = c->screen_bound[m].p;
+    a.groups = c->scan_groups_d.p;
     a.cand = cand;
     a.counters = counters;
     a.cand_cap = cand_cap;
@@ -631,7 +699,11 @@ int blamm_hip_destroy(blamm_hip_ctx* c)
     c->frag_a.release(); c->frag_b.release(); c->slot_thr.release(); c->slot_band.release();
     c->slot_band_any.release(); c->slot_band_hi.release(); c->slot_band_hi_any.release();
     c->slot_seq.release(); c->slot_w.release(); c->slot_w2.release();
-    c->slot_len.release(); c->slot_col.release(); c->groups_d.release(); c->cand.release();
+    c->slot_len.release(); c->slot_col.release(); c->scan_groups_d.release(); c->cand.release();
+    for (int m = 0; m < 2; ++m) {
+        c->screen_frag[m].release();
+        c->screen_bound[m].release();
+    }
     c->counters.release(); c->run_bits.release();
     c->packed.release(); c->lcmask.release(); c->runs.release(); c->nhits_dev.release();
     c->hits.release();
@@ -773,18 +845,21 @@ int enqueue_scan(blamm_hip_ctx* c, const uint64_t* d_packed, const uint64_t* d_l
     if (nbases > 0) {
         const uint32_t ntiles = (uint32_t)((nbases + kBf16Tile - 1) / kBf16Tile);   // 32-window tiles
         const FilterArgs a = filter_args(c, d_packed, d_lcmask, c->slot_thr.p, cand, cand_cap, counters);
+        const ScreenArgs sa = screen_args(c, d_packed, d_lcmask, c->slot_thr.p, cand, cand_cap, counters);
         WorkQueue q{};
         q.ntiles = ntiles;
-        q.chunk_tiles = std::max<uint32_t>(1, std::min<uint32_t>(c->tuning.chunk_tiles, ntiles));
+        const uint32_t full = (uint32_t)c->num_cu * (uint32_t)persistent_wgs_per_cu(c->precision, mask, false) *
+                              (uint32_t)c->filter_rounds;
+        q.ngroups = c->nscan_groups;
+        q.chunk_tiles = std::min(ntiles, item_tiles((uint64_t)ntiles * q.ngroups, full * kWavesPerBlock,
+                                                    c->tuning.chunk_tiles));
         q.nchunks = (ntiles + q.chunk_tiles - 1) / q.chunk_tiles;
-        q.ngroups = (uint32_t)c->groups.size();
-        if ((uint64_t)((q.nchunks + kXcds - 1) / kXcds) * q.ngroups >= (1ull << 32))
-            return fail(BLAMM_ERR_ARG, "scan: work queue too long");
+        const uint64_t sub = (uint64_t)((q.nchunks + kQueues - 1) / kQueues) * q.ngroups;   // items of queue 0
+        if (sub >= (1ull << 32) - (1u << 16)) return fail(BLAMM_ERR_ARG, "scan: work queue too long");
         const ListArgs l{nullptr, nullptr, nullptr};
-        const uint32_t grid =
-            (uint32_t)c->num_cu * (uint32_t)persistent_wgs_per_cu(bf, prec_lo(c->precision), mask, false) *
-            (uint32_t)c->filter_rounds;
-        hipError_t e = launch_filter(bf, prec_lo(c->precision), mask, false, a, q, l, grid, s);
+        // no more workgroups than the fullest queue has use for
+        const uint32_t grid = (uint32_t)std::min<uint64_t>(full, (sub + kWavesPerBlock - 1) / kWavesPerBlock * kQueues);
+        hipError_t e = launch_filter(c->precision, mask, false, sa, a, q, l, grid, s);
         if (e != hipSuccess) return fail(BLAMM_ERR_DEVICE, std::string("filter launch: ") + hipGetErrorString(e));
     }
     HIP_TRY(hipEventRecord(c->ev[1], s));
@@ -861,7 +936,7 @@ int blamm_hip_scan_finish(blamm_hip_ctx* c, uint64_t* nhits)
     c->pending = false;
     HIP_TRY(hipSetDevice(c->device));
     HIP_TRY(hipStreamSynchronize(c->pending_stream));
-    unsigned long long cnt[kCntSlots];
+    unsigned long long cnt[kCntStats];
     HIP_TRY(hipMemcpy(cnt, c->pending_counters, sizeof(cnt), hipMemcpyDeviceToHost));
     float ms_f = 0.f, ms_all = 0.f;
     HIP_TRY(hipEventElapsedTime(&ms_f, c->ev[0], c->ev[1]));

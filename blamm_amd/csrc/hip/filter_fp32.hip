@@ -3,9 +3,6 @@
 #include "instances.hpp"
 
 namespace blamm {
-#define BLAMM_DEF_FILTER(B, M, L) template __global__ void filter_persistent_kernel<B, M, L>(FilterArgs, WorkQueue, ListArgs);
-BLAMM_DEF_FILTER(false, false, false)
-BLAMM_DEF_FILTER(false, false, true)
-BLAMM_DEF_FILTER(false, true, false)
-BLAMM_DEF_FILTER(false, true, true)
+#define BLAMM_DEF_FP32(M, L) template __global__ void filter_fp32_kernel<M, L>(FilterArgs, WorkQueue, ListArgs);
+BLAMM_SCAN_INSTANCES(BLAMM_DEF_FP32)
 }  // namespace blamm

@@ -203,7 +203,7 @@ int blamm_hip_hist_device(blamm_hip_ctx* c, const uint64_t* d_packed, uint64_t p
     }
     HIP_TRY(hipEventRecord(c->ev[1], s));
     HIP_TRY(hipStreamSynchronize(s));
-    unsigned long long cnt[kCntSlots];
+    unsigned long long cnt[kCntStats];
     HIP_TRY(hipMemcpy(cnt, c->counters.p, sizeof(cnt), hipMemcpyDeviceToHost));
     std::vector<unsigned long long> dev(ncount);
     HIP_TRY(hipMemcpy(dev.data(), c->hist_counts.p, ncount * sizeof(unsigned long long), hipMemcpyDeviceToHost));

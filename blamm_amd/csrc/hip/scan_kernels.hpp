@@ -30,7 +30,7 @@ constexpr int kThreads = kWaveSize * kWavesPerBlock;
 constexpr int kMaxLen = 64;          // positions per column slot
 constexpr int kMaxChunks = kMaxLen / 4;
 constexpr int kWideChunks = 8;       // above this many chunks a wave holds one column block
-constexpr int kLoChunks = 16;        // lazy-lo form: chunk fragments per wave in LDS (NB x NCH)
+constexpr int kLoChunks = 16;        // split-BF16 filter: chunk fragments per wave in LDS (NB x NCH)
 constexpr int kBf16Cols = 32;        // columns per bf16 column block (MFMA N)
 constexpr int kBf16Tile = 32;        // windows per bf16 tile (MFMA M)
 constexpr int kFp32Cols = 16;        // columns per fp32 column block
@@ -39,8 +39,12 @@ constexpr int kFp32Tile = 16;        // windows per fp32 tile
 // Batch slot without a column.
 constexpr uint32_t kNoSlot = 0xFFFFFFFFu;
 
-// Counter slots in device memory.
-enum { kCntCand = 0, kCntHits = 1, kCntBand = 2, kCntQueue = 4, kCntSlots = 12 };
+// Counter slots in device memory.  The heads of the filters' work queues have
+// a cache line each: atomics on one line pass one by one (11.4 ns each, from
+// all XCDs together), on 64 lines at 0.26 ns each.
+constexpr int kQueues = 64;
+enum { kCntCand = 0, kCntHits = 1, kCntBand = 2, kCntStats = 3, kCntQueue = 4, kCntHeads = 16, kCntLine = 16,
+       kCntSlots = kCntHeads + kQueues * kCntLine };
 
 // 64 consecutive bits of a little-endian bit stream starting at bit `bit`.
 __device__ __forceinline__ uint64_t load_bits64(const uint64_t* __restrict__ words, uint64_t bit)
@@ -74,7 +78,7 @@ struct FilterArgs {
     const void* frag_b;          // bf16: lo fragments
     const float* thr;            // per slot: threshold
     const double* band;          // per slot: filter band (MFMA score vs FP64 score)
-    const double* band_hi;       // per slot: band of the hi-only score (bf16 lazy-lo stage)
+    const double* band_hi;       // per slot: band of the hi-only score (split-BF16 filter)
     const uint32_t* groups;      // column groups, see group_pack()
     uint4* cand;                 // (first window of a lane, slot, rows above the threshold, 0)
     unsigned long long* counters;
@@ -121,7 +125,7 @@ constexpr int kStage = 256;
 struct Stage {
     uint4* buf;        // this wave's LDS slice
     uint32_t n;        // staged entries (wave-uniform)
-    uint4* lo;         // bf16: this wave's lo fragments (LDS), [block][chunk][lane]
+    uint4* lo;         // split-BF16 filter: this wave's lo fragments (LDS), [block][chunk][lane]
 };
 
 template <class Args>   // FilterArgs or HistArgs: cand, counters, cand_cap
@@ -210,17 +214,10 @@ __device__ __forceinline__ uint32_t funnel32(uint32_t lo, uint32_t hi, uint32_t 
 // prefetches the next group's words one group ahead.
 constexpr int kGroup = 4;
 
-// Two forms of the bf16 filter (template flag LO), both software-pipelined
-// over two accumulator sets and both exact after finalize:
-//  - hi only (LO = false, BLAMM_PREC_BF16X2): a tile block whose hi-only
-//    score can reach the threshold records its windows at or above
-//    thr - band_hi for finalize to decide; lo products are never issued.
-//  - lazy lo (LO = true, BLAMM_PREC_BF16X2_LO): such a block gets its lo
-//    products (lo fragments kept in a per-wave LDS slice) and records its
-//    windows at or above thr - band.
-// At 100 Mbp x 2,000 columns the hi-only form issues 11% fewer MFMAs and no
-// lo-fragment LDS traffic for 14% more records (filter 21.9 -> 19.2 ms at two
-// waves per SIMD).
+// The split-BF16 filter (BLAMM_PREC_BF16X2_LO) is software-pipelined over two
+// accumulator sets: a tile block whose hi-only score can reach the threshold
+// gets its lo products (lo fragments kept in a per-wave LDS slice) and records
+// its windows at or above thr - band.
 
 // ---------------------------------------------------------------------------
 // Split-BF16 filter: W = hi + lo (bf16 each); one-hot operand is exact in bf16.
@@ -229,8 +226,8 @@ constexpr int kGroup = 4;
 // Lane l: A rows/ B cols index l%32, K half h = l/32 holds positions 2h, 2h+1
 // of the chunk; D lane l holds column l%32, rows 8(r/4) + 4h + r%4.
 // Each wave keeps the hi terms of NB column blocks (NCH chunks) in registers
-// and streams window tiles through them (the lazy-lo form keeps the lo terms
-// in its LDS slice; the histogram kernel keeps both in registers).
+// and streams window tiles through them (the filter keeps the lo terms in its
+// LDS slice, the histogram kernel both in registers).
 // ---------------------------------------------------------------------------
 // The one-hot operand of chunk j for the lane's window: bf16 1.0 (0x3F80) in
 // lane b of four per base, built in registers (no memory latency; the VALU
@@ -328,9 +325,7 @@ __device__ __forceinline__ void bf16_mfma_tile(f32x16 (&acc)[NB], const bf16x8 (
 // the split's representation error and every rounding (proved per column on
 // the host).  So a tile block whose hi-only maximum stays below that bound in
 // every lane cannot hold a candidate and its lo products are skipped; blocks
-// that pass get their lo products and the exact-band test of the plain form
-// (modes 1, 2), or record their windows with H' >= thr - band_hi as they are
-// (mode 3; the record's row mask then marks those windows).
+// that pass get their lo products and the exact-band test.
 // ---------------------------------------------------------------------------
 template <int NCH, int NB, bool MASK>
 __device__ __forceinline__ void bf16_hi_tile(f32x16 (&acc)[NB], const bf16x8 (&bh)[NB][NCH],
@@ -356,9 +351,9 @@ __device__ __forceinline__ float tile_max(const f32x16& v)
 }
 
 // Finish a tile whose hi products are in acc (R: how the first read is kept
-// clear of the matrix cores).  Lazy-lo form: the lo fragments come from the
-// wave's LDS slice.
-template <int NCH, int NB, bool MASK, bool LO, AccRead R>
+// clear of the matrix cores).  The lo fragments come from the wave's LDS
+// slice.
+template <int NCH, int NB, bool MASK, AccRead R>
 __device__ __forceinline__ void bf16_finish_tile(const FilterArgs& a, Stage& st, f32x16 (&acc)[NB],
                                                  const float (&th)[NB], const float (&thh)[NB], const OneHotSrc& bits,
                                                  uint64_t mb, uint32_t q0, uint32_t blk0, uint32_t lane)
@@ -370,50 +365,38 @@ __device__ __forceinline__ void bf16_finish_tile(const FilterArgs& a, Stage& st,
         if (__ballot(tile_max<NB>(hv[b]) >= thh[b])) need |= 1u << b;
     if (need == 0) return;
     const uint32_t qlane = q0 + 4 * (lane >> 5);
-    if constexpr (!LO) {
-        (void)th; (void)bits; (void)mb;
+    // one uniform branch per block around its whole chunk loop (a branch
+    // per MFMA would copy the accumulator at every join)
 #pragma unroll
-        for (int b = 0; b < NB; ++b)
-            if (need & (1u << b)) {
-                float v[16];
+    for (int b = 0; b < NB; ++b) {
+        if (!(need & (1u << b))) continue;
+        bf16x8 B[NCH];
 #pragma unroll
-                for (int r = 0; r < 16; ++r) v[r] = hv[b][r];
-                emit_rows<16>(a, st, v, thh[b], qlane, (blk0 + b) * kBf16Cols + (lane & 31));
-            }
-    } else {
-        // one uniform branch per block around its whole chunk loop (a branch
-        // per MFMA would copy the accumulator at every join)
+        for (int j = 0; j < NCH; ++j) B[j] = __builtin_bit_cast(bf16x8, st.lo[(b * NCH + j) * 64 + lane]);
 #pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            if (!(need & (1u << b))) continue;
-            bf16x8 B[NCH];
-#pragma unroll
-            for (int j = 0; j < NCH; ++j) B[j] = __builtin_bit_cast(bf16x8, st.lo[(b * NCH + j) * 64 + lane]);
-#pragma unroll
-            for (int j = 0; j < NCH; ++j)
-                acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(onehot_chunk<MASK>(bits, mb, j), B[j], acc[b], 0, 0, 0);
-        }
-        const f32x16 (&fv)[NB] = acc_read<AccRead::kGuard>(acc);
-#pragma unroll
-        for (int b = 0; b < NB; ++b)
-            if (need & (1u << b)) {
-                float v[16];
-#pragma unroll
-                for (int r = 0; r < 16; ++r) v[r] = fv[b][r];
-                emit_rows<16>(a, st, v, th[b], qlane, (blk0 + b) * kBf16Cols + (lane & 31));
-            }
+        for (int j = 0; j < NCH; ++j)
+            acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(onehot_chunk<MASK>(bits, mb, j), B[j], acc[b], 0, 0, 0);
     }
+    const f32x16 (&fv)[NB] = acc_read<AccRead::kGuard>(acc);
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+        if (need & (1u << b)) {
+            float v[16];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) v[r] = fv[b][r];
+            emit_rows<16>(a, st, v, th[b], qlane, (blk0 + b) * kBf16Cols + (lane & 31));
+        }
 }
 
 // Tiles [t0, t1) of column blocks blk0 .. blk0+NB-1.  Lane-private bases
 // of tile t come from packed words t and t+1 of the lane's pointer (a sliding
 // pair).  Software-pipelined: the hi products of tile t are issued before
 // tile t-1 is finished.
-template <int NCH, int NB, bool MASK, bool LO>
+template <int NCH, int NB, bool MASK>
 __device__ __forceinline__ void bf16_range(const FilterArgs& a, Stage& st, uint32_t blk0, uint32_t t0, uint32_t t1,
                                            uint32_t lane)
 {
-    static_assert(!LO || NB * NCH <= kLoChunks, "lo fragments exceed the wave's LDS slice");
+    static_assert(NB * NCH <= kLoChunks, "lo fragments exceed the wave's LDS slice");
     static_assert(NCH <= kWideChunks || NB == 1, "wide blocks are scored one per wave");
     const uint4* __restrict__ fh = (const uint4*)a.frag_a;
     const uint4* __restrict__ fl = (const uint4*)a.frag_b;
@@ -425,7 +408,7 @@ __device__ __forceinline__ void bf16_range(const FilterArgs& a, Stage& st, uint3
         for (int j = 0; j < NCH; ++j) {
             const size_t idx = ((size_t)(blk0 + b) * kMaxChunks + j) * 64 + lane;
             bh[b][j] = __builtin_bit_cast(bf16x8, fh[idx]);
-            if (LO) st.lo[(b * NCH + j) * 64 + lane] = fl[idx];   // each lane reads back only its own
+            st.lo[(b * NCH + j) * 64 + lane] = fl[idx];   // each lane reads back only its own
         }
         const uint32_t slot = (blk0 + b) * kBf16Cols + (lane & 31);
         th[b] = thr_minus(a.thr[slot], a.band[slot]);
@@ -457,12 +440,12 @@ __device__ __forceinline__ void bf16_range(const FilterArgs& a, Stage& st, uint3
         bB = onehot_src<NCH>(w0, w1, w2, sh);
         if (MASK) mB = window_mask<NCH>(m0, m1, m2, off & 31);
         bf16_hi_tile<NCH, NB, MASK>(accB, bh, bB, mB);
-        bf16_finish_tile<NCH, NB, MASK, LO, AccRead::kCovered>(a, st, accA, th, thh, bA, mA, (t - 1) * kBf16Tile, blk0,
+        bf16_finish_tile<NCH, NB, MASK, AccRead::kCovered>(a, st, accA, th, thh, bA, mA, (t - 1) * kBf16Tile, blk0,
                                                               lane);
         bA = onehot_src<NCH>(w1, w2, w3, sh);
         if (MASK) mA = window_mask<NCH>(m1, m2, m3, off & 31);
         bf16_hi_tile<NCH, NB, MASK>(accA, bh, bA, mA);
-        bf16_finish_tile<NCH, NB, MASK, LO, AccRead::kCovered>(a, st, accB, th, thh, bB, mB, t * kBf16Tile, blk0, lane);
+        bf16_finish_tile<NCH, NB, MASK, AccRead::kCovered>(a, st, accB, th, thh, bB, mB, t * kBf16Tile, blk0, lane);
         w0 = w2; w1 = w3; w2 = w4;
         if (MASK) { m0 = m2; m1 = m3; m2 = m4; }
     }
@@ -470,13 +453,13 @@ __device__ __forceinline__ void bf16_range(const FilterArgs& a, Stage& st, uint3
         bB = onehot_src<NCH>(w0, w1, w2, sh);
         if (MASK) mB = window_mask<NCH>(m0, m1, m2, off & 31);
         bf16_hi_tile<NCH, NB, MASK>(accB, bh, bB, mB);
-        bf16_finish_tile<NCH, NB, MASK, LO, AccRead::kCovered>(a, st, accA, th, thh, bA, mA, (t - 1) * kBf16Tile, blk0,
+        bf16_finish_tile<NCH, NB, MASK, AccRead::kCovered>(a, st, accA, th, thh, bA, mA, (t - 1) * kBf16Tile, blk0,
                                                               lane);
         pendingA = false;
-        bf16_finish_tile<NCH, NB, MASK, LO, AccRead::kGuard>(a, st, accB, th, thh, bB, mB, t * kBf16Tile, blk0, lane);
+        bf16_finish_tile<NCH, NB, MASK, AccRead::kGuard>(a, st, accB, th, thh, bB, mB, t * kBf16Tile, blk0, lane);
     }
     if (pendingA)
-        bf16_finish_tile<NCH, NB, MASK, LO, AccRead::kGuard>(a, st, accA, th, thh, bA, mA, (t - 1) * kBf16Tile, blk0,
+        bf16_finish_tile<NCH, NB, MASK, AccRead::kGuard>(a, st, accA, th, thh, bA, mA, (t - 1) * kBf16Tile, blk0,
                                                             lane);
 }
 
@@ -590,25 +573,28 @@ __device__ __forceinline__ void fp32_range(const FilterArgs& a, Stage& st, uint3
     }
 }
 
-// Work of the persistent filter is a set of items (tile chunk, column group).
-// Chunks are dealt to kXcds sub-queues (chunk k to sub-queue k % kXcds); a
-// workgroup starts on the sub-queue of its XCD (workgroups are dispatched
-// round-robin, so block b runs on XCD b % kXcds) and steals from the others
-// when it drains.  Inside a sub-queue items run chunk-major: all column groups
-// of a chunk follow each other, so the chunk's packed words are fetched into
-// that XCD's L2 once and reused by every group.  Groups are numbered longest
-// motifs first.
-//   implicit form (one stream, whole library): item j of sub-queue x is chunk
-//     (j / ngroups) * kXcds + x, group j % ngroups;
-//   list form (a batch of requests): sub-queue x holds
+// Work of the filter is a set of items (tile chunk, column group).  Chunks are
+// dealt to kQueues queues (chunk k to queue k % kQueues); a workgroup's home is
+// queue blockIdx % kQueues (workgroups are dispatched round-robin to the XCDs,
+// so a queue's waves share an XCD).  A queue's items run chunk-major: all
+// column groups of a chunk follow each other, so the chunk's packed words are
+// fetched into that XCD's L2 once and reused by every group.  Groups are
+// numbered longest motifs first.
+//   implicit form (one stream, whole library): item j of queue x is chunk
+//     (j / ngroups) * kQueues + x, group j % ngroups;
+//   list form (a batch of requests): queue x holds
 //     items[sub_begin[x] .. sub_begin[x+1]), each (chunk, group), and a chunk
 //     is (first tile, end tile, request); groups, fragments and per-slot
 //     tables then describe the batch's own column blocks (each request's
 //     selected columns packed into blocks of their own).
-constexpr int kXcds = 8;
+// A wave's first item is the one of its rank in its home; further ones come
+// from the queue's head, and when the home is empty from any queue that a look
+// at all heads shows unfinished, so a small scan asks nothing and a large one
+// ends evenly (equal shares fixed in advance were 15% slower at 62.5 Mbp x
+// 4,000 columns: the XCDs do not run at one speed).
 struct WorkQueue {
     uint32_t ntiles;
-    uint32_t nchunks;
+    uint32_t nchunks;       // implicit form: chunk k is tiles [k chunk_tiles, (k + 1) chunk_tiles)
     uint32_t chunk_tiles;
     uint32_t ngroups;
 };
@@ -626,7 +612,7 @@ struct GroupedHit {
 };
 
 struct BatchDesc {
-    uint32_t sub_begin[kXcds + 1];
+    uint32_t sub_begin[kQueues + 1];
     uint32_t nreq;
     uint32_t nbases;
     uint32_t nruns;
@@ -641,14 +627,14 @@ struct ListArgs {
 };
 
 // One item: tiles [t0, t1) against one column group.
-template <bool BF, bool MASK, bool LO>
+template <bool BF, bool MASK>
 __device__ __forceinline__ void filter_item(const FilterArgs& a, Stage& st, uint32_t grp,
                                             uint32_t t0, uint32_t t1, uint32_t lane)
 {
     const uint32_t blk0 = grp & 0xFFFFFu, nch = (grp >> 20) & 63u, nb = grp >> 26;
     if constexpr (BF) {
         switch (nch * 8 + nb) {
-#define BLAMM_BF(N, B) case N * 8 + B: bf16_range<N, B, MASK, LO>(a, st, blk0, t0, t1, lane); break;
+#define BLAMM_BF(N, B) case N * 8 + B: bf16_range<N, B, MASK>(a, st, blk0, t0, t1, lane); break;
         BLAMM_BF(1, 1) BLAMM_BF(2, 1) BLAMM_BF(3, 1) BLAMM_BF(4, 1)
         BLAMM_BF(5, 1) BLAMM_BF(6, 1) BLAMM_BF(7, 1) BLAMM_BF(8, 1)
         BLAMM_BF(1, 2) BLAMM_BF(2, 2) BLAMM_BF(3, 2) BLAMM_BF(4, 2)
@@ -675,67 +661,97 @@ __device__ __forceinline__ void filter_item(const FilterArgs& a, Stage& st, uint
     }
 }
 
-// One launch for the whole work set: every resident wave pulls items until
-// all sub-queues are empty (one atomic per item).
-template <bool BF, bool MASK, bool LIST, bool LO>
+// item(group, t0, t1) for every item that this wave takes.  It must be
+// always_inline: as a function of its own it would take the item as per-lane
+// values and the stage through memory, and its long branches would go through
+// the register pair that holds its return address.
+template <bool LIST, typename Item>
+__device__ __forceinline__ void for_each_item(unsigned long long* counters, const uint32_t* groups, const WorkQueue& q,
+                                              const ListArgs& l, Item&& item)
+{
+    const uint32_t home = blockIdx.x % kQueues;
+    auto items_of = [&](uint32_t x) __attribute__((always_inline)) {
+        if constexpr (LIST) return l.desc->sub_begin[x + 1] - l.desc->sub_begin[x];
+        else return x < q.nchunks ? ((q.nchunks - x + kQueues - 1) / kQueues) * q.ngroups : 0u;
+    };
+    auto waves_of = [&](uint32_t x) __attribute__((always_inline)) {
+        return x < gridDim.x ? ((gridDim.x - x + kQueues - 1) / kQueues) * (uint32_t)kWavesPerBlock : 0u;
+    };
+    auto head_of = [&](uint32_t x) __attribute__((always_inline)) {
+        return (unsigned int*)(counters + kCntHeads + x * kCntLine);
+    };
+    uint32_t x = home, n = __builtin_amdgcn_readfirstlane(items_of(home)), w = waves_of(home);
+    uint32_t j = (blockIdx.x / kQueues) * kWavesPerBlock + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    bool ask = false;
+    for (;;) {
+        if (ask) {
+            j = n;
+            if (n > w) {
+                uint32_t got = 0;
+                if ((threadIdx.x & 63) == 0) got = atomicAdd(head_of(x), 1u);
+                j = w + __builtin_amdgcn_readfirstlane(got);
+            }
+        }
+        ask = true;
+        if (j >= n) {
+            // lane y looks at queue home + y
+            const uint32_t y = (home + (threadIdx.x & 63)) % kQueues;
+            const uint32_t ny = items_of(y), wy = waves_of(y);
+            bool open = false;
+            if (ny > wy) open = __hip_atomic_load(head_of(y), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < ny - wy;
+            const uint64_t m = __ballot(open);
+            if (!m) break;
+            const uint32_t at = (uint32_t)__builtin_ctzll(m);
+            x = (home + at) % kQueues;
+            n = __builtin_amdgcn_readlane(ny, at);
+            w = waves_of(x);
+            continue;
+        }
+        uint32_t grp, t0, t1;
+        if constexpr (LIST) {
+            const uint2 it = l.items[l.desc->sub_begin[x] + j];
+            const uint4 ch = l.chunks[__builtin_amdgcn_readfirstlane(it.x)];
+            grp = __builtin_amdgcn_readfirstlane(groups[__builtin_amdgcn_readfirstlane(it.y)]);
+            t0 = __builtin_amdgcn_readfirstlane(ch.x);
+            t1 = __builtin_amdgcn_readfirstlane(ch.y);
+        } else {
+            const uint32_t k = (j / q.ngroups) * kQueues + x;
+            grp = __builtin_amdgcn_readfirstlane(groups[j % q.ngroups]);
+            t0 = k * q.chunk_tiles;
+            t1 = min(q.ntiles, t0 + q.chunk_tiles);
+        }
+        item(grp, t0, t1);
+    }
+}
+static_assert(kQueues == 64, "one lane looks at one queue");
+
+template <bool BF, bool MASK, bool LIST>
 __device__ __forceinline__ void filter_body(const FilterArgs& a, const WorkQueue& q, const ListArgs& l)
 {
     const uint32_t lane = threadIdx.x & 63;
     __shared__ uint4 stage_lds[kWavesPerBlock][kStage];
-    // lazy-lo form: per-wave lo fragments (kLoChunks chunk fragments x 64 lanes)
-    __shared__ uint4 lo_lds[LO ? kWavesPerBlock * kLoChunks * 64 : 1];
-    Stage st{stage_lds[threadIdx.x >> 6], 0u, LO ? lo_lds + (threadIdx.x >> 6) * kLoChunks * 64 : lo_lds};
-    const uint32_t home = blockIdx.x % kXcds;
-    for (uint32_t hop = 0; hop < (uint32_t)kXcds; ++hop) {
-        const uint32_t x = (home + hop) % kXcds;
-        uint32_t items = 0, base = 0;
-        if constexpr (LIST) {
-            base = __builtin_amdgcn_readfirstlane(l.desc->sub_begin[x]);
-            items = __builtin_amdgcn_readfirstlane(l.desc->sub_begin[x + 1]) - base;
-        } else {
-            if (x >= q.nchunks) continue;
-            items = ((q.nchunks - x + kXcds - 1) / kXcds) * q.ngroups;
-        }
-        for (;;) {
-            uint32_t j = 0;
-            if (lane == 0) j = atomicAdd((unsigned int*)&a.counters[kCntQueue + x], 1u);
-            j = __builtin_amdgcn_readfirstlane(__shfl(j, 0));
-            if (j >= items) break;
-            uint32_t grp, t0, t1;
-            if constexpr (LIST) {
-                const uint2 it = l.items[base + j];
-                const uint4 ch = l.chunks[__builtin_amdgcn_readfirstlane(it.x)];
-                grp = __builtin_amdgcn_readfirstlane(a.groups[__builtin_amdgcn_readfirstlane(it.y)]);
-                t0 = __builtin_amdgcn_readfirstlane(ch.x);
-                t1 = __builtin_amdgcn_readfirstlane(ch.y);
-            } else {
-                const uint32_t k = (j / q.ngroups) * kXcds + x;
-                grp = __builtin_amdgcn_readfirstlane(a.groups[j % q.ngroups]);
-                t0 = k * q.chunk_tiles;
-                t1 = min(q.ntiles, t0 + q.chunk_tiles);
-            }
-            filter_item<BF, MASK, LO>(a, st, grp, t0, t1, lane);
-        }
-    }
+    // bf16: per-wave lo fragments (kLoChunks chunk fragments x 64 lanes)
+    __shared__ uint4 lo_lds[BF ? kWavesPerBlock * kLoChunks * 64 : 1];
+    Stage st{stage_lds[threadIdx.x >> 6], 0u, BF ? lo_lds + (threadIdx.x >> 6) * kLoChunks * 64 : lo_lds};
+    for_each_item<LIST>(a.counters, a.groups, q, l, [&](uint32_t grp, uint32_t t0, uint32_t t1) __attribute__((always_inline)) {
+        filter_item<BF, MASK>(a, st, grp, t0, t1, lane);
+    });
     stage_flush(a, st);
 }
 
-// The bf16 filter in its hi-only form (BF) and the FP32 filter.  The bf16
-// form fits in 168 VGPRs for three waves per SIMD (a few values spilled,
-// reloaded only where staged records are flushed and between work items;
-// 1.6% faster than two waves at 180 VGPRs); the FP32 form keeps its 210-220.
-template <bool BF, bool MASK, bool LIST>
-__global__ __launch_bounds__(kThreads, BF ? 3 : 1) void filter_persistent_kernel(FilterArgs a, WorkQueue q, ListArgs l)
+// The FP32 filter (210-220 VGPRs).
+template <bool MASK, bool LIST>
+__global__ __launch_bounds__(kThreads, 1) void filter_fp32_kernel(FilterArgs a, WorkQueue q, ListArgs l)
 {
-    filter_body<BF, MASK, LIST, false>(a, q, l);
+    filter_body<false, MASK, LIST>(a, q, l);
 }
 
-// The bf16 filter in its lazy-lo form (80 KiB of LDS per block: two blocks
-// per CU, so two waves per SIMD and at most 256 registers).
+// The split-BF16 filter (80 KiB of LDS per block: two blocks per CU, so two
+// waves per SIMD and at most 256 registers).
 template <bool MASK, bool LIST>
 __global__ __launch_bounds__(kThreads, 2) void filter_lo_kernel(FilterArgs a, WorkQueue q, ListArgs l)
 {
-    filter_body<true, MASK, LIST, true>(a, q, l);
+    filter_body<true, MASK, LIST>(a, q, l);
 }
 
 struct FinalizeArgs {
@@ -1022,7 +1038,8 @@ __global__ __launch_bounds__(kThreads) void finalize_kernel(FinalizeArgs a)
 #ifndef BLAMM_INSTANTIATE   // small kernels: launched from the main unit only
 static __global__ void zero_counters_kernel(unsigned long long* c)
 {
-    if (threadIdx.x < kCntSlots) c[threadIdx.x] = 0ull;
+    for (uint32_t i = threadIdx.x; i < (uint32_t)kCntHeads; i += 64) c[i] = 0ull;
+    for (uint32_t i = threadIdx.x; i < (uint32_t)kQueues; i += 64) c[kCntHeads + i * kCntLine] = 0ull;
 }
 
 // Run-start bits for finalize_kernel: bit i is set when a run starts at base
@@ -1177,7 +1194,6 @@ static __global__ __launch_bounds__(kGroupThreads) void group_scatter_kernel(Gro
     }
 }
 #endif  // BLAMM_INSTANTIATE
-static_assert(kCntQueue + kXcds <= kCntSlots, "queue counters");
 
 // Column blocks of a batch: batch slot s takes the fragments of library slot
 // slot_map[s] (an empty slot gets zero weights).  Bands are the library's

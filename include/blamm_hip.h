@@ -55,9 +55,10 @@ enum blamm_status {
 
 enum blamm_precision {
     BLAMM_PREC_FP32 = 0,      /* FP32 MFMA, FP32 accumulate */
-    BLAMM_PREC_BF16X2 = 1,    /* PWM split into bf16 hi+lo; the filter multiplies the hi
-                                 terms on BF16 MFMA (FP32 accumulate) and keeps every
-                                 window the proven hi-only band cannot rule out */
+    BLAMM_PREC_BF16X2 = 1,    /* default.  The filter is an integer upper bound of every
+                                 window's score (exact sums on the matrix cores) and keeps
+                                 every window the bound cannot rule out; histograms use
+                                 the PWM split into bf16 hi+lo */
     BLAMM_PREC_BF16X2_LO = 2  /* PWM split into bf16 hi+lo; tile blocks the hi terms do
                                  not rule out also get their lo products on BF16 MFMA */
 };
@@ -197,12 +198,16 @@ int blamm_hip_last_stats(blamm_hip_ctx *ctx, blamm_scan_stats *stats);
  * filter, set directly or by blamm_hip_autotune().
  * ------------------------------------------------------------------------ */
 typedef struct blamm_tuning {
-    uint32_t chunk_tiles;      /* window tile: 32-window tiles per work item */
+    uint32_t chunk_tiles;      /* window tile: 32-window tiles per work item at
+                                  most (smaller scans use smaller items) */
     uint32_t blocks_per_wave;  /* motif tile: column blocks (32 bf16 / 16 fp32
                                   columns each) a wave scores at once: 1, 2
-                                  (bf16 at most 2, fp32 at most 4) */
+                                  (bf16 at most 2, fp32 at most 4); the default
+                                  form scores 4 times as many blocks of motifs
+                                  up to 16 positions, twice as many up to 32 */
     uint32_t kpad_positions;   /* K-padding: a block's motif length is rounded
-                                  up to a multiple of 4 or 8 positions */
+                                  up to a multiple of 4 or 8 positions (the
+                                  default form: always 16) */
 } blamm_tuning;
 
 int blamm_hip_get_tuning(blamm_hip_ctx *ctx, blamm_tuning *t);
