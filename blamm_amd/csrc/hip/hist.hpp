@@ -6,17 +6,22 @@ namespace {
 
 // Bin parameters of every library slot for histograms on [mins[col],
 // maxs[col]] with nbins bins (kernels in hist_kernels.hpp).
-void hist_slot_params(const blamm_hip_ctx* c, const float* mins, const float* maxs, uint32_t nbins,
-                      std::vector<HistSlot>& hs)
+// clamp[block]: some column's scores may leave [-0.5, nbins + 0.5] bins (mask:
+// windows may hold lowercase bases).
+void hist_slot_params(const blamm_hip_ctx* c, const float* mins, const float* maxs, uint32_t nbins, bool mask,
+                      std::vector<HistSlot>& hs, std::vector<char>& clamp)
 {
-    hs.assign((size_t)c->nslots, HistSlot{0.f, 0.f, -1.f, 0.f, 0.f, 0.f, 0u, 0u});
+    // hm < 0 and fthr = 2^32 - 1: every window binned exactly
+    const HistSlot none{0.f, 0.f, -1.f, 1.5f, ~0u, 0.f, 0.f, 0u};
+    hs.assign((size_t)c->nslots, none);
+    clamp.assign((size_t)c->nslots / kBf16Cols + 1, 0);
     std::vector<uint32_t> blk_nch((size_t)c->nslots / kBf16Cols + 1, kMaxChunks);
     for (const GroupInfo& g : c->groups)
         for (uint32_t i = 0; i < g.nb; ++i) blk_nch[g.blk0 + i] = g.nch;
     for (int s = 0; s < c->nslots; ++s) {
         const int col = c->slot_col_h[s];
         if (col < 0) continue;
-        HistSlot h{0.f, 0.f, -1.f, 0.f, 0.f, 0.f, 0u, 0u};   // hm < 0: every window binned exactly
+        HistSlot h = none;
         const int L = c->lib_len[col];
         const float mn = mins[col], mx = maxs[col];
         const float wd = (mx - mn) / (float)nbins;          // motif.h:64
@@ -25,19 +30,24 @@ void hist_slot_params(const blamm_hip_ctx* c, const float* mins, const float* ma
         h.len = (uint32_t)L;
         const float* w = c->lib_P.data() + (size_t)col * c->ldp;
         double smax = 0.0, ssplit = 0.0, rep = 0.0;   // sum_p max_b |w|, |hi| + |lo|, |w - hi - lo|
+        double least = 0.0, most = 0.0;               // sums of the least and largest weights
         for (int p = 0; p < L; ++p) {
-            double m = 0.0, ms = 0.0, me = 0.0;
+            double m = 0.0, ms = 0.0, me = 0.0, wl = mask ? 0.0 : w[4 * p], wm = wl;
             for (int b = 0; b < 4; ++b) {
                 const float x = w[4 * p + b];
                 const float hf = bf16_to_float(bf16_rne(x));
                 const float lf = bf16_to_float(bf16_rne(x - hf));
                 m = std::max(m, (double)std::fabs(x));
+                wl = std::min(wl, (double)x);
+                wm = std::max(wm, (double)x);
                 ms = std::max(ms, std::fabs((double)hf) + std::fabs((double)lf));
                 me = std::max(me, std::fabs((double)x - (double)hf - (double)lf));
             }
             smax += m;
             ssplit += ms;
             rep += me;
+            least += wl;
+            most += wm;
         }
         // |MFMA score - FP32 left-to-right score|.  MFMA side: the split's
         // representation error plus the accumulation error.  A window's row
@@ -55,6 +65,8 @@ void hist_slot_params(const blamm_hip_ctx* c, const float* mins, const float* ma
             h.iw = 0.f;
             h.c = 0.5f;
             h.hm = 0.5f;
+            h.fc = 1.5f;
+            h.fthr = 0u;
         } else if (std::isfinite(mn) && std::isfinite(wd) && wd > 0.f) {
             const float iw = 1.0f / wd;
             const float cf = -(mn * iw);
@@ -77,6 +89,19 @@ void hist_slot_params(const blamm_hip_ctx* c, const float* mins, const float* ma
                 h.iw = iw;
                 h.c = cf;
                 h.hm = hmf;
+                // fixed point: fc (or, clamped, the fma) and the sum with
+                // 2^kHistInt are rounded to half a unit each, so with e = one
+                // unit (and FP32's rounding of a far-off fc) and the bias
+                // M = m + e the FP32 score's coordinate lies in
+                // [v - 1 - 2 M, v - 1]: in the unit interval of v - 1 when
+                // fract(v) >= 2 M
+                const double unit = std::ldexp(1.0, -kHistFrac);
+                const double M = m + unit + (std::fabs((double)cf) + 2.0) * 0x1p-23;
+                h.fc = (float)(std::nearbyint(((double)cf + 1.0 + M) / unit) * unit);
+                h.fthr = (uint32_t)((uint64_t)std::ceil(2.0 * M / unit) << (32 - kHistFrac));
+                const double lo = (least - ds - (double)mn) * inv, hi = (most + ds - (double)mn) * inv;
+                if (lo < -0.5 || hi > (double)nbins + 0.5 || std::fabs((double)cf) > 1000.0)
+                    clamp[(size_t)s / kBf16Cols] = 1;
             }
         }
         hs[(size_t)s] = h;
@@ -128,18 +153,20 @@ int blamm_hip_hist_device(blamm_hip_ctx* c, const uint64_t* d_packed, uint64_t p
     if (qend > nbases) qend = nbases;
 
     std::vector<HistSlot> hs;
-    hist_slot_params(c, min_score, max_score, nbins, hs);
+    std::vector<char> clamp;
+    const bool mask = d_lcmask != nullptr;
+    hist_slot_params(c, min_score, max_score, nbins, mask, hs, clamp);
     // one column block per work item (the kernel keeps one block's
     // fragments in registers at four waves per SIMD); its histograms live in
     // LDS when its 32 columns x nbins counters fit
-    const bool lds = (uint64_t)nbins * kBf16Cols * 4 <= kHistLdsBytes;
+    const bool lds = nbins <= kHistMaxBins;
     // blocks of motifs up to 32 positions first, then the wide ones (their
     // own launch at two waves per SIMD)
     std::vector<uint32_t> groups;
     for (int pass = 0; pass < 2; ++pass)
         for (const GroupInfo& g : c->groups)
             if ((g.nch > (uint32_t)kWideChunks) == (pass == 1))
-                for (uint32_t i = 0; i < g.nb; ++i) groups.push_back(group_pack(g.blk0 + i, g.nch, 1));
+                for (uint32_t i = 0; i < g.nb; ++i) groups.push_back(group_pack(g.blk0 + i, g.nch, clamp[g.blk0 + i] ? 2 : 1));
     uint32_t nnarrow = 0;
     for (const GroupInfo& g : c->groups)
         if (g.nch <= (uint32_t)kWideChunks) nnarrow += g.nb;
@@ -150,8 +177,7 @@ int blamm_hip_hist_device(blamm_hip_ctx* c, const uint64_t* d_packed, uint64_t p
     HIP_TRY(hipMemcpyAsync(c->hist_slots.p, hs.data(), hs.size() * sizeof(HistSlot), hipMemcpyHostToDevice, s));
     HIP_TRY(hipMemcpyAsync(c->hist_groups.p, groups.data(), groups.size() * sizeof(uint32_t), hipMemcpyHostToDevice,
                            s));
-    const bool mask = d_lcmask != nullptr;
-    const uint32_t dyn = lds ? kBf16Cols * nbins * 4 : 0u;
+    const uint32_t dyn = lds ? hist_words(nbins) * 4 : 0u;
 
     HistArgs a{};
     a.packed = d_packed;
@@ -184,9 +210,11 @@ int blamm_hip_hist_device(blamm_hip_ctx* c, const uint64_t* d_packed, uint64_t p
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kp, kThreads, dyn) != hipSuccess || per_cu < 1)
             per_cu = 1;
         const uint32_t grid = (uint32_t)c->num_cu * (uint32_t)per_cu;
-        // about four items per workgroup, 16..1024 tiles per item
-        const uint64_t want = ((uint64_t)w.ntiles * w.ngroups + 4ull * grid - 1) / (4ull * grid);
-        w.chunk_tiles = (uint32_t)std::min<uint64_t>(1024, std::max<uint64_t>(16, want));
+        // about two items per workgroup, 64..1024 tiles per item: every item
+        // adds its histogram to HBM, which bounds the small calls (400 kbp x
+        // 64 columns: 0.12 ms at 16 tiles, 0.08 at 64)
+        const uint64_t want = ((uint64_t)w.ntiles * w.ngroups + 2ull * grid - 1) / (2ull * grid);
+        w.chunk_tiles = (uint32_t)std::min<uint64_t>(1024, std::max<uint64_t>(64, want));
         const uint64_t nchunks = (w.ntiles + w.chunk_tiles - 1) / w.chunk_tiles;
         if (nchunks * w.ngroups >= (1ull << 32)) return fail(BLAMM_ERR_ARG, "hist: work list too long");
         w.nitems = (uint32_t)(nchunks * w.ngroups);
