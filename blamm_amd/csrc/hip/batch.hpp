@@ -400,8 +400,10 @@ int batch_enqueue_kernels(blamm_hip_batch* b, bool mask, uint32_t grid)
         ga.slot_map = b->slot_map.p;
         ga.lib_a = (const uint4*)c->frag_a.p;
         ga.lib_b = (const uint4*)c->frag_b.p;
-        ga.lib_w = (const float*)c->frag_a.p;
-        ga.lib_band = c->slot_band_any.p;
+        const bool three = !bf && !mask;
+        ga.lib_w = three ? c->frag3.p : (const float*)c->frag_a.p;
+        ga.rows = three ? kFp32Rows3 : kMaxLen;
+        ga.lib_band = three ? c->slot_off3.p : c->slot_band_any.p;
         ga.lib_band_hi = c->slot_band_hi_any.p;
         ga.out_a = b->frag_a.p;
         ga.out_b = b->frag_b.p;
@@ -725,7 +727,6 @@ int blamm_hip_batch_submit(blamm_hip_batch* b, const blamm_request* reqs, uint32
     const size_t nslots = (size_t)c->nslots;
     const uint32_t cpb = (uint32_t)c->cols_per_blk;
     const bool bf = prec_bf(c->precision), screen = prec_screen(c->precision);
-    const uint32_t nbmax = std::min<uint32_t>(c->tuning.blocks_per_wave, bf ? kNbMaxBf16 : kNbMaxFp32);
     const int kstep = (int)c->tuning.kpad_positions / 4;
 
     // Each request's selected columns (finite or -inf threshold), in library
@@ -769,7 +770,7 @@ int blamm_hip_batch_submit(blamm_hip_batch* b, const blamm_request* reqs, uint32
             size_t e = i;
             while (e < nchs.size() && nchs[e] == nchs[i]) ++e;
             size_t bb = i;
-            const uint32_t nbg = nchs[i] > kWideChunks ? 1u : nbmax;
+            const uint32_t nbg = group_blocks(c, (uint32_t)nchs[i]);
             for (uint32_t nb = nbg; nb >= 1; nb /= 2)
                 while (e - bb >= nb) {
                     gr.push_back({blk_first + (uint32_t)bb, (uint32_t)nchs[i], nb});

@@ -183,6 +183,8 @@ struct blamm_hip_ctx {
     std::vector<double> band_h, seq_h;         // per slot
     double max_filter_band = 0.0, max_score_error = 0.0;
     DevBuf<uint8_t> frag_a, frag_b;
+    DevBuf<float> frag3;                       // FP32 form: three products per position
+    DevBuf<double> slot_off3;                  // and what its threshold is lowered by
     DevBuf<float> slot_thr, slot_w, slot_w2;   // w2: FP32 sums of position pairs
     DevBuf<double> slot_band, slot_band_any, slot_seq;   // band_any: valid in a block of any length
     DevBuf<double> slot_band_hi, slot_band_hi_any;      // hi-only stage of the bf16 filter
@@ -323,6 +325,14 @@ std::vector<GroupInfo> screen_groups(const std::vector<int>& blk_len, uint32_t b
     return out;
 }
 
+// Column blocks of a group of nch chunks (FP32 and split-BF16 forms).
+uint32_t group_blocks(const blamm_hip_ctx* c, uint32_t nch)
+{
+    const uint32_t unit = c->tuning.blocks_per_wave;
+    if (!prec_bf(c->precision)) return (uint32_t)fp32_blocks((int)nch, (int)unit);
+    return nch > kWideChunks ? 1u : std::min<uint32_t>(unit, kNbMaxBf16);
+}
+
 // Lay the stored library out for the kernels under the context's tuning and
 // upload it.
 int relayout(blamm_hip_ctx* c)
@@ -332,7 +342,6 @@ int relayout(blamm_hip_ctx* c)
     const int* lengths = c->lib_len.data();
     const float* P = c->lib_P.data();
     const int cols_per_blk = bf ? kBf16Cols : kFp32Cols;
-    const uint32_t nbmax = std::min<uint32_t>(c->tuning.blocks_per_wave, bf ? kNbMaxBf16 : kNbMaxFp32);
     const int kstep = (int)c->tuning.kpad_positions / 4;   // chunk granularity
 
     // Columns by non-decreasing length (stable); consecutive runs of
@@ -355,7 +364,7 @@ int relayout(blamm_hip_ctx* c)
         nch = std::min(kMaxChunks, (nch + kstep - 1) / kstep * kstep);
         blk_nch.push_back(nch);
     }
-    // Groups: runs of equal chunk count cut into nbmax blocks (one block for
+    // Groups: runs of equal chunk count cut into group_blocks() blocks (one for
     // motifs longer than 4 kWideChunks positions), the remainder into
     // smaller powers of two, so no padding block is scored.
     std::vector<GroupInfo> groups;
@@ -365,7 +374,7 @@ int relayout(blamm_hip_ctx* c)
         while (e < blocks.size() && blk_nch[e] == blk_nch[i]) ++e;
         size_t b = i;
         max_nch = std::max(max_nch, blk_nch[i]);
-        const uint32_t nbg = blk_nch[i] > kWideChunks ? 1u : nbmax;
+        const uint32_t nbg = group_blocks(c, (uint32_t)blk_nch[i]);
         for (uint32_t nb = nbg; nb >= 1; nb /= 2)
             while (e - b >= nb) {
                 groups.push_back({(uint32_t)b, (uint32_t)blk_nch[i], nb});
@@ -392,6 +401,7 @@ int relayout(blamm_hip_ctx* c)
     std::vector<uint32_t> s_col(nslots, 0);
     std::vector<double> s_band(nslots, 0.0), s_band_any(nslots, 0.0), s_seq(nslots, 0.0);
     std::vector<double> s_band_hi(nslots, 0.0), s_band_hi_any(nslots, 0.0);
+    std::vector<double> s_off3(bf ? 0 : nslots, 0.0);
     std::vector<uint16_t> hi16((size_t)nslots * kMaxLen * 4, 0), lo16((size_t)nslots * kMaxLen * 4, 0);
     double max_band = 0.0, max_err = 0.0;
     const double u24 = std::ldexp(1.0, -24), u53 = std::ldexp(1.0, -53);
@@ -404,7 +414,20 @@ int relayout(blamm_hip_ctx* c)
             const int L = lengths[col];
             const float* w = P + (size_t)col * ldp;
             double sum_max = 0.0, sum_split = 0.0, rep_err = 0.0, sum_lo = 0.0;
+            double off3 = 0.0, sum3 = 0.0, rep3 = 0.0;
             for (int p = 0; p < L; ++p) {
+                if (!bf) {
+                    double m3 = 0.0, e3 = 0.0;
+                    for (int b = 0; b < 3; ++b) {
+                        const double exact = (double)w[4 * p + b] - (double)w[4 * p + 3];
+                        const float d = (float)exact;
+                        m3 = std::max(m3, (double)std::fabs(d));
+                        e3 = std::max(e3, std::fabs(exact - (double)d) + std::fabs(exact) * u53);
+                    }
+                    off3 += (double)w[4 * p + 3];
+                    sum3 += m3;
+                    rep3 += e3;
+                }
                 double mx = 0.0, mxs = 0.0, me = 0.0, ml = 0.0;
                 for (int b = 0; b < 4; ++b) {
                     const float x = w[4 * p + b];
@@ -437,6 +460,16 @@ int relayout(blamm_hip_ctx* c)
             // roundoff 2^-22 to allow for truncating accumulation.
             const double nterms = bf ? 32.0 * nch : 16.0 * nch;
             const double band = 2.0 * (rep_err + gamma_n(nterms, std::ldexp(1.0, -22)) * sum_split + fp64_err) + 1e-30;
+            if (!bf && !(sum3 < 0x1p126))
+                // differences or their sums out of FP32's range: the column's
+                // entries stay zero and every window is a record
+                s_off3[slot] = INFINITY;
+            else if (!bf)
+                // three products per position: the threshold loses the
+                // constant sum and a band as above (any block: 12 entries per
+                // chunk; the constant's own rounding)
+                s_off3[slot] = off3 + 2.0 * (rep3 + gamma_n(12.0 * max_nch, std::ldexp(1.0, -22)) * sum3 + fp64_err +
+                                             gamma_n(L, u53) * sum_max) + 1e-30;
             // a batch may place the column in a block of any chunk count the
             // library has
             const double nterms_any = bf ? 32.0 * max_nch : 16.0 * max_nch;
@@ -494,6 +527,21 @@ int relayout(blamm_hip_ctx* c)
                 }
         fb.assign(16, 0);
     }
+    std::vector<float> f3;
+    if (!bf) {
+        // [block][MFMA][lane]: lane l holds entry f = 4 i + l/16 of column
+        // l%16, the FP32 difference w[f/3][f%3] - w[f/3][T]
+        f3.assign((size_t)nblk * kFp32Rows3 * 64, 0.f);
+        for (int bi = 0; bi < nblk; ++bi)
+            for (int i = 0; i < kFp32Rows3; ++i)
+                for (int l = 0; l < 64; ++l) {
+                    const int f = 4 * i + (l >> 4);
+                    const int slot = bi * kFp32Cols + (l & 15);
+                    if (!std::isfinite(s_off3[slot])) continue;
+                    const float* w = &s_w[((size_t)slot * kMaxLen + f / 3) * 4];
+                    f3[((size_t)bi * kFp32Rows3 + i) * 64 + l] = (float)((double)w[f % 3] - (double)w[3]);
+                }
+    }
     std::vector<uint32_t> gpk(scan_groups.size());
     for (size_t g = 0; g < scan_groups.size(); ++g)
         gpk[g] = group_pack(scan_groups[g].blk0, scan_groups[g].nch, scan_groups[g].nb);
@@ -502,6 +550,12 @@ int relayout(blamm_hip_ctx* c)
     HIP_TRY(hipStreamSynchronize(c->stream));
     HIP_TRY(c->frag_a.reserve(fa.size()));
     HIP_TRY(c->frag_b.reserve(fb.size()));
+    if (!bf) {
+        HIP_TRY(c->frag3.reserve(f3.size()));
+        HIP_TRY(c->slot_off3.reserve(nslots));
+        HIP_TRY(hipMemcpy(c->frag3.p, f3.data(), f3.size() * sizeof(float), hipMemcpyHostToDevice));
+        HIP_TRY(hipMemcpy(c->slot_off3.p, s_off3.data(), nslots * sizeof(double), hipMemcpyHostToDevice));
+    }
     HIP_TRY(c->slot_thr.reserve(nslots));
     HIP_TRY(c->slot_band.reserve(nslots));
     HIP_TRY(c->slot_band_any.reserve(nslots));
@@ -572,10 +626,11 @@ FilterArgs filter_args(const blamm_hip_ctx* c, const uint64_t* packed, const uin
     FilterArgs a;
     a.packed = packed;
     a.lcmask = lcmask;
-    a.frag_a = c->frag_a.p;
+    const bool three = c->precision == BLAMM_PREC_FP32 && !lcmask;
+    a.frag_a = three ? (const void*)c->frag3.p : (const void*)c->frag_a.p;
     a.frag_b = c->frag_b.p;
     a.thr = thr;
-    a.band = c->slot_band.p;
+    a.band = three ? c->slot_off3.p : c->slot_band.p;
     a.band_hi = c->slot_band_hi.p;
     a.groups = c->scan_groups_d.p;
     a.cand = cand;
@@ -696,7 +751,7 @@ int blamm_hip_destroy(blamm_hip_ctx* c)
     if (!c) return BLAMM_OK;
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
-    c->frag_a.release(); c->frag_b.release(); c->slot_thr.release(); c->slot_band.release();
+    c->frag_a.release(); c->frag_b.release(); c->frag3.release(); c->slot_off3.release(); c->slot_thr.release(); c->slot_band.release();
     c->slot_band_any.release(); c->slot_band_hi.release(); c->slot_band_hi_any.release();
     c->slot_seq.release(); c->slot_w.release(); c->slot_w2.release();
     c->slot_len.release(); c->slot_col.release(); c->scan_groups_d.release(); c->cand.release();

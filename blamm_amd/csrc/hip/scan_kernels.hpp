@@ -105,6 +105,15 @@ __device__ __forceinline__ float thr_plus(float t, double b)
     return __double2float_ru(d);
 }
 
+// Largest float <= t - b for b of either sign (the margin covers the rounding
+// of the difference).
+__device__ __forceinline__ float thr_less(float t, double b)
+{
+    if (!__builtin_isfinite(t)) return t;
+    const double d = (double)t - b;
+    return __double2float_rd(d - (__builtin_fabs((double)t) + __builtin_fabs(b)) * 0x1p-50 - 0x1p-1000);
+}
+
 // A column group is nb consecutive blocks of one length class (nch chunks of
 // 4 positions), scored together by one wave.
 __host__ __device__ constexpr uint32_t group_pack(uint32_t blk0, uint32_t nch, uint32_t nb)
@@ -197,22 +206,12 @@ __device__ __forceinline__ const V& acc_read(const V& acc)
     return acc;
 }
 
-// 64 bits of the 128-bit value (hi:lo) starting at bit s (0 <= s < 64),
-// without a branch for s == 0.
-__device__ __forceinline__ uint64_t funnel64(uint64_t lo, uint64_t hi, uint32_t s, uint32_t s_inv)
-{
-    return (lo >> s) | ((hi << 1) << s_inv);   // s_inv = 63 - s
-}
-
 __device__ __forceinline__ uint32_t funnel32(uint32_t lo, uint32_t hi, uint32_t s)
 {
     return __builtin_amdgcn_alignbit(hi, lo, s);
 }
 
-// Tiles are 32 consecutive windows; a wave walks tiles [t0, t1) of its
-// range.  The FP32 loop keeps a register window of kGroup+1 packed words and
-// prefetches the next group's words one group ahead.
-constexpr int kGroup = 4;
+// Tiles are 32 consecutive windows; a wave walks tiles [t0, t1) of its range.
 
 // The split-BF16 filter (BLAMM_PREC_BF16X2_LO) is software-pipelined over two
 // accumulator sets: a tile block whose hi-only score can reach the threshold
@@ -464,112 +463,158 @@ __device__ __forceinline__ void bf16_range(const FilterArgs& a, Stage& st, uint3
 }
 
 // ---------------------------------------------------------------------------
-// FP32 filter: v_mfma_f32_16x16x4_f32, one motif position per MFMA.
-// A = one-hot (16 windows x 4 bases), B = W_c[p][.] (4 x 16 columns).
-// Lane l: A[l%16][l/16], B[l/16][l%16]; D lane l holds column l%16,
-// rows 4(l/16) + r.  A 32-window tile is two 16-window sub-tiles.
+// FP32 filter: v_mfma_f32_16x16x4_f32, A = one-hot entries (16 windows x 4),
+// B = weights (4 x 16 columns).  Lane l: A[l%16][l/16], B[l/16][l%16]; D lane
+// l holds column l%16, rows 4(l/16) + r.  A 32-window tile is two 16-window
+// sub-tiles.
+// Bound by the matrix cores (32 cycles an MFMA), so entries are saved:
+//  - without a lowercase mask a window has one base per position, and its
+//    score is the sum of w[p][T] (a constant, taken off the threshold) plus
+//    d[p][b] = w[p][b] - w[p][T] for the positions that hold b = A, C or G:
+//    three entries per position, four positions in 3 MFMAs.  Entry f = 3 p + b
+//    is k = f % 4 of MFMA f / 4.
+//  - a lowercase base has none of the four, which the constant cannot
+//    express: with a mask one MFMA per position, k = base.
+// The entries: the window's codes, shifted to the lane's first position of an
+// MFMA, are compared with the lane's base for 16 positions at once, which
+// leaves a byte 0 or 1 per chunk of four positions; v_cvt_f32_ubyte makes the
+// operand, one instruction per MFMA where a test per position took five.
+// 6 Mbp x 1,000 columns of 5..30 positions: 8.9 ms with four entries, two
+// blocks per wave and a test per position; 6.3 ms with three entries, 5.8 ms
+// with up to four blocks per wave too (the matrix cores alone need 4.7 ms).
+// 24 Mbp x 1,000 of 6..25 positions with a mask: 35.0 -> 27.0 ms.
 // ---------------------------------------------------------------------------
-template <int NCH, int NB, bool MASK>
-__device__ __forceinline__ void fp32_subtile(const FilterArgs& a, Stage& st, const float (&bw)[NB][4 * NCH],
-                                             const float (&th)[NB], uint32_t q0,
-                                             uint64_t bits, uint64_t bits2, uint64_t mb, uint32_t k, uint32_t blk0,
-                                             uint32_t lane)
+constexpr int kFp32Rows3 = 3 * kMaxChunks;   // MFMAs of the longest column, three entries per position
+
+// Column blocks one wave scores at once for blocks of nch chunks, for motif
+// tile 1, 2 (the default) or 4.  The operand of a tile is built once for all
+// of them; up to 24 chunks of weights (72 registers, 96 with a mask) leave
+// room for three waves per SIMD (two), so that another wave's products run
+// while one builds operands and checks scores.
+__host__ __device__ constexpr int fp32_blocks(int nch, int unit)
 {
-    constexpr int NP = 4 * NCH;
-    f32x4 acc[NB];
-#pragma unroll
-    for (int b = 0; b < NB; ++b) acc[b] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int p = 0; p < NP; ++p) {
-        const uint32_t base = (uint32_t)((p < 32 ? bits >> (2 * p) : bits2 >> (2 * (p - 32)))) & 3u;
-        bool on = (base == k);
-        if (MASK) on = on && !((mb >> p) & 1);
-        const float av = on ? 1.0f : 0.0f;
-#pragma unroll
-        for (int b = 0; b < NB; ++b)
-            acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, bw[b][p], acc[b], 0, 0, 0);
-    }
-    const uint32_t qlane = q0 + 4 * k;     // windows qlane + 0..3
-    const f32x4 (&av)[NB] = acc_read<AccRead::kGuard>(acc);
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-        const float v[4] = {av[b][0], av[b][1], av[b][2], av[b][3]};
-        emit_rows<4>(a, st, v, th[b], qlane, (blk0 + b) * kFp32Cols + (lane & 15));
-    }
+    const int most = nch <= 6 ? 4 : nch <= kWideChunks ? 2 : 1;
+    return 2 * unit < most ? 2 * unit : most;
 }
 
-// Tiles [t0, t1) of column blocks blk0 .. blk0+NB-1 (FP32 path).  A register
-// window of kGroup + 2 packed words covers a group of tiles and the 64 bases
-// past its last window; the next group's words are loaded a group ahead.
+template <int NCH, bool MASK>
+struct Fp32Rows {
+    static constexpr int NH = (NCH + 3) / 4;   // dwords of 16 positions
+    static constexpr int NJ = MASK ? 4 : 3;    // MFMAs per chunk
+    uint32_t z[NJ][NH];                        // byte g of z[j][h]: chunk 4 h + g, MFMA j
+    // d: packed dwords from sub-tile u's first window on; m: mask dwords of the tile
+    __device__ __forceinline__ void build(const uint32_t* d, const uint32_t* m, int u, uint32_t i,
+                                          const uint32_t (&sj)[NJ], const uint32_t (&tj)[NJ])
+    {
+        uint32_t x[NH], low[NH];
+#pragma unroll
+        for (int h = 0; h < NH; ++h) x[h] = funnel32(d[h], d[h + 1], 2 * i);
+        if constexpr (MASK) {
+#pragma unroll
+            for (int h = 0; h < NH; ++h) {     // byte g: lowercase flags of chunk 4 h + g
+                const int q = (u + h) / 2;
+                uint32_t f = (u + h) % 2 ? funnel32(m[q], m[q + 1], i + 16) : m[q] >> i;
+                f &= 0xFFFFu;
+                f = (f | (f << 8)) & 0x00FF00FFu;
+                low[h] = f | (f << 4);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int h = 0; h < NH; ++h) {
+                uint32_t y = (x[h] >> sj[j]) ^ tj[j];
+                y |= y >> 1;
+                if constexpr (MASK) y |= low[h] >> j;
+                z[j][h] = ~y & 0x01010101u;
+            }
+    }
+    __device__ __forceinline__ float entry(int c, int j) const
+    {
+        return (float)((z[j][c >> 2] >> (8 * (c & 3))) & 0xFFu);
+    }
+};
+
+// Tiles [t0, t1) of column blocks blk0 .. blk0+NB-1 (FP32 path).
 template <int NCH, int NB, bool MASK>
 __device__ __forceinline__ void fp32_range(const FilterArgs& a, Stage& st, uint32_t blk0, uint32_t t0, uint32_t t1,
                                            uint32_t lane)
 {
-    static_assert(NCH <= kWideChunks || NB == 1, "wide blocks are scored one per wave");
+    static_assert(NB <= fp32_blocks(NCH, 4), "weights exceed the registers");
+    using Rows = Fp32Rows<NCH, MASK>;
+    constexpr int NJ = Rows::NJ, NH = Rows::NH, R = MASK ? kMaxLen : kFp32Rows3;
     const float* __restrict__ fw = (const float*)a.frag_a;
-    constexpr int NP = 4 * NCH;
-    constexpr bool WIDE = NCH > kWideChunks;
-    float bw[NB][NP];
+    float bw[NB][NJ * NCH];
     float th[NB];
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
 #pragma unroll
-        for (int p = 0; p < NP; ++p) bw[b][p] = fw[((size_t)(blk0 + b) * kMaxLen + p) * 64 + lane];
+        for (int r = 0; r < NJ * NCH; ++r) bw[b][r] = fw[((size_t)(blk0 + b) * R + r) * 64 + lane];
         const uint32_t slot = (blk0 + b) * kFp32Cols + (lane & 15);
-        th[b] = thr_minus(a.thr[slot], a.band[slot]);
+        th[b] = MASK ? thr_minus(a.thr[slot], a.band[slot]) : thr_less(a.thr[slot], a.band[slot]);
     }
     const uint32_t i = lane & 15, k = lane >> 4;
-    const uint32_t s0 = 2 * i, s1 = 2 * (i + 16);    // bit offsets of the two sub-tiles
+    uint32_t sj[NJ], tj[NJ];
+#pragma unroll
+    for (uint32_t j = 0; j < (uint32_t)NJ; ++j) {
+        sj[j] = MASK ? 2 * j : 2 * ((4 * j + k) / 3);
+        tj[j] = (MASK ? k : (4 * j + k) % 3) * 0x55555555u;
+    }
+    // dwords 2t .. 2t + NH + 1 of the packed stream and t .. t + NH/2 + 1 of
+    // the mask: tile t's windows (both sub-tiles), loaded one tile ahead
+    constexpr int NW = (NH + 3) / 2, NM = MASK ? NH / 2 + 2 : 1;
     const uint64_t* __restrict__ pk = a.packed;
     const uint32_t* __restrict__ mk = (const uint32_t*)a.lcmask;
-    uint64_t w[kGroup + 2];
-    uint32_t mw[kGroup + 2];
+    uint64_t w[NW], nx[NW];
+    uint32_t m[NM] = {}, nm[NM] = {};
 #pragma unroll
-    for (int u = 0; u <= kGroup + 1; ++u) {
-        w[u] = pk[t0 + u];
-        mw[u] = MASK ? mk[t0 + u] : 0u;
-    }
-    for (uint32_t t = t0; t < t1; t += kGroup) {
-        uint64_t nx[kGroup];
-        uint32_t nm[kGroup];
-        if (t + kGroup < t1) {
+    for (int q = 0; q < NW; ++q) w[q] = pk[t0 + q];
+    if constexpr (MASK)
 #pragma unroll
-            for (int u = 0; u < kGroup; ++u) {
-                nx[u] = pk[t + kGroup + 2 + u];
-                nm[u] = MASK ? mk[t + kGroup + 2 + u] : 0u;
-            }
+        for (int q = 0; q < NM; ++q) m[q] = mk[t0 + q];
+    for (uint32_t t = t0; t < t1; ++t) {
+#pragma unroll
+        for (int q = 0; q < NW; ++q) nx[q] = pk[t + 1 + q];
+        if constexpr (MASK)
+#pragma unroll
+            for (int q = 0; q < NM; ++q) nm[q] = mk[t + 1 + q];
+        uint32_t d[2 * NW];
+#pragma unroll
+        for (int q = 0; q < NW; ++q) {
+            d[2 * q] = (uint32_t)w[q];
+            d[2 * q + 1] = (uint32_t)(w[q] >> 32);
         }
-#pragma unroll
-        for (int u = 0; u < kGroup; ++u) {
-            if (t + u < t1) {
-                const uint32_t q0 = (t + u) * kBf16Tile;
-                const uint64_t b0 = funnel64(w[u], w[u + 1], s0, 63 - s0);
-                const uint64_t b1 = funnel64(w[u], w[u + 1], s1, 63 - s1);
-                const uint64_t c0 = WIDE ? funnel64(w[u + 1], w[u + 2], s0, 63 - s0) : 0ull;
-                const uint64_t c1 = WIDE ? funnel64(w[u + 1], w[u + 2], s1, 63 - s1) : 0ull;
-                uint64_t m0 = 0, m1 = 0;
-                if (MASK) {
-                    m0 = funnel32(mw[u], mw[u + 1], i);
-                    m1 = funnel32(mw[u], mw[u + 1], i + 16);
-                    if (WIDE) {
-                        m0 |= (uint64_t)funnel32(mw[u + 1], mw[u + 2], i) << 32;
-                        m1 |= (uint64_t)funnel32(mw[u + 1], mw[u + 2], i + 16) << 32;
-                    }
-                }
-                fp32_subtile<NCH, NB, MASK>(a, st, bw, th, q0, b0, c0, m0, k, blk0, lane);
-                fp32_subtile<NCH, NB, MASK>(a, st, bw, th, q0 + kFp32Tile, b1, c1, m1, k, blk0, lane);
-            }
-        }
+        f32x4 acc[2][NB];
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
-            w[u] = w[kGroup + u];
-            mw[u] = mw[kGroup + u];
-        }
+            Rows rows;
+            rows.build(d + u, m, u, i, sj, tj);
 #pragma unroll
-        for (int u = 0; u < kGroup; ++u) {
-            w[u + 2] = nx[u];
-            mw[u + 2] = nm[u];
+            for (int b = 0; b < NB; ++b) acc[u][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int c = 0; c < NCH; ++c)
+#pragma unroll
+                for (int j = 0; j < NJ; ++j) {
+                    const float av = rows.entry(c, j);
+#pragma unroll
+                    for (int b = 0; b < NB; ++b)
+                        acc[u][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, bw[b][NJ * c + j], acc[u][b], 0, 0, 0);
+                }
         }
+        const f32x4 (&av)[2][NB] = acc_read<AccRead::kGuard>(acc);
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                const float v[4] = {av[u][b][0], av[u][b][1], av[u][b][2], av[u][b][3]};
+                emit_rows<4>(a, st, v, th[b], t * kBf16Tile + u * kFp32Tile + 4 * k,
+                             (blk0 + b) * kFp32Cols + (lane & 15));
+            }
+#pragma unroll
+        for (int q = 0; q < NW; ++q) w[q] = nx[q];
+        if constexpr (MASK)
+#pragma unroll
+            for (int q = 0; q < NM; ++q) m[q] = nm[q];
     }
 }
 
@@ -652,7 +697,7 @@ __device__ __forceinline__ void filter_item(const FilterArgs& a, Stage& st, uint
         BLAMM_F32(1, 2) BLAMM_F32(2, 2) BLAMM_F32(3, 2) BLAMM_F32(4, 2)
         BLAMM_F32(5, 2) BLAMM_F32(6, 2) BLAMM_F32(7, 2) BLAMM_F32(8, 2)
         BLAMM_F32(1, 4) BLAMM_F32(2, 4) BLAMM_F32(3, 4) BLAMM_F32(4, 4)
-        BLAMM_F32(5, 4) BLAMM_F32(6, 4) BLAMM_F32(7, 4) BLAMM_F32(8, 4)
+        BLAMM_F32(5, 4) BLAMM_F32(6, 4)
         BLAMM_F32(9, 1) BLAMM_F32(10, 1) BLAMM_F32(11, 1) BLAMM_F32(12, 1)
         BLAMM_F32(13, 1) BLAMM_F32(14, 1) BLAMM_F32(15, 1) BLAMM_F32(16, 1)
 #undef BLAMM_F32
@@ -739,9 +784,9 @@ __device__ __forceinline__ void filter_body(const FilterArgs& a, const WorkQueue
     stage_flush(a, st);
 }
 
-// The FP32 filter (210-220 VGPRs).
+// The FP32 filter.
 template <bool MASK, bool LIST>
-__global__ __launch_bounds__(kThreads, 1) void filter_fp32_kernel(FilterArgs a, WorkQueue q, ListArgs l)
+__global__ __launch_bounds__(kThreads, MASK ? 2 : 3) void filter_fp32_kernel(FilterArgs a, WorkQueue q, ListArgs l)
 {
     filter_body<false, MASK, LIST>(a, q, l);
 }
@@ -1203,7 +1248,8 @@ struct GatherArgs {
     const uint32_t* slot_map;
     const uint4* lib_a;                   // bf16: [block][chunk][lane] hi / fp32: weights as uint4 view unused
     const uint4* lib_b;
-    const float* lib_w;                   // fp32: [block][position][lane]
+    const float* lib_w;                   // fp32: [block][row][lane]
+    uint32_t rows;                        // fp32: rows of a block
     const double* lib_band;               // per library slot, any block
     const double* lib_band_hi;            // per library slot, any block (hi-only stage)
     uint4* out_a;
@@ -1236,13 +1282,13 @@ __global__ __launch_bounds__(256) void gather_kernel(GatherArgs g)
             g.out_b[i] = vb;
         }
     } else {
-        const uint64_t total = (uint64_t)nblk * kMaxLen * 64;
+        const uint64_t total = (uint64_t)nblk * g.rows * 64;
         for (uint64_t i = t0; i < total; i += stride) {
-            const uint32_t l = (uint32_t)(i & 63), p = (uint32_t)((i >> 6) % kMaxLen);
-            const uint32_t b = (uint32_t)(i / (64 * kMaxLen));
+            const uint32_t l = (uint32_t)(i & 63), p = (uint32_t)((i >> 6) % g.rows);
+            const uint32_t b = (uint32_t)(i / (64 * (uint64_t)g.rows));
             const uint32_t lib = g.slot_map[b * cpb + (l & 15)];
             float v = 0.f;
-            if (lib != kNoSlot) v = g.lib_w[((size_t)(lib / cpb) * kMaxLen + p) * 64 + (lib % cpb) + 16 * (l >> 4)];
+            if (lib != kNoSlot) v = g.lib_w[((size_t)(lib / cpb) * g.rows + p) * 64 + (lib % cpb) + 16 * (l >> 4)];
             g.out_w[i] = v;
         }
     }

@@ -204,7 +204,9 @@ typedef struct blamm_tuning {
                                   columns each) a wave scores at once: 1, 2
                                   (bf16 at most 2, fp32 at most 4); the default
                                   form scores 4 times as many blocks of motifs
-                                  up to 16 positions, twice as many up to 32 */
+                                  up to 16 positions, twice as many up to 32;
+                                  the fp32 form twice as many, up to 4 (motifs
+                                  up to 24 positions) or 2 (up to 32) */
     uint32_t kpad_positions;   /* K-padding: a block's motif length is rounded
                                   up to a multiple of 4 or 8 positions (the
                                   default form: always 16) */
