@@ -134,6 +134,8 @@ def hip_lib() -> ctypes.CDLL:
         lib.blamm_hip_scan_finish.argtypes = [vp, _u64p]
         lib.blamm_hip_scan_pinned.argtypes = [vp, _u64p, _u64p, ctypes.c_uint64, _u64p, ctypes.c_uint64,
                                               ctypes.POINTER(vp), _u64p]
+        lib.blamm_hip_scan_keep.argtypes = [vp, _u64p, _u64p, ctypes.c_uint64, _u64p, ctypes.c_uint64, _u64p]
+        lib.blamm_hip_scan_fetch.argtypes = [vp, vp, ctypes.c_uint64]
         lib.blamm_hip_last_stats.argtypes = [vp, ctypes.POINTER(ScanStats)]
         lib.blamm_hip_get_tuning.argtypes = [vp, ctypes.POINTER(Tuning)]
         lib.blamm_hip_set_tuning.argtypes = [vp, ctypes.POINTER(Tuning)]
@@ -148,6 +150,7 @@ def hip_lib() -> ctypes.CDLL:
         lib.blamm_hip_batch_query.argtypes = [vp]
         lib.blamm_hip_batch_wait.argtypes = [vp, _u64p]
         lib.blamm_hip_batch_hits.argtypes = [vp, ctypes.c_uint32, ctypes.POINTER(vp), _u64p]
+        lib.blamm_hip_batch_read.argtypes = [vp, ctypes.c_uint32, vp, ctypes.c_uint64, _u64p]
         lib.blamm_hip_batch_stats.argtypes = [vp, ctypes.POINTER(ScanStats)]
         lib.blamm_hip_server_create.argtypes = [vp, ctypes.POINTER(ServerConfig), ctypes.POINTER(vp)]
         lib.blamm_hip_server_submit.argtypes = [vp, ctypes.POINTER(Request), _u64p]
@@ -187,6 +190,18 @@ def host_lib() -> ctypes.CDLL:
 
 def _ptr(a: np.ndarray, t):
     return a.ctypes.data_as(ctypes.POINTER(t))
+
+
+def _words(a, need: int) -> np.ndarray:
+    """The first `need` words of a packed stream or mask, for the engine to read
+    in place: the caller's array itself when it has them as aligned uint64, else
+    a copy (zeros past the end)."""
+    if (isinstance(a, np.ndarray) and a.dtype == np.uint64 and a.ndim == 1 and len(a) >= max(need, 1)
+            and a.flags.c_contiguous and a.flags.aligned):
+        return a
+    buf = np.zeros(max(need, 1), dtype=np.uint64)
+    buf[:min(len(a), need)] = a[:need]
+    return buf
 
 
 def _check(rc: int) -> None:
@@ -307,41 +322,26 @@ class HipScanner:
 
     def scan(self, codes: np.ndarray, nbases: int, run_starts=None, lower: Optional[np.ndarray] = None,
              cap: int = 1 << 20) -> np.ndarray:
-        """Scan a packed stream held in host memory; returns the hit records."""
-        pw = int(self.lib.blamm_hip_packed_words(nbases))
-        cbuf = np.zeros(pw, dtype=np.uint64)
-        cbuf[:min(len(codes), pw)] = codes[:pw]
-        mbuf = None
-        if lower is not None:
-            mw = int(self.lib.blamm_hip_mask_words(nbases))
-            mbuf = np.zeros(mw, dtype=np.uint64)
-            mbuf[:min(len(lower), mw)] = lower[:mw]
+        """Scan a packed stream held in host memory; returns the hit records
+        (as many as there are: cap is no limit)."""
+        cbuf = _words(codes, (nbases + 31) // 32)
+        mbuf = _words(lower, (nbases + 63) // 64) if lower is not None else None
         runs = np.ascontiguousarray(run_starts if run_starts is not None else [], dtype=np.uint64)
-        while True:
-            hits = np.zeros(max(cap, 1), dtype=HIT_DTYPE)
-            n = ctypes.c_uint64()
-            rc = self.lib.blamm_hip_scan(self.ctx, _ptr(cbuf, ctypes.c_uint64),
-                                         _ptr(mbuf, ctypes.c_uint64) if mbuf is not None else None,
-                                         nbases, _ptr(runs, ctypes.c_uint64) if len(runs) else None, len(runs),
-                                         hits.ctypes.data, cap, ctypes.byref(n))
-            if rc == BLAMM_ERR_OVERFLOW and n.value > cap:
-                cap = int(n.value)
-                continue
-            _check(rc)
-            return hits[:n.value].copy()
+        n = ctypes.c_uint64()
+        _check(self.lib.blamm_hip_scan_keep(self.ctx, _ptr(cbuf, ctypes.c_uint64),
+                                            _ptr(mbuf, ctypes.c_uint64) if mbuf is not None else None,
+                                            nbases, _ptr(runs, ctypes.c_uint64) if len(runs) else None, len(runs),
+                                            ctypes.byref(n)))
+        hits = np.empty(n.value, dtype=HIT_DTYPE)
+        _check(self.lib.blamm_hip_scan_fetch(self.ctx, hits.ctypes.data, n.value))
+        return hits
 
     def scan_pinned(self, codes: np.ndarray, nbases: int, run_starts=None,
                     lower: Optional[np.ndarray] = None) -> np.ndarray:
         """Scan a host stream; the engine keeps the hits in its pinned buffer
         (returned here as a copy)."""
-        pw = int(self.lib.blamm_hip_packed_words(nbases))
-        cbuf = np.zeros(pw, dtype=np.uint64)
-        cbuf[:min(len(codes), pw)] = codes[:pw]
-        mbuf = None
-        if lower is not None:
-            mw = int(self.lib.blamm_hip_mask_words(nbases))
-            mbuf = np.zeros(mw, dtype=np.uint64)
-            mbuf[:min(len(lower), mw)] = lower[:mw]
+        cbuf = _words(codes, (nbases + 31) // 32)
+        mbuf = _words(lower, (nbases + 63) // 64) if lower is not None else None
         runs = np.ascontiguousarray(run_starts if run_starts is not None else [], dtype=np.uint64)
         p = ctypes.c_void_p()
         n = ctypes.c_uint64()
@@ -349,20 +349,16 @@ class HipScanner:
                                               _ptr(mbuf, ctypes.c_uint64) if mbuf is not None else None,
                                               nbases, _ptr(runs, ctypes.c_uint64) if len(runs) else None,
                                               len(runs), ctypes.byref(p), ctypes.byref(n)))
-        return _hits_array(p.value or 0, int(n.value))
+        hits = np.empty(n.value, dtype=HIT_DTYPE)
+        _check(self.lib.blamm_hip_scan_fetch(self.ctx, hits.ctypes.data, n.value))
+        return hits
 
     def hist(self, codes: np.ndarray, nbases: int, min_scores, max_scores, num_bins: int = 250, run_starts=None,
              lower: Optional[np.ndarray] = None, qend: Optional[int] = None) -> np.ndarray:
         """Empirical histograms (hist -e) of a host stream for every library
         column: (ncols, num_bins) uint64 counts."""
-        pw = int(self.lib.blamm_hip_packed_words(nbases))
-        cbuf = np.zeros(pw, dtype=np.uint64)
-        cbuf[:min(len(codes), pw)] = codes[:pw]
-        mbuf = None
-        if lower is not None:
-            mw = int(self.lib.blamm_hip_mask_words(nbases))
-            mbuf = np.zeros(mw, dtype=np.uint64)
-            mbuf[:min(len(lower), mw)] = lower[:mw]
+        cbuf = _words(codes, (nbases + 31) // 32)
+        mbuf = _words(lower, (nbases + 63) // 64) if lower is not None else None
         runs = np.ascontiguousarray(run_starts if run_starts is not None else [], dtype=np.uint64)
         mn = np.ascontiguousarray(min_scores, np.float32)
         mx = np.ascontiguousarray(max_scores, np.float32)
@@ -453,13 +449,6 @@ class ScanRequest:
                          self.thresholds.ctypes.data if self.thresholds is not None else None, int(expected_hits))
 
 
-def _hits_array(ptr: int, n: int) -> np.ndarray:
-    if n == 0:
-        return np.zeros(0, dtype=HIT_DTYPE)
-    buf = (ctypes.c_char * (n * HIT_DTYPE.itemsize)).from_address(ptr)
-    return np.frombuffer(buf, dtype=HIT_DTYPE).copy()
-
-
 class Batch:
     """A batch slot: many requests, one captured launch sequence."""
 
@@ -498,10 +487,11 @@ class Batch:
         return int(n.value)
 
     def hits(self, req: int) -> np.ndarray:
-        p = ctypes.c_void_p()
         n = ctypes.c_uint64()
-        _check(self.lib.blamm_hip_batch_hits(self.b, req, ctypes.byref(p), ctypes.byref(n)))
-        return _hits_array(p.value or 0, int(n.value))
+        _check(self.lib.blamm_hip_batch_read(self.b, req, None, 0, ctypes.byref(n)))
+        hits = np.empty(n.value, dtype=HIT_DTYPE)
+        _check(self.lib.blamm_hip_batch_read(self.b, req, hits.ctypes.data, n.value, ctypes.byref(n)))
+        return hits
 
     def stats(self) -> ScanStats:
         st = ScanStats()

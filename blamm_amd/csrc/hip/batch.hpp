@@ -53,24 +53,9 @@ void expand_hits(const GroupedHit* in, uint64_t n, blamm_hit* out)
     }
 }
 
-// The same for a whole batch: large ones are split over up to 16 threads (a
-// single thread moves ~10 GB/s, a batch of 20M hits is 0.6 GB).
 void expand_hits_parallel(const GroupedHit* in, uint64_t n, blamm_hit* out)
 {
-    const uint64_t per = 1ull << 21;
-    const unsigned nt = (unsigned)std::min<uint64_t>({(n + per - 1) / per, 16ull,
-                                                      std::max(1u, std::thread::hardware_concurrency())});
-    if (nt <= 1) {
-        expand_hits(in, n, out);
-        return;
-    }
-    std::vector<std::thread> pool;
-    for (unsigned t = 1; t < nt; ++t) {
-        const uint64_t b = n * t / nt, e = n * (t + 1) / nt;
-        pool.emplace_back([=] { expand_hits(in + b, e - b, out + b); });
-    }
-    expand_hits(in, n / nt, out);
-    for (auto& th : pool) th.join();
+    in_parts(n, [=](uint64_t b, uint64_t e) { expand_hits(in + b, e - b, out + b); });
 }
 
 int acquire_hits(const std::shared_ptr<HitPool>& pool, size_t want, std::shared_ptr<HitBuf>* out)
@@ -954,6 +939,19 @@ int blamm_hip_batch_hits(blamm_hip_batch* b, uint32_t req, const blamm_hit** hit
     }
     *hits = b->expanded.get() + b->out_off[req];
     *n = b->out_off[req + 1] - b->out_off[req];
+    return BLAMM_OK;
+}
+
+int blamm_hip_batch_read(blamm_hip_batch* b, uint32_t req, blamm_hit* hits, uint64_t cap, uint64_t* n)
+{
+    if (!b || !n || (cap > 0 && !hits)) return fail(BLAMM_ERR_ARG, "batch_read: null pointer");
+    if (!b->done) return fail(BLAMM_ERR_STATE, "batch_read: no finished batch");
+    if (req >= b->nreq) return fail(BLAMM_ERR_ARG, "batch_read: request index out of range");
+    const uint64_t at = b->out_off[req], nh = b->out_off[req + 1] - at;
+    *n = nh;
+    if (!hits || nh == 0) return BLAMM_OK;
+    if (cap < nh) return fail(BLAMM_ERR_OVERFLOW, "batch_read: hit capacity too small");
+    expand_hits_parallel(b->out->p + at, nh, hits);
     return BLAMM_OK;
 }
 

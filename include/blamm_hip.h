@@ -150,6 +150,16 @@ int blamm_hip_scan_pinned(blamm_hip_ctx *ctx, const uint64_t *packed, const uint
                           uint64_t nbases, const uint64_t *run_starts, uint64_t nruns,
                           const blamm_hit **hits, uint64_t *nhits);
 
+/* As blamm_hip_scan, in two calls for a caller that sizes its memory by the
+ * number of hits: the first scans and keeps the hits on the device (*nhits of
+ * them), the second copies them into hits[0..cap) (BLAMM_ERR_OVERFLOW when
+ * they do not fit; BLAMM_ERR_STATE when another scan of a host stream or a
+ * blamm_hip_reserve on the context followed the first).  After
+ * blamm_hip_scan_pinned, the second copies out of its pinned buffer. */
+int blamm_hip_scan_keep(blamm_hip_ctx *ctx, const uint64_t *packed, const uint64_t *lcmask,
+                        uint64_t nbases, const uint64_t *run_starts, uint64_t nruns, uint64_t *nhits);
+int blamm_hip_scan_fetch(blamm_hip_ctx *ctx, blamm_hit *hits, uint64_t cap);
+
 /* Enqueue a scan of device-resident buffers on `stream` (a hipStream_t, or
  * NULL for the context's own stream) without synchronising.  Buffer sizes are
  * passed so they can be checked.  The hit count is written to d_nhits
@@ -282,6 +292,10 @@ int blamm_hip_batch_wait(blamm_hip_batch *batch, uint64_t *nhits);
  * position, column, score); the first call after a wait rebuilds them as
  * blamm_hit. */
 int blamm_hip_batch_hits(blamm_hip_batch *batch, uint32_t req, const blamm_hit **hits, uint64_t *n);
+/* The same into the caller's memory: *n = the request's hits, written to
+ * hits[0..cap) unless `hits` is NULL (BLAMM_ERR_OVERFLOW when they do not
+ * fit). */
+int blamm_hip_batch_read(blamm_hip_batch *batch, uint32_t req, blamm_hit *hits, uint64_t cap, uint64_t *n);
 /* kernel_ms = the whole captured launch sequence of the last batch. */
 int blamm_hip_batch_stats(blamm_hip_batch *batch, blamm_scan_stats *stats);
 
