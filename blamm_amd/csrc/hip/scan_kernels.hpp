@@ -126,10 +126,9 @@ __host__ __device__ constexpr uint32_t group_pack(uint32_t blk0, uint32_t nch, u
 // candidates per scan), so each wave collects up to kStage candidates in its
 // own LDS slice and reserves global space with one atomic per flush.  Only
 // the owning wave touches its slice; LDS operations of one wave complete in
-// program order, so no barrier is needed.  256 entries (16 KiB per block)
-// need half the reservations of 128 (measured: -0.5% per scan of 100 Mbp x
-// 2,000 columns).
-constexpr int kStage = 256;
+// program order, so no barrier is needed.  252 entries: with the split-BF16
+// filter's fragments and last_places' words just under 80 KiB per block.
+constexpr int kStage = 252;
 
 struct Stage {
     uint4* buf;        // this wave's LDS slice
@@ -137,8 +136,7 @@ struct Stage {
     uint4* lo;         // split-BF16 filter: this wave's lo fragments (LDS), [block][chunk][lane]
 };
 
-template <class Args>   // FilterArgs or HistArgs: cand, counters, cand_cap
-__device__ __forceinline__ void stage_flush(const Args& a, Stage& st)
+__device__ __forceinline__ void stage_flush(const FilterArgs& a, Stage& st)
 {
     if (st.n == 0) return;
     const uint32_t lane = threadIdx.x & 63;
@@ -150,6 +148,37 @@ __device__ __forceinline__ void stage_flush(const Args& a, Stage& st)
         if (at < a.cand_cap) a.cand[at] = st.buf[i];
     }
     st.n = 0;
+}
+
+// Reserve room behind *counter for what each wave of the workgroup still
+// holds (n) when it ends; returns the wave's first place.  Called by all
+// waves.  Reservations on one line take 11 ns each, one after the other: a
+// scan of 1 Mbp x 128 columns, where 4,096 waves end with three records each,
+// spent 47 of 74 us in them (45 us with one per workgroup).
+__device__ __forceinline__ uint64_t last_places(unsigned long long* counter, uint32_t n)
+{
+    __shared__ uint32_t held[kWavesPerBlock];
+    __shared__ unsigned long long first;
+    const uint32_t wave = threadIdx.x >> 6;
+    if ((threadIdx.x & 63) == 0) held[wave] = n;
+    __syncthreads();
+    uint32_t sum = 0, before = 0;
+    for (uint32_t w = 0; w < (uint32_t)kWavesPerBlock; ++w) {
+        if (w == wave) before = sum;
+        sum += held[w];
+    }
+    if (threadIdx.x == 0 && sum > 0) first = atomicAdd(counter, (unsigned long long)sum);
+    __syncthreads();
+    return sum > 0 ? (uint64_t)first + before : 0u;
+}
+
+// The records that the workgroup's waves still hold at the end.
+template <class Args>   // FilterArgs or ScreenArgs: cand, counters, cand_cap
+__device__ __forceinline__ void last_records(const Args& a, const uint4* buf, uint32_t n)
+{
+    const uint64_t base = last_places(&a.counters[kCntCand], n);
+    for (uint32_t i = threadIdx.x & 63; i < n; i += 64)
+        if (base + i < a.cand_cap) a.cand[base + i] = buf[i];
 }
 
 // Record the lanes whose accumulator maximum clears the filter threshold.
@@ -781,7 +810,7 @@ __device__ __forceinline__ void filter_body(const FilterArgs& a, const WorkQueue
     for_each_item<LIST>(a.counters, a.groups, q, l, [&](uint32_t grp, uint32_t t0, uint32_t t1) __attribute__((always_inline)) {
         filter_item<BF, MASK>(a, st, grp, t0, t1, lane);
     });
-    stage_flush(a, st);
+    last_records(a, st.buf, st.n);
 }
 
 // The FP32 filter.
@@ -866,7 +895,8 @@ __device__ __forceinline__ T wave_add_by_key(T* counter, uint32_t key, bool on)
 // Hits staged per wave before one atomic reserves their range: every flush
 // is an atomic on one counter, and at ~30M hits per scan those atomics bound
 // the kernel (512: 1.37 ms, 256: 1.8 ms at 100 Mbp x 2,000 columns; 1,024
-// halves the resident waves and is slower).
+// halves the resident waves and is slower).  What is left at the end goes out
+// with one atomic per workgroup (6.7M records: 0.30 -> 0.23 ms).
 constexpr int kHitStage = 512;
 
 // Windows a filter record stands for: record window q covers q + off(r).
@@ -1070,7 +1100,9 @@ __global__ __launch_bounds__(kThreads) void finalize_kernel(FinalizeArgs a)
             }
         }
     }
-    flush();
+    const uint64_t at0 = last_places(&a.counters_rw[kCntHits], sn);
+    for (uint32_t i = lane; i < sn; i += 64)
+        if (at0 + i < a.hit_cap) hits[at0 + i] = sbuf[i];
     if constexpr (LIST) {
         if (req_in_lds) {
             __syncthreads();
