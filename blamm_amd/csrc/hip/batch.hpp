@@ -170,18 +170,17 @@ bool dma_setup(DmaReadback& d, const void* device_ptr)
     return true;
 }
 
-// Gathered fragments per column block of a batch (uint4 elements of frag_a,
-// and of frag_b in the split-BF16 form).
+// Gathered fragments per column block of a batch (uint4 elements).
 size_t batch_frag_elems(int precision)
 {
-    return prec_screen(precision) ? kScreenBlock / 2 : prec_bf(precision) ? (size_t)kMaxChunks * 64 : (size_t)kMaxLen * 16;
+    return prec_bf(precision) ? kScreenBlock / 2 : (size_t)kMaxLen * 16;
 }
 
 // Device bytes of one column block of a batch: its fragments and the
 // per-slot threshold, slot map and band tables.
 uint64_t batch_block_bytes(const blamm_hip_ctx* c)
 {
-    return (c->precision == BLAMM_PREC_BF16X2_LO ? 2 : 1) * batch_frag_elems(c->precision) * sizeof(uint4) +
+    return batch_frag_elems(c->precision) * sizeof(uint4) +
            (uint64_t)c->cols_per_blk * (4 + 4 + 8 + 8);
 }
 
@@ -225,8 +224,8 @@ struct blamm_hip_batch {
     MetaView<uint64_t> runs;        // run starts of the batch stream
     MetaView<uint2> items;          // (chunk, group), per queue
     // device-written
-    DevBuf<uint4> frag_a, frag_b;   // gathered fragments (fp32 weights in frag_a)
-    DevBuf<double> band, band_hi;   // per batch slot
+    DevBuf<uint4> frag;             // gathered fragments or FP32 weights
+    DevBuf<double> band;            // FP32 form: per batch slot
     DevBuf<double2> bound;          // per batch slot (screen)
     DevBuf<uint32_t> req_count;
     DevBuf<unsigned long long> req_off, cursor;
@@ -361,54 +360,35 @@ int batch_enqueue_kernels(blamm_hip_batch* b, bool mask, uint32_t grid)
     // the batch's column blocks from the library's fragments
     FilterArgs a{};
     ScreenArgs sa{};
-    if (prec_screen(c->precision)) {
+    if (bf) {
         ScreenGatherArgs ga;
         ga.desc = b->desc.p;
         ga.slot_map = b->slot_map.p;
         ga.lib_frag = c->screen_frag[mask ? 1 : 0].p;
         ga.lib_bound = c->screen_bound[mask ? 1 : 0].p;
-        ga.out_frag = (uint2*)b->frag_a.p;
+        ga.out_frag = (uint2*)b->frag.p;
         ga.out_bound = b->bound.p;
         hipLaunchKernelGGL(screen_gather_kernel, dim3((uint32_t)c->num_cu * 4), dim3(256), 0, b->stream, ga);
-        sa.packed = b->packed.p;
-        sa.lcmask = mask ? b->lcmask.p : nullptr;
-        sa.frag = (const uint2*)b->frag_a.p;
-        sa.thr = b->thr.p;
+        sa = screen_args(c, b->packed.p, mask ? b->lcmask.p : nullptr, b->thr.p, b->cand.p, b->cand.n, b->counters.p);
+        sa.frag = (const uint2*)b->frag.p;
         sa.bound = b->bound.p;
         sa.groups = b->groups.p;
-        sa.cand = b->cand.p;
-        sa.counters = b->counters.p;
-        sa.cand_cap = b->cand.n;
+        sa.slot_map = b->slot_map.p;
+        sa.band = c->slot_band_any.p;
     } else {
+        a = filter_args(c, b->packed.p, mask ? b->lcmask.p : nullptr, b->thr.p, b->cand.p, b->cand.n, b->counters.p);
         GatherArgs ga;
         ga.desc = b->desc.p;
         ga.slot_map = b->slot_map.p;
-        ga.lib_a = (const uint4*)c->frag_a.p;
-        ga.lib_b = (const uint4*)c->frag_b.p;
-        const bool three = !bf && !mask;
-        ga.lib_w = three ? c->frag3.p : (const float*)c->frag_a.p;
-        ga.rows = three ? kFp32Rows3 : kMaxLen;
-        ga.lib_band = three ? c->slot_off3.p : c->slot_band_any.p;
-        ga.lib_band_hi = c->slot_band_hi_any.p;
-        ga.out_a = b->frag_a.p;
-        ga.out_b = b->frag_b.p;
-        ga.out_w = (float*)b->frag_a.p;
+        ga.lib_w = a.weights;
+        ga.rows = mask ? kMaxLen : kFp32Rows3;
+        ga.lib_band = mask ? c->slot_band_any.p : c->slot_off3.p;
+        ga.out_w = (float*)b->frag.p;
         ga.out_band = b->band.p;
-        ga.out_band_hi = b->band_hi.p;
-        const dim3 gg((uint32_t)c->num_cu * 4);
-        if (bf) hipLaunchKernelGGL(gather_kernel<true>, gg, dim3(256), 0, b->stream, ga);
-        else hipLaunchKernelGGL(gather_kernel<false>, gg, dim3(256), 0, b->stream, ga);
-        a.packed = b->packed.p;
-        a.lcmask = mask ? b->lcmask.p : nullptr;
-        a.frag_a = b->frag_a.p;
-        a.frag_b = b->frag_b.p;
-        a.thr = b->thr.p;
+        hipLaunchKernelGGL(gather_kernel, dim3((uint32_t)c->num_cu * 4), dim3(256), 0, b->stream, ga);
+        a.weights = (const float*)b->frag.p;
         a.band = b->band.p;
-        a.band_hi = b->band_hi.p;
         a.groups = b->groups.p;
-        a.cand = b->cand.p;
-        a.counters = b->counters.p;
-        a.cand_cap = b->cand.n;
     }
     HIP_TRY(hipGetLastError());
     const WorkQueue q{0, 0, 1, 1};
@@ -649,8 +629,8 @@ int blamm_hip_batch_destroy(blamm_hip_batch* b)
     if (b->dma.ready || b->dma.sig.handle) (void)hsa_signal_destroy(b->dma.sig);
     drop_graphs(b);
     b->packed.release(); b->lcmask.release(); b->run_bits.release(); b->meta.release();
-    b->frag_a.release(); b->frag_b.release(); b->band.release();
-    b->band_hi.release(); b->bound.release();
+    b->frag.release(); b->band.release();
+    b->bound.release();
     b->req_count.release(); b->req_off.release(); b->cursor.release();
     b->cand.release(); b->counters.release();
     b->hits.release(); b->grouped.release();
@@ -669,8 +649,8 @@ int blamm_hip_batch_destroy(blamm_hip_batch* b)
 uint64_t blamm_hip_batch_device_bytes(const blamm_hip_batch* b)
 {
     if (!b) return 0;
-    return (b->packed.n + b->lcmask.n + b->run_bits.n) * 8 + b->meta.n + (b->frag_a.n + b->frag_b.n) * 16 +
-           (b->band.n + b->band_hi.n) * 8 + b->bound.n * sizeof(double2) + b->req_count.n * 4 + (b->req_off.n + b->cursor.n) * 8 + b->cand.n * 16 +
+    return (b->packed.n + b->lcmask.n + b->run_bits.n) * 8 + b->meta.n + b->frag.n * 16 +
+           b->band.n * 8 + b->bound.n * sizeof(double2) + b->req_count.n * 4 + (b->req_off.n + b->cursor.n) * 8 + b->cand.n * 16 +
            b->hits.n * sizeof(DevHit) + b->grouped.n * sizeof(GroupedHit) + kCntSlots * 8;
 }
 
@@ -711,7 +691,7 @@ int blamm_hip_batch_submit(blamm_hip_batch* b, const blamm_request* reqs, uint32
     const uint64_t pw = total / 32 + 16, mw = mask ? total / 64 + 16 : 0;
     const size_t nslots = (size_t)c->nslots;
     const uint32_t cpb = (uint32_t)c->cols_per_blk;
-    const bool bf = prec_bf(c->precision), screen = prec_screen(c->precision);
+    const bool screen = prec_bf(c->precision);
     const int kstep = (int)c->tuning.kpad_positions / 4;
 
     // Each request's selected columns (finite or -inf threshold), in library
@@ -816,13 +796,11 @@ int blamm_hip_batch_submit(blamm_hip_batch* b, const blamm_request* reqs, uint32
     need[kMetaItems] = std::max<size_t>(nitems, 1);
     BLAMM_TRY(meta_fit(b, need));
     const size_t fr = (size_t)std::max<uint32_t>(nblk, 1) * batch_frag_elems(c->precision);
-    BLAMM_TRY(batch_grow(b, b->frag_a, fr));
+    BLAMM_TRY(batch_grow(b, b->frag, fr));
     if (screen) {
         BLAMM_TRY(batch_grow(b, b->bound, nbs));
     } else {
         BLAMM_TRY(batch_grow(b, b->band, nbs));
-        BLAMM_TRY(batch_grow(b, b->band_hi, nbs));
-        BLAMM_TRY(batch_grow(b, b->frag_b, bf ? fr : 1));
     }
     BLAMM_TRY(batch_grow(b, b->req_count, nreq));
     BLAMM_TRY(batch_grow(b, b->req_off, (size_t)nreq + 1));

@@ -188,7 +188,6 @@ struct blamm_hip_ctx {
     DevBuf<double> slot_off3;                  // and what its threshold is lowered by
     DevBuf<float> slot_thr, slot_w, slot_w2;   // w2: FP32 sums of position pairs
     DevBuf<double> slot_band, slot_band_any, slot_seq;   // band_any: valid in a block of any length
-    DevBuf<double> slot_band_hi, slot_band_hi_any;      // hi-only stage of the bf16 filter
     DevBuf<int> slot_len;
     DevBuf<uint32_t> slot_col, scan_groups_d;
     // screen layout (default form): fragments and bounds for streams without
@@ -225,17 +224,16 @@ struct blamm_hip_ctx {
 
 namespace {
 
-// Precision modes: FP32, split bf16 with the lo products on the matrix cores,
-// or (default) split bf16 behind the screen.  Both bf16 modes keep the hi and
-// lo terms on the device (histograms use them).
+// Precision modes: FP32, or one of the two behind the screen (the split-BF16
+// form also scores what passes it with hi and lo products).  Both of these keep
+// the bf16 hi and lo terms on the device (histograms use them).
 inline bool prec_bf(int p) { return p == BLAMM_PREC_BF16X2 || p == BLAMM_PREC_BF16X2_LO; }
-inline bool prec_screen(int p) { return p == BLAMM_PREC_BF16X2; }
 
 template <bool MASK, bool LIST>
 const void* filter_kernel_ptr(int precision)
 {
-    return precision == BLAMM_PREC_BF16X2      ? (const void*)screen_kernel<MASK, LIST>
-           : precision == BLAMM_PREC_BF16X2_LO ? (const void*)filter_lo_kernel<MASK, LIST>
+    return precision == BLAMM_PREC_BF16X2      ? (const void*)screen_kernel<MASK, LIST, false>
+           : precision == BLAMM_PREC_BF16X2_LO ? (const void*)screen_kernel<MASK, LIST, true>
                                                : (const void*)filter_fp32_kernel<MASK, LIST>;
 }
 
@@ -272,7 +270,7 @@ hipError_t launch_filter(int precision, bool mask, bool list, const ScreenArgs& 
     ListArgs la = l;
     ScreenArgs sa = a;
     FilterArgs fa = f;
-    void* args[] = {prec_screen(precision) ? (void*)&sa : (void*)&fa, &qa, &la};
+    void* args[] = {prec_bf(precision) ? (void*)&sa : (void*)&fa, &qa, &la};
     return hipLaunchKernel(filter_kernel(precision, mask, list), dim3(grid), dim3(kThreads), args, 0, s);
 }
 
@@ -390,7 +388,7 @@ int relayout(blamm_hip_ctx* c)
     const int nslots = nblk * cols_per_blk;
     // The scan's groups: those of the screen in the default form.
     std::vector<GroupInfo> scan_groups = groups;
-    if (prec_screen(c->precision)) {
+    if (prec_bf(c->precision)) {
         std::vector<int> blk_len(nblk, 1);
         for (int i = 0; i < nblk; ++i)
             for (int col : blocks[i])
@@ -403,7 +401,6 @@ int relayout(blamm_hip_ctx* c)
     std::vector<int> s_len(nslots, 1), s_colh(nslots, -1);
     std::vector<uint32_t> s_col(nslots, 0);
     std::vector<double> s_band(nslots, 0.0), s_band_any(nslots, 0.0), s_seq(nslots, 0.0);
-    std::vector<double> s_band_hi(nslots, 0.0), s_band_hi_any(nslots, 0.0);
     std::vector<double> s_off3(bf ? 0 : nslots, 0.0);
     std::vector<uint16_t> hi16((size_t)nslots * kMaxLen * 4, 0), lo16((size_t)nslots * kMaxLen * 4, 0);
     double max_band = 0.0, max_err = 0.0;
@@ -416,7 +413,7 @@ int relayout(blamm_hip_ctx* c)
             const int slot = bi * cols_per_blk + k;
             const int L = lengths[col];
             const float* w = P + (size_t)col * ldp;
-            double sum_max = 0.0, sum_split = 0.0, rep_err = 0.0, sum_lo = 0.0;
+            double sum_max = 0.0, sum_split = 0.0, rep_err = 0.0;
             double off3 = 0.0, sum3 = 0.0, rep3 = 0.0;
             for (int p = 0; p < L; ++p) {
                 if (!bf) {
@@ -431,7 +428,7 @@ int relayout(blamm_hip_ctx* c)
                     sum3 += m3;
                     rep3 += e3;
                 }
-                double mx = 0.0, mxs = 0.0, me = 0.0, ml = 0.0;
+                double mx = 0.0, mxs = 0.0, me = 0.0;
                 for (int b = 0; b < 4; ++b) {
                     const float x = w[4 * p + b];
                     s_w[((size_t)slot * kMaxLen + p) * 4 + b] = x;
@@ -445,7 +442,6 @@ int relayout(blamm_hip_ctx* c)
                         lo16[((size_t)slot * kMaxLen + p) * 4 + b] = l;
                         me = std::max(me, std::fabs((double)x - (double)hf - (double)lf));
                         mxs = std::max(mxs, std::fabs((double)hf) + std::fabs((double)lf));
-                        ml = std::max(ml, std::fabs((double)lf));
                     } else {
                         mxs = std::max(mxs, (double)std::fabs(x));
                     }
@@ -453,7 +449,6 @@ int relayout(blamm_hip_ctx* c)
                 sum_max += mx;
                 sum_split += mxs;
                 rep_err += me;
-                sum_lo += ml;
             }
             // |FP64 left-to-right sum - exact sum| (binary64, L-1 additions)
             const double fp64_err = gamma_n(L, u53) * sum_max;
@@ -478,12 +473,6 @@ int relayout(blamm_hip_ctx* c)
             const double nterms_any = bf ? 32.0 * max_nch : 16.0 * max_nch;
             s_band_any[slot] =
                 2.0 * (rep_err + gamma_n(nterms_any, std::ldexp(1.0, -22)) * sum_split + fp64_err) + 1e-30;
-            // hi-only score H': the lo terms it leaves out are bounded by
-            // sum_p max_b |lo|; rounding as for the full sum
-            s_band_hi[slot] =
-                2.0 * (sum_lo + rep_err + gamma_n(nterms, std::ldexp(1.0, -22)) * sum_split + fp64_err) + 1e-30;
-            s_band_hi_any[slot] =
-                2.0 * (sum_lo + rep_err + gamma_n(nterms_any, std::ldexp(1.0, -22)) * sum_split + fp64_err) + 1e-30;
             // Sequential FP32 band used by finalize (RNE adds, L-1 of them).
             const double seq = 2.0 * (gamma_n(L, u24) * sum_max + fp64_err) + 1e-30;
             s_thr[slot] = c->lib_thr[col];
@@ -562,8 +551,6 @@ int relayout(blamm_hip_ctx* c)
     HIP_TRY(c->slot_thr.reserve(nslots));
     HIP_TRY(c->slot_band.reserve(nslots));
     HIP_TRY(c->slot_band_any.reserve(nslots));
-    HIP_TRY(c->slot_band_hi.reserve(nslots));
-    HIP_TRY(c->slot_band_hi_any.reserve(nslots));
     HIP_TRY(c->slot_seq.reserve(nslots));
     HIP_TRY(c->slot_w.reserve(s_w.size()));
     // finalize's pair table: entry b1 + 4 b2 of pair q is w[2q][b1] + w[2q+1][b2]
@@ -585,15 +572,12 @@ int relayout(blamm_hip_ctx* c)
     HIP_TRY(hipMemcpy(c->slot_thr.p, s_thr.data(), nslots * sizeof(float), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(c->slot_band.p, s_band.data(), nslots * sizeof(double), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(c->slot_band_any.p, s_band_any.data(), nslots * sizeof(double), hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(c->slot_band_hi.p, s_band_hi.data(), nslots * sizeof(double), hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(c->slot_band_hi_any.p, s_band_hi_any.data(), nslots * sizeof(double),
-                      hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(c->slot_seq.p, s_seq.data(), nslots * sizeof(double), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(c->slot_w.p, s_w.data(), s_w.size() * sizeof(float), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(c->slot_len.p, s_len.data(), nslots * sizeof(int), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(c->slot_col.p, s_col.data(), nslots * sizeof(uint32_t), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(c->scan_groups_d.p, gpk.data(), gpk.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
-    if (prec_screen(c->precision)) {
+    if (prec_bf(c->precision)) {
         ScreenLayoutArgs a;
         a.slot_w = c->slot_w.p;
         a.slot_len = c->slot_len.p;
@@ -630,11 +614,9 @@ FilterArgs filter_args(const blamm_hip_ctx* c, const uint64_t* packed, const uin
     a.packed = packed;
     a.lcmask = lcmask;
     const bool three = c->precision == BLAMM_PREC_FP32 && !lcmask;
-    a.frag_a = three ? (const void*)c->frag3.p : (const void*)c->frag_a.p;
-    a.frag_b = c->frag_b.p;
+    a.weights = three ? c->frag3.p : (const float*)c->frag_a.p;
     a.thr = thr;
     a.band = three ? c->slot_off3.p : c->slot_band.p;
-    a.band_hi = c->slot_band_hi.p;
     a.groups = c->scan_groups_d.p;
     a.cand = cand;
     a.counters = counters;
@@ -656,6 +638,11 @@ ScreenArgs screen_args(const blamm_hip_ctx* c, const uint64_t* packed, const uin
     a.cand = cand;
     a.counters = counters;
     a.cand_cap = cand_cap;
+    a.hi = (const uint4*)c->frag_a.p;
+    a.lo = (const uint4*)c->frag_b.p;
+    a.band = c->slot_band.p;
+    a.len = c->slot_len.p;
+    a.slot_map = nullptr;
     return a;
 }
 
@@ -755,7 +742,7 @@ int blamm_hip_destroy(blamm_hip_ctx* c)
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     c->frag_a.release(); c->frag_b.release(); c->frag3.release(); c->slot_off3.release(); c->slot_thr.release(); c->slot_band.release();
-    c->slot_band_any.release(); c->slot_band_hi.release(); c->slot_band_hi_any.release();
+    c->slot_band_any.release();
     c->slot_seq.release(); c->slot_w.release(); c->slot_w2.release();
     c->slot_len.release(); c->slot_col.release(); c->scan_groups_d.release(); c->cand.release();
     for (int m = 0; m < 2; ++m) {

@@ -266,7 +266,7 @@ __device__ __forceinline__ uint32_t hist_range(const HistArgs& a, Stage& st, uin
         }
         // every window of the tile fits its run for every length <= 4 NCH
         const bool fast = q0 + (kBf16Tile - 1) + 4 * NCH <= rnext && q0 + kBf16Tile <= a.qend;
-        const f32x16& av = acc_read<AccRead::kGuard>(acc[0]);
+        const f32x16& av = acc_read(acc[0]);
         const uint32_t qlane = q0 + 4 * (lane >> 5);
         const uint32_t defer = fast ? hist_rows<true, LDS, CLAMP>(a, hl, av, hv, qlane, jr, rnext)
                                     : hist_rows<false, LDS, CLAMP>(a, hl, av, hv, qlane, jr, rnext);
@@ -301,7 +301,7 @@ __global__ __launch_bounds__(kThreads, WIDE ? 2 : 4) void hist_filter_kernel(His
     __shared__ uint4 stage_lds[kWavesPerBlock][kHistStage];
     __shared__ uint32_t item_s;
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    Stage st{stage_lds[wave], 0u, nullptr};
+    Stage st{stage_lds[wave], 0u};
     uint32_t exact = 0;
     for (;;) {
         if (threadIdx.x == 0) item_s = (uint32_t)atomicAdd(&a.counters[kCntQueue + a.queue], 1ull);

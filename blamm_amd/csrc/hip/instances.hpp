@@ -1,6 +1,6 @@
 // The filter and histogram kernels are compiled in translation units of their
-// own (screen.hip, filter_bf16.hip, filter_fp32.hip, hist_filter.hip) so that the library
-// builds in parallel; the launching code sees these declarations and leaves
+// own (screen.hip, filter_fp32.hip, hist_filter.hip) so that the library builds
+// in parallel; the launching code sees these declarations and leaves
 // the instantiation to those units.
 #pragma once
 
@@ -17,9 +17,9 @@ namespace blamm {
     X(false, false, true) X(false, true, true) X(true, false, true) X(true, true, true)
 
 #ifndef BLAMM_INSTANTIATE
-#define BLAMM_EXTERN_SCREEN(M, L) extern template __global__ void screen_kernel<M, L>(ScreenArgs, WorkQueue, ListArgs);
+#define BLAMM_EXTERN_SCREEN(M, L) extern template __global__ void screen_kernel<M, L, false>(ScreenArgs, WorkQueue, ListArgs);
 #define BLAMM_EXTERN_FP32(M, L) extern template __global__ void filter_fp32_kernel<M, L>(FilterArgs, WorkQueue, ListArgs);
-#define BLAMM_EXTERN_LO(M, L) extern template __global__ void filter_lo_kernel<M, L>(FilterArgs, WorkQueue, ListArgs);
+#define BLAMM_EXTERN_LO(M, L) extern template __global__ void screen_kernel<M, L, true>(ScreenArgs, WorkQueue, ListArgs);
 #define BLAMM_EXTERN_HIST(M, L, W) extern template __global__ void hist_filter_kernel<M, L, W>(HistArgs);
 BLAMM_SCAN_INSTANCES(BLAMM_EXTERN_SCREEN)
 BLAMM_SCAN_INSTANCES(BLAMM_EXTERN_FP32)

@@ -30,7 +30,6 @@ constexpr int kThreads = kWaveSize * kWavesPerBlock;
 constexpr int kMaxLen = 64;          // positions per column slot
 constexpr int kMaxChunks = kMaxLen / 4;
 constexpr int kWideChunks = 8;       // above this many chunks a wave holds one column block
-constexpr int kLoChunks = 16;        // split-BF16 filter: chunk fragments per wave in LDS (NB x NCH)
 constexpr int kBf16Cols = 32;        // columns per bf16 column block (MFMA N)
 constexpr int kBf16Tile = 32;        // windows per bf16 tile (MFMA M)
 constexpr int kFp32Cols = 16;        // columns per fp32 column block
@@ -74,11 +73,9 @@ __device__ __forceinline__ uint64_t wave_reserve(unsigned long long* counter, ui
 struct FilterArgs {
     const uint64_t* packed;      // 2-bit codes
     const uint64_t* lcmask;      // lowercase bits (MASK variants only)
-    const void* frag_a;          // bf16: hi fragments; fp32: weights
-    const void* frag_b;          // bf16: lo fragments
+    const float* weights;
     const float* thr;            // per slot: threshold
     const double* band;          // per slot: filter band (MFMA score vs FP64 score)
-    const double* band_hi;       // per slot: band of the hi-only score (split-BF16 filter)
     const uint32_t* groups;      // column groups, see group_pack()
     uint4* cand;                 // (first window of a lane, slot, rows above the threshold, 0)
     unsigned long long* counters;
@@ -126,14 +123,12 @@ __host__ __device__ constexpr uint32_t group_pack(uint32_t blk0, uint32_t nch, u
 // candidates per scan), so each wave collects up to kStage candidates in its
 // own LDS slice and reserves global space with one atomic per flush.  Only
 // the owning wave touches its slice; LDS operations of one wave complete in
-// program order, so no barrier is needed.  252 entries: with the split-BF16
-// filter's fragments and last_places' words just under 80 KiB per block.
-constexpr int kStage = 252;
+// program order, so no barrier is needed.
+constexpr int kStage = 256;
 
 struct Stage {
     uint4* buf;        // this wave's LDS slice
     uint32_t n;        // staged entries (wave-uniform)
-    uint4* lo;         // split-BF16 filter: this wave's lo fragments (LDS), [block][chunk][lane]
 };
 
 __device__ __forceinline__ void stage_flush(const FilterArgs& a, Stage& st)
@@ -221,17 +216,11 @@ __device__ __forceinline__ void mfma_result_guard()
     __builtin_amdgcn_sched_barrier(0);
 }
 
-// Every VALU read of an MFMA accumulator goes through acc_read: kGuard places
-// the guard's wait states first; kCovered states, at the call, that the
-// MFMAs of a whole further tile were issued after the last MFMA that wrote
-// the accumulator (the software-pipelined loops), which covers the result
-// latency many times over.
-enum class AccRead { kGuard, kCovered };
-
-template <AccRead R, typename V>
+// Every VALU read of an MFMA accumulator goes through acc_read.
+template <typename V>
 __device__ __forceinline__ const V& acc_read(const V& acc)
 {
-    if constexpr (R == AccRead::kGuard) mfma_result_guard();
+    mfma_result_guard();
     return acc;
 }
 
@@ -242,20 +231,15 @@ __device__ __forceinline__ uint32_t funnel32(uint32_t lo, uint32_t hi, uint32_t 
 
 // Tiles are 32 consecutive windows; a wave walks tiles [t0, t1) of its range.
 
-// The split-BF16 filter (BLAMM_PREC_BF16X2_LO) is software-pipelined over two
-// accumulator sets: a tile block whose hi-only score can reach the threshold
-// gets its lo products (lo fragments kept in a per-wave LDS slice) and records
-// its windows at or above thr - band.
-
 // ---------------------------------------------------------------------------
-// Split-BF16 filter: W = hi + lo (bf16 each); one-hot operand is exact in bf16.
+// Split-BF16 products: W = hi + lo (bf16 each); one-hot operand is exact in bf16.
 // MFMA v_mfma_f32_32x32x16_bf16: A = one-hot (32 windows x 16 = 4 positions x
 // 4 bases), B = PWM chunk (16 x 32 columns), D = 32x32 FP32 scores.
 // Lane l: A rows/ B cols index l%32, K half h = l/32 holds positions 2h, 2h+1
 // of the chunk; D lane l holds column l%32, rows 8(r/4) + 4h + r%4.
-// Each wave keeps the hi terms of NB column blocks (NCH chunks) in registers
-// and streams window tiles through them (the filter keeps the lo terms in its
-// LDS slice, the histogram kernel both in registers).
+// The histogram kernel keeps both terms of NB column blocks (NCH chunks) in
+// registers and streams window tiles through them; the split-BF16 form of the
+// scan scores the tile blocks that its screen cannot rule out.
 // ---------------------------------------------------------------------------
 // The one-hot operand of chunk j for the lane's window: bf16 1.0 (0x3F80) in
 // lane b of four per base, built in registers (no memory latency; the VALU
@@ -347,148 +331,12 @@ __device__ __forceinline__ void bf16_mfma_tile(f32x16 (&acc)[NB], const bf16x8 (
     }
 }
 
-// ---------------------------------------------------------------------------
-// Lazy lo.  The hi products alone give a score H'; a window's FP64 score can
-// reach thr only if H' >= thr - band_hi, where band_hi bounds the lo terms,
-// the split's representation error and every rounding (proved per column on
-// the host).  So a tile block whose hi-only maximum stays below that bound in
-// every lane cannot hold a candidate and its lo products are skipped; blocks
-// that pass get their lo products and the exact-band test.
-// ---------------------------------------------------------------------------
-template <int NCH, int NB, bool MASK>
-__device__ __forceinline__ void bf16_hi_tile(f32x16 (&acc)[NB], const bf16x8 (&bh)[NB][NCH],
-                                             const OneHotSrc& bits, uint64_t mb)
-{
-#pragma unroll
-    for (int b = 0; b < NB; ++b) acc[b] = (f32x16){0.f};
-#pragma unroll
-    for (int j = 0; j < NCH; ++j) {
-        const bf16x8 A = onehot_chunk<MASK>(bits, mb, j);
-#pragma unroll
-        for (int b = 0; b < NB; ++b) acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A, bh[b][j], acc[b], 0, 0, 0);
-    }
-}
-
-template <int NB>
 __device__ __forceinline__ float tile_max(const f32x16& v)
 {
     float mx = v[0];
 #pragma unroll
     for (int r = 1; r < 16; ++r) mx = fmaxf(mx, v[r]);
     return mx;
-}
-
-// Finish a tile whose hi products are in acc (R: how the first read is kept
-// clear of the matrix cores).  The lo fragments come from the wave's LDS
-// slice.
-template <int NCH, int NB, bool MASK, AccRead R>
-__device__ __forceinline__ void bf16_finish_tile(const FilterArgs& a, Stage& st, f32x16 (&acc)[NB],
-                                                 const float (&th)[NB], const float (&thh)[NB], const OneHotSrc& bits,
-                                                 uint64_t mb, uint32_t q0, uint32_t blk0, uint32_t lane)
-{
-    uint32_t need = 0;
-    const f32x16 (&hv)[NB] = acc_read<R>(acc);
-#pragma unroll
-    for (int b = 0; b < NB; ++b)
-        if (__ballot(tile_max<NB>(hv[b]) >= thh[b])) need |= 1u << b;
-    if (need == 0) return;
-    const uint32_t qlane = q0 + 4 * (lane >> 5);
-    // one uniform branch per block around its whole chunk loop (a branch
-    // per MFMA would copy the accumulator at every join)
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-        if (!(need & (1u << b))) continue;
-        bf16x8 B[NCH];
-#pragma unroll
-        for (int j = 0; j < NCH; ++j) B[j] = __builtin_bit_cast(bf16x8, st.lo[(b * NCH + j) * 64 + lane]);
-#pragma unroll
-        for (int j = 0; j < NCH; ++j)
-            acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(onehot_chunk<MASK>(bits, mb, j), B[j], acc[b], 0, 0, 0);
-    }
-    const f32x16 (&fv)[NB] = acc_read<AccRead::kGuard>(acc);
-#pragma unroll
-    for (int b = 0; b < NB; ++b)
-        if (need & (1u << b)) {
-            float v[16];
-#pragma unroll
-            for (int r = 0; r < 16; ++r) v[r] = fv[b][r];
-            emit_rows<16>(a, st, v, th[b], qlane, (blk0 + b) * kBf16Cols + (lane & 31));
-        }
-}
-
-// Tiles [t0, t1) of column blocks blk0 .. blk0+NB-1.  Lane-private bases
-// of tile t come from packed words t and t+1 of the lane's pointer (a sliding
-// pair).  Software-pipelined: the hi products of tile t are issued before
-// tile t-1 is finished.
-template <int NCH, int NB, bool MASK>
-__device__ __forceinline__ void bf16_range(const FilterArgs& a, Stage& st, uint32_t blk0, uint32_t t0, uint32_t t1,
-                                           uint32_t lane)
-{
-    static_assert(NB * NCH <= kLoChunks, "lo fragments exceed the wave's LDS slice");
-    static_assert(NCH <= kWideChunks || NB == 1, "wide blocks are scored one per wave");
-    const uint4* __restrict__ fh = (const uint4*)a.frag_a;
-    const uint4* __restrict__ fl = (const uint4*)a.frag_b;
-    bf16x8 bh[NB][NCH];
-    float th[NB], thh[NB];
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-#pragma unroll
-        for (int j = 0; j < NCH; ++j) {
-            const size_t idx = ((size_t)(blk0 + b) * kMaxChunks + j) * 64 + lane;
-            bh[b][j] = __builtin_bit_cast(bf16x8, fh[idx]);
-            st.lo[(b * NCH + j) * 64 + lane] = fl[idx];   // each lane reads back only its own
-        }
-        const uint32_t slot = (blk0 + b) * kBf16Cols + (lane & 31);
-        th[b] = thr_minus(a.thr[slot], a.band[slot]);
-        thh[b] = thr_minus(a.thr[slot], a.band_hi[slot]);
-    }
-
-    const uint32_t off = (lane & 31) + 2 * (lane >> 5);   // first base of the lane's window, 0..33
-    // pk[t]: dwords 2t + off/16 and the next of the packed stream, so the
-    // window of tile t starts at bit sh < 32 of pk[t] and continues through
-    // pk[t + 1] (and pk[t + 2] for motifs longer than 48 positions)
-    const uint32_t sh = 2 * (off & 15);
-    const u64_a4* __restrict__ pk = (const u64_a4*)((const uint32_t*)a.packed + (off >> 4));
-    const uint32_t* __restrict__ mk = (const uint32_t*)a.lcmask + (off >> 5);
-    f32x16 accA[NB], accB[NB];
-    OneHotSrc bA, bB{};
-    uint64_t mA = 0, mB = 0;
-    uint32_t m0 = 0, m1 = 0, m2 = 0;
-    bA = onehot_src<NCH>(pk[t0], pk[t0 + 1], pk[t0 + 2], sh);
-    if (MASK) mA = window_mask<NCH>(mk[t0], mk[t0 + 1], mk[t0 + 2], off & 31);
-    bf16_hi_tile<NCH, NB, MASK>(accA, bh, bA, mA);
-    uint64_t w0 = pk[t0 + 1], w1 = pk[t0 + 2], w2 = pk[t0 + 3];
-    if (MASK) { m0 = mk[t0 + 1]; m1 = mk[t0 + 2]; m2 = mk[t0 + 3]; }
-    uint32_t t = t0 + 1;
-    bool pendingA = true;           // accA holds tile t-1, not yet finished
-    for (; t + 1 < t1; t += 2) {
-        const uint64_t w3 = pk[t + 3], w4 = pk[t + 4];
-        uint32_t m3 = 0, m4 = 0;
-        if (MASK) { m3 = mk[t + 3]; m4 = mk[t + 4]; }
-        bB = onehot_src<NCH>(w0, w1, w2, sh);
-        if (MASK) mB = window_mask<NCH>(m0, m1, m2, off & 31);
-        bf16_hi_tile<NCH, NB, MASK>(accB, bh, bB, mB);
-        bf16_finish_tile<NCH, NB, MASK, AccRead::kCovered>(a, st, accA, th, thh, bA, mA, (t - 1) * kBf16Tile, blk0,
-                                                              lane);
-        bA = onehot_src<NCH>(w1, w2, w3, sh);
-        if (MASK) mA = window_mask<NCH>(m1, m2, m3, off & 31);
-        bf16_hi_tile<NCH, NB, MASK>(accA, bh, bA, mA);
-        bf16_finish_tile<NCH, NB, MASK, AccRead::kCovered>(a, st, accB, th, thh, bB, mB, t * kBf16Tile, blk0, lane);
-        w0 = w2; w1 = w3; w2 = w4;
-        if (MASK) { m0 = m2; m1 = m3; m2 = m4; }
-    }
-    if (t < t1) {                   // one tile left: t
-        bB = onehot_src<NCH>(w0, w1, w2, sh);
-        if (MASK) mB = window_mask<NCH>(m0, m1, m2, off & 31);
-        bf16_hi_tile<NCH, NB, MASK>(accB, bh, bB, mB);
-        bf16_finish_tile<NCH, NB, MASK, AccRead::kCovered>(a, st, accA, th, thh, bA, mA, (t - 1) * kBf16Tile, blk0,
-                                                              lane);
-        pendingA = false;
-        bf16_finish_tile<NCH, NB, MASK, AccRead::kGuard>(a, st, accB, th, thh, bB, mB, t * kBf16Tile, blk0, lane);
-    }
-    if (pendingA)
-        bf16_finish_tile<NCH, NB, MASK, AccRead::kGuard>(a, st, accA, th, thh, bA, mA, (t - 1) * kBf16Tile, blk0,
-                                                            lane);
 }
 
 // ---------------------------------------------------------------------------
@@ -572,7 +420,7 @@ __device__ __forceinline__ void fp32_range(const FilterArgs& a, Stage& st, uint3
     static_assert(NB <= fp32_blocks(NCH, 4), "weights exceed the registers");
     using Rows = Fp32Rows<NCH, MASK>;
     constexpr int NJ = Rows::NJ, NH = Rows::NH, R = MASK ? kMaxLen : kFp32Rows3;
-    const float* __restrict__ fw = (const float*)a.frag_a;
+    const float* __restrict__ fw = a.weights;
     float bw[NB][NJ * NCH];
     float th[NB];
 #pragma unroll
@@ -630,7 +478,7 @@ __device__ __forceinline__ void fp32_range(const FilterArgs& a, Stage& st, uint3
                         acc[u][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, bw[b][NJ * c + j], acc[u][b], 0, 0, 0);
                 }
         }
-        const f32x4 (&av)[2][NB] = acc_read<AccRead::kGuard>(acc);
+        const f32x4 (&av)[2][NB] = acc_read(acc);
 #pragma unroll
         for (int u = 0; u < 2; ++u)
 #pragma unroll
@@ -700,38 +548,24 @@ struct ListArgs {
     const uint4* chunks;    // (t0, t1, request, 0)
 };
 
-// One item: tiles [t0, t1) against one column group.
-template <bool BF, bool MASK>
-__device__ __forceinline__ void filter_item(const FilterArgs& a, Stage& st, uint32_t grp,
-                                            uint32_t t0, uint32_t t1, uint32_t lane)
+// One item of the FP32 filter: tiles [t0, t1) against one column group.
+template <bool MASK>
+__device__ __forceinline__ void fp32_item(const FilterArgs& a, Stage& st, uint32_t grp, uint32_t t0, uint32_t t1,
+                                          uint32_t lane)
 {
     const uint32_t blk0 = grp & 0xFFFFFu, nch = (grp >> 20) & 63u, nb = grp >> 26;
-    if constexpr (BF) {
-        switch (nch * 8 + nb) {
-#define BLAMM_BF(N, B) case N * 8 + B: bf16_range<N, B, MASK>(a, st, blk0, t0, t1, lane); break;
-        BLAMM_BF(1, 1) BLAMM_BF(2, 1) BLAMM_BF(3, 1) BLAMM_BF(4, 1)
-        BLAMM_BF(5, 1) BLAMM_BF(6, 1) BLAMM_BF(7, 1) BLAMM_BF(8, 1)
-        BLAMM_BF(1, 2) BLAMM_BF(2, 2) BLAMM_BF(3, 2) BLAMM_BF(4, 2)
-        BLAMM_BF(5, 2) BLAMM_BF(6, 2) BLAMM_BF(7, 2) BLAMM_BF(8, 2)
-        BLAMM_BF(9, 1) BLAMM_BF(10, 1) BLAMM_BF(11, 1) BLAMM_BF(12, 1)
-        BLAMM_BF(13, 1) BLAMM_BF(14, 1) BLAMM_BF(15, 1) BLAMM_BF(16, 1)
-#undef BLAMM_BF
-        default: break;
-        }
-    } else {
-        switch (nch * 8 + nb) {
+    switch (nch * 8 + nb) {
 #define BLAMM_F32(N, B) case N * 8 + B: fp32_range<N, B, MASK>(a, st, blk0, t0, t1, lane); break;
-        BLAMM_F32(1, 1) BLAMM_F32(2, 1) BLAMM_F32(3, 1) BLAMM_F32(4, 1)
-        BLAMM_F32(5, 1) BLAMM_F32(6, 1) BLAMM_F32(7, 1) BLAMM_F32(8, 1)
-        BLAMM_F32(1, 2) BLAMM_F32(2, 2) BLAMM_F32(3, 2) BLAMM_F32(4, 2)
-        BLAMM_F32(5, 2) BLAMM_F32(6, 2) BLAMM_F32(7, 2) BLAMM_F32(8, 2)
-        BLAMM_F32(1, 4) BLAMM_F32(2, 4) BLAMM_F32(3, 4) BLAMM_F32(4, 4)
-        BLAMM_F32(5, 4) BLAMM_F32(6, 4)
-        BLAMM_F32(9, 1) BLAMM_F32(10, 1) BLAMM_F32(11, 1) BLAMM_F32(12, 1)
-        BLAMM_F32(13, 1) BLAMM_F32(14, 1) BLAMM_F32(15, 1) BLAMM_F32(16, 1)
+    BLAMM_F32(1, 1) BLAMM_F32(2, 1) BLAMM_F32(3, 1) BLAMM_F32(4, 1)
+    BLAMM_F32(5, 1) BLAMM_F32(6, 1) BLAMM_F32(7, 1) BLAMM_F32(8, 1)
+    BLAMM_F32(1, 2) BLAMM_F32(2, 2) BLAMM_F32(3, 2) BLAMM_F32(4, 2)
+    BLAMM_F32(5, 2) BLAMM_F32(6, 2) BLAMM_F32(7, 2) BLAMM_F32(8, 2)
+    BLAMM_F32(1, 4) BLAMM_F32(2, 4) BLAMM_F32(3, 4) BLAMM_F32(4, 4)
+    BLAMM_F32(5, 4) BLAMM_F32(6, 4)
+    BLAMM_F32(9, 1) BLAMM_F32(10, 1) BLAMM_F32(11, 1) BLAMM_F32(12, 1)
+    BLAMM_F32(13, 1) BLAMM_F32(14, 1) BLAMM_F32(15, 1) BLAMM_F32(16, 1)
 #undef BLAMM_F32
-        default: break;
-        }
+    default: break;
     }
 }
 
@@ -799,33 +633,17 @@ __device__ __forceinline__ void for_each_item(unsigned long long* counters, cons
 }
 static_assert(kQueues == 64, "one lane looks at one queue");
 
-template <bool BF, bool MASK, bool LIST>
-__device__ __forceinline__ void filter_body(const FilterArgs& a, const WorkQueue& q, const ListArgs& l)
-{
-    const uint32_t lane = threadIdx.x & 63;
-    __shared__ uint4 stage_lds[kWavesPerBlock][kStage];
-    // bf16: per-wave lo fragments (kLoChunks chunk fragments x 64 lanes)
-    __shared__ uint4 lo_lds[BF ? kWavesPerBlock * kLoChunks * 64 : 1];
-    Stage st{stage_lds[threadIdx.x >> 6], 0u, BF ? lo_lds + (threadIdx.x >> 6) * kLoChunks * 64 : lo_lds};
-    for_each_item<LIST>(a.counters, a.groups, q, l, [&](uint32_t grp, uint32_t t0, uint32_t t1) __attribute__((always_inline)) {
-        filter_item<BF, MASK>(a, st, grp, t0, t1, lane);
-    });
-    last_records(a, st.buf, st.n);
-}
-
 // The FP32 filter.
 template <bool MASK, bool LIST>
 __global__ __launch_bounds__(kThreads, MASK ? 2 : 3) void filter_fp32_kernel(FilterArgs a, WorkQueue q, ListArgs l)
 {
-    filter_body<false, MASK, LIST>(a, q, l);
-}
-
-// The split-BF16 filter (80 KiB of LDS per block: two blocks per CU, so two
-// waves per SIMD and at most 256 registers).
-template <bool MASK, bool LIST>
-__global__ __launch_bounds__(kThreads, 2) void filter_lo_kernel(FilterArgs a, WorkQueue q, ListArgs l)
-{
-    filter_body<true, MASK, LIST>(a, q, l);
+    const uint32_t lane = threadIdx.x & 63;
+    __shared__ uint4 stage_lds[kWavesPerBlock][kStage];
+    Stage st{stage_lds[threadIdx.x >> 6], 0u};
+    for_each_item<LIST>(a.counters, a.groups, q, l, [&](uint32_t grp, uint32_t t0, uint32_t t1) __attribute__((always_inline)) {
+        fp32_item<MASK>(a, st, grp, t0, t1, lane);
+    });
+    last_records(a, st.buf, st.n);
 }
 
 struct FinalizeArgs {
@@ -1272,63 +1090,41 @@ static __global__ __launch_bounds__(kGroupThreads) void group_scatter_kernel(Gro
 }
 #endif  // BLAMM_INSTANTIATE
 
-// Column blocks of a batch: batch slot s takes the fragments of library slot
-// slot_map[s] (an empty slot gets zero weights).  Bands are the library's
-// bands for the longest block (valid for a column in any block).
+// Column blocks of a batch in the FP32 form: batch slot s takes the weights
+// and the band of library slot slot_map[s] (an empty slot gets zeros).  Bands
+// are the library's bands for the longest block (valid for a column in any
+// block).
 struct GatherArgs {
     const BatchDesc* desc;                // nblk
     const uint32_t* slot_map;
-    const uint4* lib_a;                   // bf16: [block][chunk][lane] hi / fp32: weights as uint4 view unused
-    const uint4* lib_b;
-    const float* lib_w;                   // fp32: [block][row][lane]
-    uint32_t rows;                        // fp32: rows of a block
+    const float* lib_w;                   // [block][row][lane]
+    uint32_t rows;                        // of a block
     const double* lib_band;               // per library slot, any block
-    const double* lib_band_hi;            // per library slot, any block (hi-only stage)
-    uint4* out_a;
-    uint4* out_b;
     float* out_w;
     double* out_band;
-    double* out_band_hi;
 };
 
-template <bool BF>
-__global__ __launch_bounds__(256) void gather_kernel(GatherArgs g)
+#ifndef BLAMM_INSTANTIATE
+static __global__ __launch_bounds__(256) void gather_kernel(GatherArgs g)
 {
     const uint32_t nblk = g.desc->nblk;
     const uint64_t stride = (uint64_t)gridDim.x * 256;
     const uint64_t t0 = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-    constexpr uint32_t cpb = BF ? kBf16Cols : kFp32Cols;
-    if constexpr (BF) {
-        const uint64_t total = (uint64_t)nblk * kMaxChunks * 64;
-        for (uint64_t i = t0; i < total; i += stride) {
-            const uint32_t l = (uint32_t)(i & 63), j = (uint32_t)((i >> 6) % kMaxChunks);
-            const uint32_t b = (uint32_t)(i / (64 * kMaxChunks));
-            const uint32_t lib = g.slot_map[b * cpb + (l & 31)];
-            uint4 va = make_uint4(0, 0, 0, 0), vb = va;
-            if (lib != kNoSlot) {
-                const size_t src = ((size_t)(lib / cpb) * kMaxChunks + j) * 64 + (lib % cpb) + 32 * (l >> 5);
-                va = g.lib_a[src];
-                vb = g.lib_b[src];
-            }
-            g.out_a[i] = va;
-            g.out_b[i] = vb;
-        }
-    } else {
-        const uint64_t total = (uint64_t)nblk * g.rows * 64;
-        for (uint64_t i = t0; i < total; i += stride) {
-            const uint32_t l = (uint32_t)(i & 63), p = (uint32_t)((i >> 6) % g.rows);
-            const uint32_t b = (uint32_t)(i / (64 * (uint64_t)g.rows));
-            const uint32_t lib = g.slot_map[b * cpb + (l & 15)];
-            float v = 0.f;
-            if (lib != kNoSlot) v = g.lib_w[((size_t)(lib / cpb) * g.rows + p) * 64 + (lib % cpb) + 16 * (l >> 4)];
-            g.out_w[i] = v;
-        }
+    constexpr uint32_t cpb = kFp32Cols;
+    const uint64_t total = (uint64_t)nblk * g.rows * 64;
+    for (uint64_t i = t0; i < total; i += stride) {
+        const uint32_t l = (uint32_t)(i & 63), p = (uint32_t)((i >> 6) % g.rows);
+        const uint32_t b = (uint32_t)(i / (64 * (uint64_t)g.rows));
+        const uint32_t lib = g.slot_map[b * cpb + (l & 15)];
+        float v = 0.f;
+        if (lib != kNoSlot) v = g.lib_w[((size_t)(lib / cpb) * g.rows + p) * 64 + (lib % cpb) + 16 * (l >> 4)];
+        g.out_w[i] = v;
     }
     for (uint64_t s = t0; s < (uint64_t)nblk * cpb; s += stride) {
         const uint32_t lib = g.slot_map[s];
         g.out_band[s] = lib != kNoSlot ? g.lib_band[lib] : 0.0;
-        g.out_band_hi[s] = lib != kNoSlot ? g.lib_band_hi[lib] : 0.0;
     }
 }
+#endif
 
 }  // namespace blamm

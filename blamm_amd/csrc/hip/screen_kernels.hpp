@@ -1,5 +1,5 @@
-// The screen: the filter of the default scan form, on FP6 x FP4 matrix-core
-// tiles.
+// The screen: the filter of the default scan form, and the first stage of the
+// split-BF16 form's, on FP6 x FP4 matrix-core tiles.
 //
 // A scan must find every window whose score clears its column's threshold;
 // nearly all of the ~1e11 windows of a scan are far below it.  The screen
@@ -63,6 +63,13 @@ struct ScreenArgs {
     uint4* cand;
     unsigned long long* counters;
     uint64_t cand_cap;
+    // LO variants: the library's split-BF16 fragments, bands and lengths, and
+    // the library slot of a batch's slot (list form)
+    const uint4* hi;                 // [block][chunk][lane]
+    const uint4* lo;
+    const double* band;
+    const int* len;
+    const uint32_t* slot_map;
 };
 
 // Smallest accumulator value a window that reaches threshold t can have,
@@ -179,24 +186,113 @@ __device__ __forceinline__ void screen_emit(const ScreenArgs& a, ScreenStage& st
     st.n += (uint32_t)__popcll(m);
 }
 
-// Test block blk of tile t.
-__device__ __forceinline__ void screen_check(const ScreenArgs& a, ScreenStage& st, const f32x16& acc, float th,
-                                             uint32_t t, uint32_t blk)
+// The split-BF16 form (LO): a tile block that the screen cannot rule out is
+// scored with the hi and lo products of its columns (as in bf16_mfma_tile), and
+// its windows at or above thr - band, the proven band of that score, become
+// records.  The screen marks such blocks over kSplitTiles tiles, one bit each,
+// and this goes through the marked tiles ts + bit of one column block with the
+// block's fragments in registers: read again for each tile block they are more
+// than the caches deliver.  One tile block in seven is marked at p = 1e-4:
+// 16 Mbp x 1,000 columns take 1.27 ms (2.35 with the fragments read for each,
+// 2.05 with hi products for every window and lo products for blocks that pass;
+// where nearly all are marked, 10 Mbp x 600 long columns at p = 1e-3, as much
+// as the latter: 2.98).
+constexpr uint32_t kSplitTiles = 64;
+
+template <int KS, bool MASK, bool LIST>
+__device__ __forceinline__ void screen_split(const ScreenArgs& a, ScreenStage& st, uint32_t blk, uint32_t ts,
+                                             uint64_t marked)
 {
-    const f32x16& v = acc_read<AccRead::kGuard>(acc);
-    const bool pred = tile_max<1>(v) >= th;
-    const uint64_t m = __ballot(pred);
-    if (m) screen_emit(a, st, v, th, pred, m, t, blk);
+    const uint32_t lane = screen_lane(), slot = blk * kBf16Cols + (lane & 31);
+    uint32_t lib = slot;
+    if constexpr (LIST) {
+        lib = a.slot_map[slot];
+        if (lib == kNoSlot) lib = 0;       // its threshold is +inf
+    }
+    const float th = thr_minus(a.thr[slot], a.band[lib]);
+    const size_t row = (size_t)(lib / kBf16Cols) * kMaxChunks * 64 + (lane & 32) + lib % kBf16Cols;
+    // chunks of four positions: up to three at the end may be empty
+    constexpr int kFull = 4 * KS - 3;
+    const int len = a.len[lib];
+    int nch = kFull;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) nch += __ballot(len > 4 * (kFull + j)) != 0;
+    bf16x8 hi[4 * KS], lo[4 * KS];
+#pragma unroll
+    for (int j = 0; j < 4 * KS; ++j) {
+        hi[j] = __builtin_bit_cast(bf16x8, a.hi[row + (size_t)j * 64]);
+        lo[j] = __builtin_bit_cast(bf16x8, a.lo[row + (size_t)j * 64]);
+    }
+    const uint32_t off = (lane & 31) + 2 * (lane >> 5);   // first base of the lane's window, 0..33
+    const uint32_t sh = 2 * (off & 15), po = 4 * (off >> 4), mo = 4 * (off >> 5);
+    constexpr int NW = KS == 1 ? 1 : KS < 4 ? 2 : 3, NM = KS > 2 ? 3 : 2;
+    uint64_t w[3] = {0, 0, 0};
+    uint32_t mw[3] = {0, 0, 0};
+    auto load = [&](uint32_t t) __attribute__((always_inline)) {
+        const char* pk = (const char*)(a.packed + t);
+#pragma unroll
+        for (int i = 0; i < NW; ++i) w[i] = *(const u64_a4*)(pk + 8 * i + po);
+        if (MASK) {
+            const char* mk = (const char*)((const uint32_t*)a.lcmask + t);
+#pragma unroll
+            for (int i = 0; i < NM; ++i) mw[i] = *(const uint32_t*)(mk + 4 * i + mo);
+        }
+    };
+    uint32_t t = ts + (uint32_t)__builtin_ctzll(marked);
+    load(t);
+    for (;;) {
+        const OneHotSrc bits = onehot_src<4 * KS>(w[0], w[1], w[2], sh);
+        const uint64_t mb = MASK ? window_mask<4 * KS>(mw[0], mw[1], mw[2], off & 31) : 0ull;
+        marked &= marked - 1;
+        const uint32_t now = t;
+        if (marked) {
+            t = ts + (uint32_t)__builtin_ctzll(marked);
+            load(t);
+        }
+        f32x16 acc = {0.f};
+        auto chunk = [&](int j) __attribute__((always_inline)) {
+            const bf16x8 A = onehot_chunk<MASK>(bits, mb, j);
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A, hi[j], acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A, lo[j], acc, 0, 0, 0);
+        };
+#pragma unroll
+        for (int j = 0; j < kFull; ++j) chunk(j);
+        if (nch > kFull) {
+            chunk(kFull);
+            if (nch > kFull + 1) {
+                chunk(kFull + 1);
+                if (nch > kFull + 2) chunk(kFull + 2);
+            }
+        }
+        const f32x16& v = acc_read(acc);
+        const bool pred = tile_max(v) >= th;
+        const uint64_t m = __ballot(pred);
+        if (m) screen_emit(a, st, v, th, pred, m, now, blk);
+        if (!marked) break;
+    }
 }
 
+// Test block blk of tile t (LO: bit `bit` of mark).
+template <bool LO>
+__device__ __forceinline__ void screen_check(const ScreenArgs& a, ScreenStage& st, const f32x16& acc, float th,
+                                             uint32_t t, uint32_t blk, uint32_t bit, uint64_t& mark)
+{
+    const f32x16& v = acc_read(acc);
+    const bool pred = tile_max(v) >= th;
+    const uint64_t m = __ballot(pred);
+    if (m) {
+        if constexpr (LO) mark |= 1ull << bit;
+        else screen_emit(a, st, v, th, pred, m, t, blk);
+    }
+}
 
 // Tiles [t0, t1) of column blocks blk0 .. blk0+NB-1.  Two accumulators
 // alternate over the tile blocks: block b + 1's products (or the next tile's
 // first) are issued before block b is tested, so the wave's own tests run
-// beside its products.
-template <int KS, int NB, bool MASK>
+// beside its products.  LO: mark[b] gets block b's tiles, from t0 on.
+template <int KS, int NB, bool MASK, bool LO>
 __device__ __forceinline__ void screen_range(const ScreenArgs& a, ScreenStage& st, uint32_t blk0, uint32_t t0,
-                                             uint32_t t1)
+                                             uint32_t t1, uint64_t (&mark)[NB])
 {
     const uint32_t lane = screen_lane();
     i32x6 B[NB][KS];
@@ -246,7 +342,7 @@ __device__ __forceinline__ void screen_range(const ScreenArgs& a, ScreenStage& s
             const f32x16 acc = product(0);
             rows.build(w, mw, sh, msh);
             load(t + 2);
-            screen_check(a, st, acc, th[0], t, blk0);
+            screen_check<LO>(a, st, acc, th[0], t, blk0, t - t0, mark[0]);
         }
     } else {
         static_assert(NB % 2 == 0, "block pairs alternate between two accumulators");
@@ -262,19 +358,42 @@ __device__ __forceinline__ void screen_range(const ScreenArgs& a, ScreenStage& s
                     load(t + 2);
                 }
                 acc[(b + 1) & 1] = product((b + 1) % NB);
-                screen_check(a, st, acc[b & 1], th[b], t, blk0 + b);
+                screen_check<LO>(a, st, acc[b & 1], th[b], t, blk0 + b, t - t0, mark[b]);
             }
         }
     }
 }
 
-template <bool MASK>
+template <int KS, int NB, bool MASK, bool LIST, bool LO>
+__device__ __forceinline__ void screen_tiles(const ScreenArgs& a, ScreenStage& st, uint32_t blk0, uint32_t t0,
+                                             uint32_t t1)
+{
+    if constexpr (LO) {
+        for (uint32_t t = t0; t < t1; t += kSplitTiles) {
+            uint64_t mark[NB] = {};
+            screen_range<KS, NB, MASK, true>(a, st, blk0, t, min(t1, t + kSplitTiles), mark);
+#pragma unroll 1
+            for (int b = 0; b < NB; ++b) {
+                uint64_t m = mark[0];
+#pragma unroll
+                for (int i = 1; i < NB; ++i)
+                    if (b == i) m = mark[i];
+                if (m) screen_split<KS, MASK, LIST>(a, st, blk0 + b, t, m);
+            }
+        }
+    } else {
+        uint64_t mark[NB];
+        screen_range<KS, NB, MASK, false>(a, st, blk0, t0, t1, mark);
+    }
+}
+
+template <bool MASK, bool LIST, bool LO>
 __device__ __forceinline__ void screen_item(const ScreenArgs& a, ScreenStage& st, uint32_t grp, uint32_t t0,
                                             uint32_t t1)
 {
     const uint32_t blk0 = grp & 0xFFFFFu, steps = (grp >> 20) & 63u, nb = grp >> 26;
     switch (steps * 16 + nb) {
-#define BLAMM_SCREEN(S, N) case S * 16 + N: screen_range<S, N, MASK>(a, st, blk0, t0, t1); break;
+#define BLAMM_SCREEN(S, N) case S * 16 + N: screen_tiles<S, N, MASK, LIST, LO>(a, st, blk0, t0, t1); break;
     BLAMM_SCREEN(1, 8) BLAMM_SCREEN(1, 4) BLAMM_SCREEN(1, 2) BLAMM_SCREEN(1, 1)
     BLAMM_SCREEN(2, 4) BLAMM_SCREEN(2, 2) BLAMM_SCREEN(2, 1)
     BLAMM_SCREEN(3, 2) BLAMM_SCREEN(3, 1)
@@ -284,13 +403,15 @@ __device__ __forceinline__ void screen_item(const ScreenArgs& a, ScreenStage& st
     }
 }
 
-template <bool MASK, bool LIST>
-__global__ __launch_bounds__(kThreads, 4) void screen_kernel(ScreenArgs a, WorkQueue q, ListArgs l)
+// (the LO variants' second look at a tile block takes registers of its own:
+// three waves per SIMD)
+template <bool MASK, bool LIST, bool LO>
+__global__ __launch_bounds__(kThreads, LO ? 3 : 4) void screen_kernel(ScreenArgs a, WorkQueue q, ListArgs l)
 {
     __shared__ uint4 stage_lds[kWavesPerBlock][kScreenStage];
     ScreenStage st{stage_lds[__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)], 0u};
     for_each_item<LIST>(a.counters, a.groups, q, l, [&](uint32_t grp, uint32_t t0, uint32_t t1) __attribute__((always_inline)) {
-        screen_item<MASK>(a, st, grp, t0, t1);
+        screen_item<MASK, LIST, LO>(a, st, grp, t0, t1);
     });
     last_records(a, st.buf, st.n);
 }

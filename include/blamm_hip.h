@@ -59,8 +59,8 @@ enum blamm_precision {
                                  window's score (exact sums on the matrix cores) and keeps
                                  every window the bound cannot rule out; histograms use
                                  the PWM split into bf16 hi+lo */
-    BLAMM_PREC_BF16X2_LO = 2  /* PWM split into bf16 hi+lo; tile blocks the hi terms do
-                                 not rule out also get their lo products on BF16 MFMA */
+    BLAMM_PREC_BF16X2_LO = 2  /* PWM split into bf16 hi+lo; tile blocks the bound does not
+                                 rule out get their hi and lo products on BF16 MFMA */
 };
 
 /* One occurrence.  pos: position in the packed stream of the scan call;
@@ -212,14 +212,14 @@ typedef struct blamm_tuning {
                                   most (smaller scans use smaller items) */
     uint32_t blocks_per_wave;  /* motif tile: column blocks (32 bf16 / 16 fp32
                                   columns each) a wave scores at once: 1, 2
-                                  (bf16 at most 2, fp32 at most 4); the default
-                                  form scores 4 times as many blocks of motifs
+                                  (bf16 at most 2, fp32 at most 4); the bf16
+                                  forms score 4 times as many blocks of motifs
                                   up to 16 positions, twice as many up to 32;
                                   the fp32 form twice as many, up to 4 (motifs
                                   up to 24 positions) or 2 (up to 32) */
     uint32_t kpad_positions;   /* K-padding: a block's motif length is rounded
                                   up to a multiple of 4 or 8 positions (the
-                                  default form: always 16) */
+                                  scans of the bf16 forms: always 16) */
 } blamm_tuning;
 
 int blamm_hip_get_tuning(blamm_hip_ctx *ctx, blamm_tuning *t);
