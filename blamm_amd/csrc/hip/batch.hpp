@@ -337,7 +337,6 @@ int batch_enqueue_kernels(blamm_hip_batch* b, bool mask, uint32_t grid)
 {
     blamm_hip_ctx* c = b->ctx;
     const bool bf = prec_bf(c->precision);
-    hipLaunchKernelGGL(zero_counters_kernel, dim3(1), dim3(64), 0, b->stream, b->counters.p);
     GroupArgs g;
     g.desc = b->desc.p;
     g.counters = b->counters.p;
@@ -349,11 +348,10 @@ int batch_enqueue_kernels(blamm_hip_batch* b, bool mask, uint32_t grid)
     g.req_off = b->req_off.p;
     g.cursor = b->cursor.p;
     g.req_start = b->req_start.p;
-    // finalize counts hits per request into req_count
-    hipLaunchKernelGGL(group_clear_kernel, dim3(64), dim3(kGroupThreads), 0, b->stream, g);
-    // run-start bits of the batch stream (request starts included)
-    hipLaunchKernelGGL(run_bits_clear_kernel, dim3((uint32_t)c->num_cu * 4), dim3(256), 0, b->stream, b->run_bits.p,
-                       0u, (const BatchDesc*)b->desc.p);
+    // counters, hits per request (finalize counts them) and the run-start bits
+    // of the batch stream (request starts included)
+    hipLaunchKernelGGL(scan_clear_kernel, dim3((uint32_t)c->num_cu * 4), dim3(256), 0, b->stream, b->counters.p,
+                       b->run_bits.p, 0u, (const BatchDesc*)b->desc.p, b->req_count.p);
     hipLaunchKernelGGL(run_bits_set_kernel, dim3((uint32_t)c->num_cu), dim3(256), 0, b->stream, b->run_bits.p,
                        (const uint64_t*)b->runs.p, 0u, 0u, (const BatchDesc*)b->desc.p);
     HIP_TRY(hipGetLastError());

@@ -875,13 +875,14 @@ int enqueue_scan(blamm_hip_ctx* c, const uint64_t* d_packed, const uint64_t* d_l
 {
     const bool bf = prec_bf(c->precision);
     const bool mask = d_lcmask != nullptr;
-    hipLaunchKernelGGL(zero_counters_kernel, dim3(1), dim3(64), 0, s, counters);
-    HIP_TRY(hipGetLastError());
     if (nruns == 0) run_bits = nullptr;   // nothing to search
-    if (run_bits) {
+    if (!run_bits) {
+        hipLaunchKernelGGL(zero_counters_kernel, dim3(1), dim3(64), 0, s, counters);
+        HIP_TRY(hipGetLastError());
+    } else {
         const uint32_t words = (uint32_t)(nbases / 64 + 2);
-        hipLaunchKernelGGL(run_bits_clear_kernel, dim3(std::min<uint32_t>((words + 255) / 256, 4096)), dim3(256), 0, s,
-                           run_bits, (uint32_t)nbases, (const BatchDesc*)nullptr);
+        hipLaunchKernelGGL(scan_clear_kernel, dim3(std::min<uint32_t>((words + 255) / 256, 4096)), dim3(256), 0, s,
+                           counters, run_bits, (uint32_t)nbases, (const BatchDesc*)nullptr, (uint32_t*)nullptr);
         hipLaunchKernelGGL(run_bits_set_kernel, dim3(std::min<uint32_t>((uint32_t)((nruns + 255) / 256), 4096)),
                            dim3(256), 0, s, run_bits, d_run_starts, (uint32_t)nruns, (uint32_t)nbases,
                            (const BatchDesc*)nullptr);

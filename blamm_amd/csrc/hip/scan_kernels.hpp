@@ -931,23 +931,31 @@ __global__ __launch_bounds__(kThreads) void finalize_kernel(FinalizeArgs a)
 }
 
 #ifndef BLAMM_INSTANTIATE   // small kernels: launched from the main unit only
-static __global__ void zero_counters_kernel(unsigned long long* c)
+__device__ __forceinline__ void zero_counters(unsigned long long* c)
 {
-    for (uint32_t i = threadIdx.x; i < (uint32_t)kCntHeads; i += 64) c[i] = 0ull;
-    for (uint32_t i = threadIdx.x; i < (uint32_t)kQueues; i += 64) c[kCntHeads + i * kCntLine] = 0ull;
+    for (uint32_t i = threadIdx.x; i < (uint32_t)kCntHeads; i += blockDim.x) c[i] = 0ull;
+    for (uint32_t i = threadIdx.x; i < (uint32_t)kQueues; i += blockDim.x) c[kCntHeads + i * kCntLine] = 0ull;
 }
+
+static __global__ void zero_counters_kernel(unsigned long long* c) { zero_counters(c); }
 
 // Run-start bits for finalize_kernel: bit i is set when a run starts at base
 // i (0 < i < nbases).  The clear kernel zeroes words [0, nbases / 64 + 2)
-// (what load_bits64 may read below q + 1 <= nbases); the set kernel then
-// sets one bit per run start.  List form: sizes from the batch descriptor.
-static __global__ __launch_bounds__(256) void run_bits_clear_kernel(uint64_t* bits, uint32_t nbases,
-                                                                    const BatchDesc* desc)
+// (what load_bits64 may read below q + 1 <= nbases), and what else a scan
+// needs cleared: the counters and a batch's hits per request, in one launch
+// (a launch costs a small scan ~8 us, the kernel 2).  The set kernel then sets
+// one bit per run start.  List form: sizes from the batch descriptor.
+static __global__ __launch_bounds__(256) void scan_clear_kernel(unsigned long long* counters, uint64_t* bits,
+                                                                uint32_t nbases, const BatchDesc* desc,
+                                                                uint32_t* req_count)
 {
     const uint32_t n = desc ? desc->nbases : nbases;
     const uint64_t words = (uint64_t)n / 64 + 2;
-    for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < words; i += (uint64_t)gridDim.x * 256)
-        bits[i] = 0ull;
+    const uint64_t first = (uint64_t)blockIdx.x * 256 + threadIdx.x, stride = (uint64_t)gridDim.x * 256;
+    if (blockIdx.x == 0) zero_counters(counters);
+    for (uint64_t i = first; i < words; i += stride) bits[i] = 0ull;
+    if (desc)
+        for (uint64_t i = first; i < desc->nreq; i += stride) req_count[i] = 0u;
 }
 
 static __global__ __launch_bounds__(256) void run_bits_set_kernel(uint64_t* bits, const uint64_t* starts,
@@ -979,20 +987,13 @@ struct GroupArgs {
     uint64_t out_cap;                     // grouped output capacity
     const DevHit* in;                     // finalize output, pos = request << 32 | batch position
     GroupedHit* out;                      // grouped, request-local positions
-    uint32_t* req_count;                  // [nreq] hits per request, cleared by group_clear_kernel
+    uint32_t* req_count;                  // [nreq] hits per request, cleared by scan_clear_kernel
     unsigned long long* req_off;          // [nreq + 1] exclusive offsets
     unsigned long long* cursor;           // [nreq] next free slot per request
     const uint32_t* req_start;            // [nreq] first batch position of each request
 };
 
 #ifndef BLAMM_INSTANTIATE
-static __global__ __launch_bounds__(kGroupThreads) void group_clear_kernel(GroupArgs g)
-{
-    const uint32_t nreq = g.desc->nreq;
-    for (uint32_t i = blockIdx.x * kGroupThreads + threadIdx.x; i < nreq; i += gridDim.x * kGroupThreads)
-        g.req_count[i] = 0u;
-}
-
 __device__ __forceinline__ uint64_t group_nhits(const GroupArgs& g)
 {
     const uint64_t n = g.counters[kCntHits];
