@@ -10,9 +10,9 @@ theoretical histogram's cutoff at p = 1e-5).  Synthetic, seeded.
 A step is one scan of all four groups, each against its own resident library
 (one engine context per group): MFMA filter kernel + exact finalize (run
 boundaries, FP64 band rescoring) + hit count read-back per group.  Inputs are
-in HBM before timing starts.  `value` is the split-BF16 (hi-only filter)
-throughput in Gbp*motifs/s; the FP32 scan of the same groups, the lazy-lo
-form and an FP64-oracle slice check ride in the same line, with the plain-GPU
+in HBM before timing starts.  `value` is the default form's throughput in
+Gbp*motifs/s; the FP32 scan of the same groups, the form with hi and lo
+products and an FP64-oracle slice check ride in the same line, with the plain-GPU
 workload (100 Mbp x 2,000 columns), the batched and serving workloads, hist -e
 and the reference's CPU configuration as side legs.  Prints one JSON line.
 """
@@ -29,7 +29,7 @@ import numpy as np
 REPO = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, REPO)
 
-PEAK_BF16_TFLOPS = 2500.0     # MI355X dense BF16 MFMA
+PEAK_FP6_TFLOPS = 10000.0     # MI355X dense FP6/FP4 MFMA
 PEAK_FP32_TFLOPS = 157.3      # MI355X FP32 MFMA
 PEAK_HBM_GBS = 8000.0
 PEAK_SCLK_MHZ = 2400.0        # MI355X peak engine clock, at which the MFMA peaks are quoted
@@ -39,7 +39,8 @@ def log(msg: str) -> None:
     print(f"[bench] {msg}", file=sys.stderr, flush=True)
 
 
-SOURCE_FILES = ("blamm_amd/csrc/hip/scan_kernels.hpp", "blamm_amd/csrc/hip/blamm_hip.hip")
+SOURCE_FILES = ("blamm_amd/csrc/hip/scan_kernels.hpp", "blamm_amd/csrc/hip/screen_kernels.hpp",
+                "blamm_amd/csrc/hip/blamm_hip.hip")
 
 
 def source_hash() -> str:
@@ -897,7 +898,7 @@ def main():
     ap.add_argument("--cpu-budget", type=float, default=15.0)
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--no-fp32", action="store_true")
-    ap.add_argument("--no-lo", action="store_true", help="skip the lazy-lo form of the split-BF16 scan")
+    ap.add_argument("--no-lo", action="store_true", help="skip the form with hi and lo products (bf16x2lo)")
     ap.add_argument("--no-tune", action="store_true", help="keep the default tile shapes")
     ap.add_argument("--no-check", action="store_true", help="skip the FP64-oracle slices")
     ap.add_argument("--tune-cache", default=os.path.join(os.path.expanduser("~"), ".cache", "blamm_amd", "tune.txt"))
@@ -954,7 +955,7 @@ def main():
     keys_bf = [hit_keys(h) for h in bf_hits]
     value = nbp * ncols / (bf["ms_per_step"] / 1e3) / 1e9
     achieved = flops_launch / (bf["filter_ms_per_launch"] / 1e3) / 1e12
-    prof = profile_figures("filter_persistent_config2_traffic.txt") or {}
+    prof = profile_figures("screen_config2_traffic.txt") or {}
     traffic = None
     if prof and not prof.get("stale") and "traffic_bytes_per_launch" in prof:
         traffic = float(prof["traffic_bytes_per_launch"])
@@ -977,38 +978,38 @@ def main():
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": "bf16x2 (hi terms on MFMA)->f32 (+f32/f64 rescoring)",
+        "dtype": "f32 scores (f64 near a threshold) behind an exact integer bound on FP6 x FP4 MFMA",
         "data": "synthetic (seeded)",
         "config": {"workload": f"precision config: {ncols // 2} motifs (L 5-30, Dirichlet 0.3) fwd+rc = {ncols} "
                                f"columns, {len(groups)} groups x {args.precision_bases / 1e6:g} Mbp GC U(0.35,0.50), "
                                f"own background/PWMs/thresholds per group, p=1e-5",
                    "bases": nbp, "columns": ncols, "groups": len(groups), "pvalue": 1e-5,
-                   "precision": "split-bf16, hi-only filter"},
-        "roofline": {"bound": "mfma", "achieved": achieved, "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
-                     "frac": achieved / PEAK_BF16_TFLOPS, "traffic": traffic,
-                     "kernel": "filter_persistent_kernel<true,false,false> (one launch per group)",
+                   "precision": "bf16x2 (default form: integer screen, f32/f64 decision)"},
+        "roofline": {"bound": "mfma", "achieved": achieved, "peak": PEAK_FP6_TFLOPS, "unit": "TFLOP/s",
+                     "frac": achieved / PEAK_FP6_TFLOPS, "traffic": traffic,
+                     "kernel": "screen_kernel<false,false,false> (one launch per group)",
                      "algorithmic_flops_per_launch": flops_launch,
-                     "traffic_source": "profiles/filter_persistent_config2_traffic.txt"
+                     "traffic_source": "profiles/screen_config2_traffic.txt"
                                        + ("" if traffic is not None else " (absent or taken on other sources)"),
                      "source_sha": source_hash()},
         # the published peak assumes the 2.4 GHz peak engine clock; under this
         # sustained MFMA load the chip holds a lower clock (sampled above)
         "clock": None if sclk is None else dict(
-            sclk, peak_at_clock_TFLOPs=PEAK_BF16_TFLOPS * sclk["median_mhz"] / PEAK_SCLK_MHZ,
-            frac_at_clock=achieved / (PEAK_BF16_TFLOPS * sclk["median_mhz"] / PEAK_SCLK_MHZ)),
+            sclk, peak_at_clock_TFLOPs=PEAK_FP6_TFLOPS * sclk["median_mhz"] / PEAK_SCLK_MHZ,
+            frac_at_clock=achieved / (PEAK_FP6_TFLOPS * sclk["median_mhz"] / PEAK_SCLK_MHZ)),
         "hbm": hbm,
         "scan": bf,
     }
     if not args.no_lo:
-        log("split-bf16 lazy-lo")
+        log("split-bf16 with hi and lo products")
         lo, lo_hits = groups_leg(args, groups, ba.PREC_BF16X2_LO, max(2, args.steps // 2), 1)
         lo["value"] = nbp * ncols / (lo["ms_per_step"] / 1e3) / 1e9
         lach = flops_launch / (lo["filter_ms_per_launch"] / 1e3) / 1e12
-        lo.update({"roofline_achieved_TFLOPs": lach, "roofline_frac": lach / PEAK_BF16_TFLOPS,
+        lo.update({"roofline_achieved_TFLOPs": lach, "roofline_frac": lach / PEAK_FP6_TFLOPS,
                    "identical_hit_set": all(np.array_equal(a, hit_keys(b)) for a, b in zip(keys_bf, lo_hits))})
         del lo_hits
         line["split_lazy_lo"] = lo
-        log(f"lazy lo: {lo}")
+        log(f"hi and lo products: {lo}")
     if not args.no_fp32:
         log("fp32")
         fp, fp_hits = groups_leg(args, groups, ba.PREC_FP32, 2, 1)
@@ -1037,7 +1038,7 @@ def main():
             pb, pb_hits = gpu_leg(args, stream, runs, P, lengths, thr, codes, ba.PREC_BF16X2, tune_sample=p_nbp)
             pb["value"] = p_nbp * len(pwms) / (pb["ms_per_step"] / 1e3) / 1e9
             pach = p_flops / (pb["filter_ms"] / 1e3) / 1e12
-            pb.update({"roofline_achieved_TFLOPs": pach, "roofline_frac": pach / PEAK_BF16_TFLOPS,
+            pb.update({"roofline_achieved_TFLOPs": pach, "roofline_frac": pach / PEAK_FP6_TFLOPS,
                        "workload": f"plain-GPU config: {len(pwms) // 2} motifs (L 5-30) fwd+rc = {len(pwms)} columns, "
                                    f"{args.bases // 1_000_000} Mbp GC 0.41 CpG 0.2x 0.5% N-runs, p={args.pvalue:g}",
                        "bases": p_nbp, "columns": len(pwms)})

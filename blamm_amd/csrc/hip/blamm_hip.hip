@@ -122,15 +122,19 @@ struct GroupInfo {
 }  // namespace
 
 // Scratch of blamm_hip_scan_device_noalloc: the scan counters (first 8,448
-// bytes) and BLAMM_NOALLOC_MAX_RECORDS filter records of 16 bytes, 64 MiB in
-// all.  Every GPU the library runs on holds its own copy until the process
+// bytes) and filter records of 16 bytes, 90 MiB in all.  The records are 1.4
+// times BLAMM_NOALLOC_MAX_RECORDS: with many lowercase bases the screen leaves
+// about a third more of them than scores on BF16 products would (416k against
+// 315k at 24 Mbp x 1,000 columns), and a scan within the limit by that count
+// must fit.  Every GPU the library runs on holds its own copy until the process
 // ends; all contexts on one GPU share it, so no-alloc scans that overlap on
 // one GPU race.  Host code never uses the array's name as an address: the
 // device address of each GPU's copy comes from hipGetSymbolAddress, taken
 // once per device in blamm_hip_create with that device current.
 constexpr uint64_t kNoAllocHeader = 8448;
+constexpr uint64_t kNoAllocRecords = (uint64_t)BLAMM_NOALLOC_MAX_RECORDS / 5 * 7;
 static_assert(kCntSlots * sizeof(unsigned long long) <= kNoAllocHeader, "counters exceed the scratch header");
-static __device__ __align__(256) uint8_t scratch[kNoAllocHeader + (uint64_t)BLAMM_NOALLOC_MAX_RECORDS * 16];
+static __device__ __align__(256) uint8_t scratch[kNoAllocHeader + kNoAllocRecords * 16];
 
 namespace {
 
@@ -972,7 +976,7 @@ int blamm_hip_scan_device_noalloc(blamm_hip_ctx* c, const uint64_t* d_packed, ui
     hipStream_t s = stream ? (hipStream_t)stream : c->stream;
     c->pending_noalloc = true;
     return enqueue_scan(c, d_packed, d_lcmask, nbases, d_run_starts, nruns, d_hits, cap, d_nhits,
-                        (uint4*)(base + kNoAllocHeader), (uint64_t)BLAMM_NOALLOC_MAX_RECORDS,
+                        (uint4*)(base + kNoAllocHeader), kNoAllocRecords,
                         (unsigned long long*)base, nullptr, s);
 }
 
@@ -1001,7 +1005,7 @@ int blamm_hip_scan_finish(blamm_hip_ctx* c, uint64_t* nhits)
         if (c->pending_noalloc)
             return fail(BLAMM_ERR_OVERFLOW, "scan_noalloc: " + std::to_string(cnt[kCntCand]) +
                                                 " filter records, more than the no-alloc scratch holds (" +
-                                                std::to_string(c->pending_cand_cap) +
+                                                std::to_string(BLAMM_NOALLOC_MAX_RECORDS) +
                                                 "); scan a shorter stream or fewer columns per call");
         // Grow the scratch so that a retry holds every candidate.
         HIP_TRY(c->cand.reserve((size_t)(cnt[kCntCand] + cnt[kCntCand] / 4 + 1024)));

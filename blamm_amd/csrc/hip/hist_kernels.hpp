@@ -9,8 +9,8 @@
 // The score binned here is the FP32 sum of the window's weights in position
 // order (lowercase bases contribute nothing).
 //
-// hist_filter_kernel scores windows with the same hi+lo MFMA tiles as the
-// scan and decides a window's bin from its MFMA score a when that is safe:
+// hist_filter_kernel scores windows with hi+lo MFMA tiles (those of the scan's
+// split-BF16 form) and decides a window's bin from its MFMA score a when that is safe:
 // x = fma(a, 1/width, -min/width) approximates the bin coordinate of the FP32
 // score to within a per-column margin m (from the split and summation error
 // bounds and the rounding of every float step, computed on the host), so when

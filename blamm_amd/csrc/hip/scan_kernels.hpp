@@ -9,7 +9,8 @@
 // from 2-bit packed bases, the product runs on MFMA with FP32 accumulation, and
 // the threshold test plus hit compaction run in the epilogue, so R never
 // reaches HBM.  The MFMA score only filters: a window becomes a candidate when
-// it clears thr - band (band = proven bound on |MFMA score - FP64 score|).
+// it clears thr - band (band = proven bound on |MFMA score - FP64 score|), or,
+// in the bf16 forms, first an upper bound of the score (screen_kernels.hpp).
 // finalize_kernel then applies the run-boundary rule and decides every
 // candidate exactly against the FP64 left-to-right sum.
 #pragma once

@@ -23,12 +23,14 @@
 // on the weights' bf16 hi terms with its proven band 14.53M (soft-masked
 // streams, set 1 of the layout below: 416k against 315k for 259k hits).
 //
-// What bounds it: VALU issue.  Per 32 x 32 tile block a wave issues one MFMA
-// per 16 positions (32 cycles of matrix core, 16 of the issue port), 9
-// instructions for the threshold test, a share of the 5 per step that build
-// the rows, and at the p-values in use ~5 on average to record windows.  62.5
-// Mbp x 4,000 columns (motifs of 5-30): 10.0 ms against 22.2 ms for the BF16
-// filter, 24 against 54 ns per SIMD and tile block.
+// What bounds it: instruction issue beside the matrix cores.  Per 32 x 32 tile
+// block a wave issues one MFMA per 16 positions (32 cycles of matrix core, 16
+// of the issue port), 9 VALU instructions for the threshold test, a share of
+// the 5 per step that build the rows, and a few on average to record windows:
+// at 62.5 Mbp x 4,000 columns (motifs of 5-30, p = 1e-5) 1.54 MFMAs and 13.2
+// VALU instructions, matrix cores busy 65 % of the time and VALU issue 69 %, at
+// the 1.8 GHz that the card holds under this load.  10.0 ms against 22.2 ms for
+// the BF16 filter, 42 against 93 ns per SIMD and tile block.
 #pragma once
 
 #include "scan_kernels.hpp"

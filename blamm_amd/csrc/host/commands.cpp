@@ -487,7 +487,7 @@ int scan_main(int argc, char** argv)
     auto open_device = [&]() {
         if (hc.ctx) return;
         hc.ctx = opener.take("device setup");
-        std::cout << "Using 1 GPU device (" << (precision == BLAMM_PREC_FP32 ? "fp32" : precision == BLAMM_PREC_BF16X2_LO ? "split-bf16, lazy lo" : "split-bf16")
+        std::cout << "Using 1 GPU device (" << (precision == BLAMM_PREC_FP32 ? "fp32" : precision == BLAMM_PREC_BF16X2_LO ? "split-bf16, hi and lo" : "split-bf16")
                   << " MFMA) and " << numThreads << " host thread(s)" << std::endl;
     };
 

@@ -183,11 +183,11 @@ int blamm_hip_scan_finish(blamm_hip_ctx *ctx, uint64_t *nhits);
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc): blamm_hip_scan_device with its scratch -- the scan
  * counters and the filter records -- in a static device array of the library
- * (64 MiB per GPU, held until the process ends) instead of context buffers.
+ * (90 MiB per GPU, held until the process ends) instead of context buffers.
  * It calls no hipMalloc/hipFree, nor does blamm_hip_scan_finish after it.
  * Arguments, result and completion (blamm_hip_scan_finish) are those of
- * blamm_hip_scan_device.  A scan whose filter records exceed
- * BLAMM_NOALLOC_MAX_RECORDS is rejected by scan_finish with
+ * blamm_hip_scan_device.  A scan with up to BLAMM_NOALLOC_MAX_RECORDS filter
+ * records fits; one whose records exceed the array is rejected by scan_finish with
  * BLAMM_ERR_OVERFLOW and *nhits = 0 (nothing is grown; split the stream).
  * Every context on one GPU shares that GPU's array, which keeps the last
  * call's contents: no-alloc scans that overlap on one GPU race. */
