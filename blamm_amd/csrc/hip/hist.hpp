@@ -6,8 +6,8 @@ namespace {
 
 // Bin parameters of every library slot for histograms on [mins[col],
 // maxs[col]] with nbins bins (kernels in hist_kernels.hpp).
-// clamp[block]: some column's scores may leave [-0.5, nbins + 0.5] bins (mask:
-// windows may hold lowercase bases).
+// clamp[block]: some column's scores may leave [-0.5, nbins + 0.5] bins or
+// FP32's range (mask: windows may hold lowercase bases).
 void hist_slot_params(const blamm_hip_ctx* c, const float* mins, const float* maxs, uint32_t nbins, bool mask,
                       std::vector<HistSlot>& hs, std::vector<char>& clamp)
 {
@@ -59,7 +59,12 @@ void hist_slot_params(const blamm_hip_ctx* c, const float* mins, const float* ma
         // i.e. gamma_{10 nch}.  FP32 side: L - 1 round-to-nearest adds.
         const double ds = rep + gamma_n(10.0 * blk_nch[(size_t)s / kBf16Cols], 0x1p-22) * ssplit +
                           gamma_n(L, 0x1p-24) * smax;
-        if (std::isfinite(mn) && std::isfinite(mx) && wd == 0.f) {
+        if (!(smax + ssplit + std::fabs((double)mn) < 0x1p126)) {
+            // a sum, or its distance from mn, may leave FP32's range: bins of
+            // infinite scores only the exact pass knows, and the coordinate
+            // that its windows have all the same stays inside LDS when clamped
+            clamp[(size_t)s / kBf16Cols] = 1;
+        } else if (std::isfinite(mn) && std::isfinite(mx) && wd == 0.f) {
             // (score - min) / 0 is +-inf or NaN for every score; int() of
             // those is INT_MIN, clamped to bin 0
             h.iw = 0.f;

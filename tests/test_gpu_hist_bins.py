@@ -69,3 +69,29 @@ def test_scores_on_bin_edges():
     for nbins in (64, 128):
         got = check(text, runs, pwms, mn, [a + nbins for a in mn], nbins)
     assert got.sum() > 0
+
+
+@pytest.mark.parametrize("longest", [24, 40])
+@pytest.mark.parametrize("lower", [0.0, 0.3])
+@pytest.mark.parametrize("nbins", [1, 250, 512])
+def test_scores_beyond_fp32(nbins, lower, longest):
+    """Finite weights whose sums overflow FP32, beside ordinary columns: an
+    infinite score has no bin coordinate and is counted in the first bin, as
+    int() of the reference's quotient gives it; the same for a width of zero
+    and for a minimum so low that the distance from it overflows."""
+    text, runs, pwms = inputs(nbins + 7, 9_001, [2, 2, 2, 6, 9, longest, 12, 5], lower)
+    mn, mx = (np.asarray(v, np.float64) for v in ranges(pwms))
+    big = 2e38
+    pwms[0] = np.array([[big, -big, 1, 0], [big, -big, 0, 1]], np.float32)
+    mn[0], mx[0] = 0.0, 3e38
+    pwms[1] = pwms[0].copy()
+    mn[1] = mx[1] = 1.0
+    pwms[2] = np.array([[3.4e38, -3.4e38, 1e38, 0], [1, 0, 2, 3]], np.float32)     # bf16 rounds these to infinity
+    mn[2], mx[2] = -1e38, 2e38
+    pwms[3][0, 1] = 2e38
+    mn[3], mx[3] = -2.5e38, 0.5e38
+    pwms[5] = (pwms[5] * 1e37).astype(np.float32)
+    mn[5], mx[5] = -3e37, 2e38
+    with np.errstate(over="ignore"):
+        got = check(text, runs, pwms, mn, mx, nbins)
+    assert got[:3, 0].min() > 0
