@@ -198,7 +198,9 @@ __device__ __forceinline__ uint32_t hist_rows(const HistArgs& a, uint32_t* hl, c
         const int last = (int)a.nbins - 1;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            const float x = __builtin_fmaf(acc[r], h.iw, h.c);
+            // (coordinates are below 2^30; a score that is no number becomes
+            // one, which the columns with such scores never decide: hm < 0)
+            const float x = __builtin_amdgcn_fmed3f(__builtin_fmaf(acc[r], h.iw, h.c), -0x1p30f, 0x1p30f);
             const bool ok = __builtin_fabsf(__builtin_amdgcn_fractf(x) - 0.5f) <= h.hm;
             const uint32_t bin = (uint32_t)min(max((int)x, 0), last);
             if (ok && ((valid >> r) & 1u)) atomicAdd(&a.counts[(size_t)h.slot * a.nbins + bin], 1ull);

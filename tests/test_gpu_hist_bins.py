@@ -73,7 +73,7 @@ def test_scores_on_bin_edges():
 
 @pytest.mark.parametrize("longest", [24, 40])
 @pytest.mark.parametrize("lower", [0.0, 0.3])
-@pytest.mark.parametrize("nbins", [1, 250, 512])
+@pytest.mark.parametrize("nbins", [1, 250, 512, 513])
 def test_scores_beyond_fp32(nbins, lower, longest):
     """Finite weights whose sums overflow FP32, beside ordinary columns: an
     infinite score has no bin coordinate and is counted in the first bin, as
