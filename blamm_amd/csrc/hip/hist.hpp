@@ -32,18 +32,18 @@ void hist_slot_params(const blamm_hip_ctx* c, const float* mins, const float* ma
         double smax = 0.0, ssplit = 0.0, rep = 0.0;   // sum_p max_b |w|, |hi| + |lo|, |w - hi - lo|
         double least = 0.0, most = 0.0;               // sums of the least and largest weights
         for (int p = 0; p < L; ++p) {
-            double m = 0.0, ms = 0.0, me = 0.0, wl = mask ? 0.0 : w[4 * p], wm = wl;
+            double ms = 0.0, me = 0.0;
+            float wl = mask ? 0.f : w[4 * p], wm = wl;
             for (int b = 0; b < 4; ++b) {
                 const float x = w[4 * p + b];
                 const float hf = bf16_to_float(bf16_rne(x));
                 const float lf = bf16_to_float(bf16_rne(x - hf));
-                m = std::max(m, (double)std::fabs(x));
-                wl = std::min(wl, (double)x);
-                wm = std::max(wm, (double)x);
+                wl = std::min(wl, x);
+                wm = std::max(wm, x);
                 ms = std::max(ms, std::fabs((double)hf) + std::fabs((double)lf));
                 me = std::max(me, std::fabs((double)x - (double)hf - (double)lf));
             }
-            smax += m;
+            smax += std::max(-wl, wm);
             ssplit += ms;
             rep += me;
             least += wl;
@@ -100,10 +100,13 @@ void hist_slot_params(const blamm_hip_ctx* c, const float* mins, const float* ma
                 // M = m + e the FP32 score's coordinate lies in
                 // [v - 1 - 2 M, v - 1]: in the unit interval of v - 1 when
                 // fract(v) >= 2 M
-                const double unit = std::ldexp(1.0, -kHistFrac);
+                constexpr double unit = 1.0 / (1 << kHistFrac);
                 const double M = m + unit + (std::fabs((double)cf) + 2.0) * 0x1p-23;
-                h.fc = (float)(std::nearbyint(((double)cf + 1.0 + M) / unit) * unit);
-                h.fthr = (uint32_t)((uint64_t)std::ceil(2.0 * M / unit) << (32 - kHistFrac));
+                // (the sum with 1.5 x 2^52 rounds to a whole number, and a
+                // whole unit more than the margin does no harm: nearbyint and
+                // ceil are calls, 15 us for 1,000 columns)
+                h.fc = (float)((((double)cf + 1.0 + M) / unit + 0x1.8p52 - 0x1.8p52) * unit);
+                h.fthr = (uint32_t)(((uint64_t)(2.0 * M / unit) + 1) << (32 - kHistFrac));
                 const double lo = (least - ds - (double)mn) * inv, hi = (most + ds - (double)mn) * inv;
                 if (lo < -0.5 || hi > (double)nbins + 0.5 || std::fabs((double)cf) > 1000.0)
                     clamp[(size_t)s / kBf16Cols] = 1;
@@ -215,11 +218,16 @@ int blamm_hip_hist_device(blamm_hip_ctx* c, const uint64_t* d_packed, uint64_t p
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kp, kThreads, dyn) != hipSuccess || per_cu < 1)
             per_cu = 1;
         const uint32_t grid = (uint32_t)c->num_cu * (uint32_t)per_cu;
-        // about two items per workgroup, 64..1024 tiles per item: every item
-        // adds its histogram to HBM, which bounds the small calls (400 kbp x
-        // 64 columns: 0.12 ms at 16 tiles, 0.08 at 64)
-        const uint64_t want = ((uint64_t)w.ntiles * w.ngroups + 2ull * grid - 1) / (2ull * grid);
-        w.chunk_tiles = (uint32_t)std::min<uint64_t>(1024, std::max<uint64_t>(64, want));
+        // About two items per workgroup, up to 1,024 tiles each: every item
+        // adds its histogram to HBM, which bounds the small calls.  Those take
+        // items of 16 to 64 tiles, one for every fourth workgroup, so that a
+        // tiny call still spreads (2 kbp x 8 columns: 25 us of kernel, 34 with
+        // one item of 64 tiles) and a small one adds few histograms (20 kbp x
+        // 1,000: 70 us, 116 with 16 tiles each; 400 kbp x 64: 80 and 127).
+        const uint64_t work = (uint64_t)w.ntiles * w.ngroups;
+        const uint64_t want = (work + 2ull * grid - 1) / (2ull * grid);
+        const uint64_t least = std::min<uint64_t>(64, std::max<uint64_t>(16, 4 * work / grid));
+        w.chunk_tiles = (uint32_t)std::min<uint64_t>(1024, std::max<uint64_t>(least, want));
         const uint64_t nchunks = (w.ntiles + w.chunk_tiles - 1) / w.chunk_tiles;
         if (nchunks * w.ngroups >= (1ull << 32)) return fail(BLAMM_ERR_ARG, "hist: work list too long");
         w.nitems = (uint32_t)(nchunks * w.ngroups);

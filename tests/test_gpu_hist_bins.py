@@ -95,3 +95,11 @@ def test_scores_beyond_fp32(nbins, lower, longest):
     with np.errstate(over="ignore"):
         got = check(text, runs, pwms, mn, mx, nbins)
     assert got[:3, 0].min() > 0
+
+
+@pytest.mark.parametrize("n", [1, 33, 511, 513, 2_049, 70_001])
+@pytest.mark.parametrize("columns", [3, 70])
+def test_small_calls(n, columns):
+    """Calls of one work item and of many short ones."""
+    text, runs, pwms = inputs(n, n, [6 + i % 19 for i in range(columns)])
+    check(text, runs, pwms, *ranges(pwms), 250)
