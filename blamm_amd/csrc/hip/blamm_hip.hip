@@ -121,19 +121,20 @@ struct GroupInfo {
 
 }  // namespace
 
-// Scratch of blamm_hip_scan_device_noalloc: the scan counters (first 8,448
+// Scratch of blamm_hip_scan_device_noalloc: two sets of scan counters (16,896
 // bytes) and filter records of 16 bytes, 90 MiB in all.  The records are 1.4
-// times BLAMM_NOALLOC_MAX_RECORDS: with many lowercase bases the screen leaves
-// about a third more of them than scores on BF16 products would (416k against
-// 315k at 24 Mbp x 1,000 columns), and a scan within the limit by that count
-// must fit.  Every GPU the library runs on holds its own copy until the process
-// ends; all contexts on one GPU share it, so no-alloc scans that overlap on
-// one GPU race.  Host code never uses the array's name as an address: the
-// device address of each GPU's copy comes from hipGetSymbolAddress, taken
-// once per device in blamm_hip_create with that device current.
-constexpr uint64_t kNoAllocHeader = 8448;
+// times BLAMM_NOALLOC_MAX_RECORDS, so that most scans with that many records by
+// scores fit at once: the screen leaves up to 1.25 times as many for motifs of
+// 5-25 positions and 1.4 to 1.6 times as many for 24-60 (1 Mbp x 300 columns,
+// p = 1e-2 to 1e-5); the others are filtered a second time (enqueue_scan).
+// Every GPU the library runs on holds its own copy until the process ends; all
+// contexts on one GPU share it, so no-alloc scans that overlap on one GPU race.
+// Host code never uses the array's name as an address: the device address of
+// each GPU's copy comes from hipGetSymbolAddress, taken once per device in
+// blamm_hip_create with that device current.
+constexpr uint64_t kNoAllocHeader = 2 * kCntSet * sizeof(unsigned long long);
 constexpr uint64_t kNoAllocRecords = (uint64_t)BLAMM_NOALLOC_MAX_RECORDS / 5 * 7;
-static_assert(kCntSlots * sizeof(unsigned long long) <= kNoAllocHeader, "counters exceed the scratch header");
+static_assert(kCntSlots <= kCntSet && kNoAllocHeader % 256 == 0, "counters exceed the scratch header");
 static __device__ __align__(256) uint8_t scratch[kNoAllocHeader + kNoAllocRecords * 16];
 
 namespace {
@@ -187,6 +188,7 @@ struct blamm_hip_ctx {
     std::vector<int> slot_col_h;               // -1 = empty slot
     std::vector<double> band_h, seq_h;         // per slot
     double max_filter_band = 0.0, max_score_error = 0.0;
+    bool split_finite = false;                 // no sum of hi and lo terms can leave FP32's range
     DevBuf<uint8_t> frag_a, frag_b;
     DevBuf<float> frag3;                       // FP32 form: three products per position
     DevBuf<double> slot_off3;                  // and what its threshold is lowered by
@@ -223,6 +225,7 @@ struct blamm_hip_ctx {
     uint64_t pending_hit_cap = 0;
     uint64_t pending_cand_cap = 0;            // record capacity the filter was launched with
     unsigned long long* pending_counters = nullptr;
+    unsigned long long* pending_again = nullptr;   // of the filter that ran again if there was no room
     hipStream_t pending_stream = nullptr;
     blamm_scan_stats stats{};
 };
@@ -412,7 +415,7 @@ int relayout(blamm_hip_ctx* c)
     std::vector<double> s_band(nslots, 0.0), s_band_any(nslots, 0.0), s_seq(nslots, 0.0);
     std::vector<double> s_off3(bf ? 0 : nslots, 0.0);
     std::vector<uint16_t> hi16((size_t)nslots * kMaxLen * 4, 0), lo16((size_t)nslots * kMaxLen * 4, 0);
-    double max_band = 0.0, max_err = 0.0;
+    double max_band = 0.0, max_err = 0.0, max_split = 0.0;
     const double u24 = std::ldexp(1.0, -24), u53 = std::ldexp(1.0, -53);
     for (int bi = 0; bi < nblk; ++bi) {
         const int nch = blk_nch[bi];
@@ -491,6 +494,7 @@ int relayout(blamm_hip_ctx* c)
             s_band[slot] = band;
             s_seq[slot] = seq;
             max_band = std::max(max_band, band);
+            max_split = std::max(max_split, sum_split);
             max_err = std::max(max_err, seq);
         }
     }
@@ -611,6 +615,7 @@ int relayout(blamm_hip_ctx* c)
     c->seq_h = s_seq;
     c->max_filter_band = max_band;
     c->max_score_error = max_err;
+    c->split_finite = max_split < 0x1p126;
     c->lib_gen++;
     c->have_lib = true;
     return BLAMM_OK;
@@ -652,6 +657,7 @@ ScreenArgs screen_args(const blamm_hip_ctx* c, const uint64_t* packed, const uin
     a.band = c->slot_band.p;
     a.len = c->slot_len.p;
     a.slot_map = nullptr;
+    a.before = nullptr;
     return a;
 }
 
@@ -662,6 +668,7 @@ FinalizeArgs finalize_args(const blamm_hip_ctx* c, const uint4* cand, uint64_t c
     f.cand = cand;
     f.counters = counters;
     f.counters_rw = counters;
+    f.again = nullptr;
     f.cand_cap = cand_cap;
     f.packed = packed;
     f.lcmask = lcmask;
@@ -886,8 +893,18 @@ int enqueue_scan(blamm_hip_ctx* c, const uint64_t* d_packed, const uint64_t* d_l
     const bool bf = prec_bf(c->precision);
     const bool mask = d_lcmask != nullptr;
     if (nruns == 0) run_bits = nullptr;   // nothing to search
+    // How many records the screen leaves is up to its rounding, which has no
+    // bound in terms of hits (1.1 to 1.6 per hit for 5-60 positions, 3 where a
+    // pseudocount near zero makes one position's weights huge).  Where they
+    // must fit and might not, the split-BF16 filter is launched after it and
+    // runs if they did not: its records are the windows within their band of
+    // the threshold.  If all is well that is a launch that ends at once.
+    unsigned long long* again = nullptr;
+    if (c->pending_noalloc && c->precision == BLAMM_PREC_BF16X2 && c->split_finite &&
+        (nbases + kBf16Tile - 1) / kBf16Tile * 2 * (uint64_t)c->nslots > cand_cap)
+        again = counters + kCntSet;
     if (!run_bits) {
-        hipLaunchKernelGGL(zero_counters_kernel, dim3(1), dim3(64), 0, s, counters);
+        hipLaunchKernelGGL(zero_counters_kernel, dim3(again ? 2 : 1), dim3(64), 0, s, counters);
         HIP_TRY(hipGetLastError());
     } else {
         const uint32_t words = (uint32_t)(nbases / 64 + 2);
@@ -903,21 +920,32 @@ int enqueue_scan(blamm_hip_ctx* c, const uint64_t* d_packed, const uint64_t* d_l
         const uint32_t ntiles = (uint32_t)((nbases + kBf16Tile - 1) / kBf16Tile);   // 32-window tiles
         const FilterArgs a = filter_args(c, d_packed, d_lcmask, c->slot_thr.p, cand, cand_cap, counters);
         const ScreenArgs sa = screen_args(c, d_packed, d_lcmask, c->slot_thr.p, cand, cand_cap, counters);
-        WorkQueue q{};
-        q.ntiles = ntiles;
-        const uint32_t full = (uint32_t)c->num_cu * (uint32_t)persistent_wgs_per_cu(c->precision, mask, false) *
-                              (uint32_t)c->filter_rounds;
-        q.ngroups = c->nscan_groups;
-        q.chunk_tiles = std::min(ntiles, item_tiles((uint64_t)ntiles * q.ngroups, full * kWavesPerBlock,
-                                                    c->tuning.chunk_tiles));
-        q.nchunks = (ntiles + q.chunk_tiles - 1) / q.chunk_tiles;
-        const uint64_t sub = (uint64_t)((q.nchunks + kQueues - 1) / kQueues) * q.ngroups;   // items of queue 0
-        if (sub >= (1ull << 32) - (1u << 16)) return fail(BLAMM_ERR_ARG, "scan: work queue too long");
         const ListArgs l{nullptr, nullptr, nullptr};
-        // no more workgroups than the fullest queue has use for
-        const uint32_t grid = (uint32_t)std::min<uint64_t>(full, (sub + kWavesPerBlock - 1) / kWavesPerBlock * kQueues);
-        hipError_t e = launch_filter(c->precision, mask, false, sa, a, q, l, grid, s);
-        if (e != hipSuccess) return fail(BLAMM_ERR_DEVICE, std::string("filter launch: ") + hipGetErrorString(e));
+        auto filter = [&](int precision, const ScreenArgs& screen) {
+            WorkQueue q{};
+            q.ntiles = ntiles;
+            const uint32_t full = (uint32_t)c->num_cu * (uint32_t)persistent_wgs_per_cu(precision, mask, false) *
+                                  (uint32_t)c->filter_rounds;
+            q.ngroups = c->nscan_groups;
+            q.chunk_tiles = std::min(ntiles, item_tiles((uint64_t)ntiles * q.ngroups, full * kWavesPerBlock,
+                                                        c->tuning.chunk_tiles));
+            q.nchunks = (ntiles + q.chunk_tiles - 1) / q.chunk_tiles;
+            const uint64_t sub = (uint64_t)((q.nchunks + kQueues - 1) / kQueues) * q.ngroups;   // items of queue 0
+            if (sub >= (1ull << 32) - (1u << 16)) return fail(BLAMM_ERR_ARG, "scan: work queue too long");
+            // no more workgroups than the fullest queue has use for
+            const uint32_t grid =
+                (uint32_t)std::min<uint64_t>(full, (sub + kWavesPerBlock - 1) / kWavesPerBlock * kQueues);
+            hipError_t e = launch_filter(precision, mask, false, screen, a, q, l, grid, s);
+            if (e != hipSuccess) return fail(BLAMM_ERR_DEVICE, std::string("filter launch: ") + hipGetErrorString(e));
+            return (int)BLAMM_OK;
+        };
+        BLAMM_TRY(filter(c->precision, sa));
+        if (again) {
+            ScreenArgs split = sa;
+            split.before = counters;
+            split.counters = again;
+            BLAMM_TRY(filter(BLAMM_PREC_BF16X2_LO, split));
+        }
     }
     HIP_TRY(hipEventRecord(c->ev[1], s));
     {
@@ -925,6 +953,7 @@ int enqueue_scan(blamm_hip_ctx* c, const uint64_t* d_packed, const uint64_t* d_l
         f.nbases = (uint32_t)nbases;
         f.nruns = (uint32_t)nruns;
         f.run_bits = run_bits;
+        f.again = again;
         f.hits = d_hits;
         f.hit_cap = cap;
         hipError_t e = launch_finalize(bf, false, f, (uint32_t)c->num_cu * 8, s);
@@ -940,6 +969,7 @@ int enqueue_scan(blamm_hip_ctx* c, const uint64_t* d_packed, const uint64_t* d_l
     c->pending_hit_cap = cap;
     c->pending_cand_cap = cand_cap;
     c->pending_counters = counters;
+    c->pending_again = again;
     c->pending_stream = s;
     return BLAMM_OK;
 }
@@ -995,9 +1025,11 @@ int blamm_hip_scan_finish(blamm_hip_ctx* c, uint64_t* nhits)
     HIP_TRY(hipSetDevice(c->device));
     HIP_TRY(hipStreamSynchronize(c->pending_stream));
     unsigned long long cnt[kCntStats];
-    if (c->pending_noalloc)
+    if (c->pending_noalloc) {
         HIP_TRY(hipMemcpy(cnt, c->pending_counters, sizeof(cnt), hipMemcpyDeviceToHost));
-    else
+        if (c->pending_again && cnt[kCntCand] > c->pending_cand_cap)
+            HIP_TRY(hipMemcpy(&cnt[kCntCand], c->pending_again + kCntCand, sizeof(cnt[0]), hipMemcpyDeviceToHost));
+    } else
         std::memcpy(cnt, c->counters_h.p, sizeof(cnt));
     float ms_f = 0.f, ms_all = 0.f;
     HIP_TRY(hipEventElapsedTime(&ms_f, c->ev[0], c->ev[1]));
@@ -1015,8 +1047,9 @@ int blamm_hip_scan_finish(blamm_hip_ctx* c, uint64_t* nhits)
         if (c->pending_noalloc)
             return fail(BLAMM_ERR_OVERFLOW, "scan_noalloc: " + std::to_string(cnt[kCntCand]) +
                                                 " filter records, more than the no-alloc scratch holds (" +
+                                                std::to_string(kNoAllocRecords) + "; up to " +
                                                 std::to_string(BLAMM_NOALLOC_MAX_RECORDS) +
-                                                "); scan a shorter stream or fewer columns per call");
+                                                " always fit); scan a shorter stream or fewer columns per call");
         // Grow the scratch so that a retry holds every candidate.
         HIP_TRY(c->cand.reserve((size_t)(cnt[kCntCand] + cnt[kCntCand] / 4 + 1024)));
         return fail(BLAMM_ERR_OVERFLOW, "scan: candidate scratch overflowed (grown; retry the scan)");

@@ -45,6 +45,7 @@ constexpr uint32_t kNoSlot = 0xFFFFFFFFu;
 constexpr int kQueues = 64;
 enum { kCntCand = 0, kCntHits = 1, kCntBand = 2, kCntStats = 3, kCntQueue = 4, kCntHeads = 16, kCntLine = 16,
        kCntSlots = kCntHeads + kQueues * kCntLine };
+constexpr int kCntSet = 1056;        // distance of a second set of counters
 
 // 64 consecutive bits of a little-endian bit stream starting at bit `bit`.
 __device__ __forceinline__ uint64_t load_bits64(const uint64_t* __restrict__ words, uint64_t bit)
@@ -650,6 +651,7 @@ __global__ __launch_bounds__(kThreads, MASK ? 2 : 3) void filter_fp32_kernel(Fil
 struct FinalizeArgs {
     const uint4* cand;
     const unsigned long long* counters;   // kCntCand read, kCntHits/kCntBand written
+    const unsigned long long* again;      // null, or the counters of the filter that ran again if there was no room
     unsigned long long* counters_rw;
     uint64_t cand_cap;
     const uint64_t* packed;
@@ -742,7 +744,8 @@ __global__ __launch_bounds__(kThreads) void finalize_kernel(FinalizeArgs a)
         nbases = __builtin_amdgcn_readfirstlane(a.desc->nbases);
         nruns = __builtin_amdgcn_readfirstlane(a.desc->nruns);
     }
-    const uint64_t ncand_raw = a.counters[kCntCand];
+    uint64_t ncand_raw = a.counters[kCntCand];
+    if (a.again && ncand_raw > a.cand_cap) ncand_raw = a.again[kCntCand];
     const uint64_t ncand = ncand_raw < a.cand_cap ? ncand_raw : a.cand_cap;
     const uint32_t lane = threadIdx.x & 63;
     const uint64_t wave = (uint64_t)blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6);
@@ -938,7 +941,8 @@ __device__ __forceinline__ void zero_counters(unsigned long long* c)
     for (uint32_t i = threadIdx.x; i < (uint32_t)kQueues; i += blockDim.x) c[kCntHeads + i * kCntLine] = 0ull;
 }
 
-static __global__ void zero_counters_kernel(unsigned long long* c) { zero_counters(c); }
+// One block per set of counters.
+static __global__ void zero_counters_kernel(unsigned long long* c) { zero_counters(c + blockIdx.x * kCntSet); }
 
 // Run-start bits for finalize_kernel: bit i is set when a run starts at base
 // i (0 < i < nbases).  The clear kernel zeroes words [0, nbases / 64 + 2)

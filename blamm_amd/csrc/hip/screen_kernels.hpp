@@ -72,6 +72,7 @@ struct ScreenArgs {
     const double* band;
     const int* len;
     const uint32_t* slot_map;
+    const unsigned long long* before;   // if set: run only if that filter's records had no room
 };
 
 // Smallest accumulator value a window that reaches threshold t can have,
@@ -410,6 +411,7 @@ __device__ __forceinline__ void screen_item(const ScreenArgs& a, ScreenStage& st
 template <bool MASK, bool LIST, bool LO>
 __global__ __launch_bounds__(kThreads, LO ? 3 : 4) void screen_kernel(ScreenArgs a, WorkQueue q, ListArgs l)
 {
+    if (LO && a.before && a.before[kCntCand] <= a.cand_cap) return;
     __shared__ uint4 stage_lds[kWavesPerBlock][kScreenStage];
     ScreenStage st{stage_lds[__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)], 0u};
     for_each_item<LIST>(a.counters, a.groups, q, l, [&](uint32_t grp, uint32_t t0, uint32_t t1) __attribute__((always_inline)) {

@@ -186,9 +186,13 @@ int blamm_hip_scan_finish(blamm_hip_ctx *ctx, uint64_t *nhits);
  * (90 MiB per GPU, held until the process ends) instead of context buffers.
  * It calls no hipMalloc/hipFree, nor does blamm_hip_scan_finish after it.
  * Arguments, result and completion (blamm_hip_scan_finish) are those of
- * blamm_hip_scan_device.  A scan with up to BLAMM_NOALLOC_MAX_RECORDS filter
- * records fits; one whose records exceed the array is rejected by scan_finish with
- * BLAMM_ERR_OVERFLOW and *nhits = 0 (nothing is grown; split the stream).
+ * blamm_hip_scan_device.  A scan fits if at most BLAMM_NOALLOC_MAX_RECORDS
+ * groups of windows (16 in the bf16 forms, 4 in the fp32 form, of one column)
+ * hold one whose score reaches the threshold or is within the score's error of
+ * it (if the default form's bound leaves more records than the array holds, the
+ * scan filters again with the split-BF16 products); one that does not fit is
+ * rejected by scan_finish with BLAMM_ERR_OVERFLOW and *nhits = 0 (nothing is
+ * grown; split the stream).
  * Every context on one GPU shares that GPU's array, which keeps the last
  * call's contents: no-alloc scans that overlap on one GPU race. */
 #define BLAMM_NOALLOC_MAX_RECORDS 4194304u

@@ -138,3 +138,52 @@ def test_noalloc_rejects_records_beyond_scratch():
         with pytest.raises(ba.BlammError) as e:
             sc.scan_finish()
         assert e.value.code == ba.BLAMM_ERR_OVERFLOW
+
+
+def coarse_library(ncols, seed):
+    """Columns whose first position has one huge negative weight, which leaves
+    the default form's integer bound hardly any resolution for the others, and
+    thresholds that about one window in 2,000 reaches."""
+    rng = np.random.default_rng(seed)
+    pwms = [rng.normal(0, 1, size=(12, 4)).astype(np.float32) for _ in range(ncols)]
+    for w in pwms:
+        w[0] = [-400, 0, 0, 0]
+    sample = synth.CODE2BASE[rng.integers(0, 4, 20_000)]
+    codes = np.searchsorted(np.frombuffer(b"ACGT", np.uint8), sample)
+    thr = []
+    for w in pwms:
+        score = sum(w[p][codes[p:codes.size - 11 + p]] for p in range(12))
+        thr.append(np.partition(score, -10)[-10])
+    return pwms, np.asarray(thr, np.float32)
+
+
+@pytest.mark.parametrize("lower", [0, 7])
+@pytest.mark.parametrize("n", [800_000, 2_000_003])
+def test_noalloc_takes_scans_that_the_bound_leaves_too_many_records_of(n, lower):
+    """Records between the stated maximum and the scratch's size (800,000
+    bases), and more than fit: as long as few windows are near their
+    threshold, both scans succeed, with the hits of scan_device."""
+    import torch
+    rng = np.random.default_rng(n + lower)
+    text = synth.CODE2BASE[rng.integers(0, 4, n)].copy()
+    if lower:
+        text[rng.integers(0, n, n // lower)] |= 0x20
+    text, runs = text.tobytes(), [0, 1000, n // 2]
+    pwms, thr = coarse_library(96, 5)
+    P, L, _ = ba.build_pattern_matrix(pwms)
+    cap = 1 << 20
+    with ba.HipScanner(0) as sc:
+        sc.set_library(P, L, thr, ba.PREC_BF16X2)
+        sc.reserve(1 << 24)
+        d_codes, d_low, d_runs = device_stream(text, runs)
+        d_hits = torch.zeros(2 * cap, dtype=torch.int64, device="cuda:0")
+        sc.scan_device(d_codes, d_low, n, d_runs, len(runs), d_hits, cap, None)
+        assert sc.scan_finish() > 1000
+        records = sc.stats().candidates
+        say(f"noalloc: {n} bases, {records} records of the default form")
+        assert records > MAX_RECORDS and (n < 1_000_000) == (records <= MAX_RECORDS // 5 * 7)
+        for _ in range(2):
+            a, b = run_both(sc, text, runs, cap)
+            assert np.array_equal(a["pos"], b["pos"]) and np.array_equal(a["col"], b["col"])
+            assert np.array_equal(a["score"].view(np.uint32), b["score"].view(np.uint32))
+        assert sc.stats().candidates < MAX_RECORDS or n < 1_000_000
