@@ -53,6 +53,11 @@ int fail(int code, const std::string& msg)
 constexpr int kNbMaxBf16 = 2;
 constexpr int kNbMaxFp32 = 4;
 
+// Filter records that the default form may leave per hit: 1.1 for motifs of 5-30
+// positions, 1.2 to 1.4 with lowercase bases, 1.6 for 24-60 positions (p = 1e-3
+// to 1e-6), with some room.
+constexpr uint64_t kRecordsPerHit = 2;
+
 template <typename T>
 struct DevBuf {
     T* p = nullptr;
@@ -852,9 +857,14 @@ int blamm_hip_reserve(blamm_hip_ctx* c, uint64_t n)
     if (c->pending) return fail(BLAMM_ERR_STATE, "reserve: a scan is in flight (call scan_finish first)");
     HIP_TRY(hipSetDevice(c->device));
     HIP_TRY(hipStreamSynchronize(c->stream));
-    HIP_TRY(c->cand.reserve(n));
     c->have_kept = false;
     HIP_TRY(c->hits.reserve(n));
+    // (the default form leaves up to kRecordsPerHit records where a caller
+    // counts one; less room only where there is not so much memory)
+    if (c->cand.reserve(kRecordsPerHit * n) != hipSuccess) {
+        (void)hipGetLastError();
+        HIP_TRY(c->cand.reserve(n));
+    }
     return BLAMM_OK;
 }
 

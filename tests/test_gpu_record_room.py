@@ -1,0 +1,52 @@
+"""Room for filter records: long motifs and lowercase bases leave the default
+form more than one record per hit, which callers that state their hits need not
+know (needs the GPU)."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import blamm_amd as ba
+from blamm_amd import synth
+from helpers import library, stream_case
+
+pytestmark = pytest.mark.gpu
+
+
+def workload(lmin, lmax, lower_every, n=1_500_000):
+    text, runs, bg = stream_case(lmin + lower_every, n, lower_every=lower_every)
+    pwms, thr = library(synth.motifs(120, lmin, lmax, 0.4, seed=lmax), bg, pvalue=1e-3)
+    P, lengths, _ = ba.build_pattern_matrix(pwms)
+    packed, lower = ba.pack(text)
+    return P, lengths, thr, packed, lower, len(text), runs
+
+
+@pytest.mark.parametrize("lmin,lmax,lower_every", [(24, 60, 0), (6, 25, 400)])
+def test_reserve_holds_a_record_per_score(lmin, lmax, lower_every):
+    """Room reserved for the records of a filter by scores (those of the
+    split-BF16 form, and a tenth more) is enough for the default form's first
+    scan."""
+    import torch
+    P, lengths, thr, packed, lower, n, runs = workload(lmin, lmax, lower_every)
+    records = 0
+    for prec in (ba.PREC_BF16X2_LO, ba.PREC_BF16X2):
+        with ba.HipScanner(0) as sc:
+            sc.set_library(P, lengths, thr, prec)
+            if records:
+                sc.reserve(int(1.1 * records))
+            else:
+                sc.reserve(1 << 23)
+            words = np.zeros(int(sc.lib.blamm_hip_packed_words(n)), np.uint64)
+            words[:packed.size] = packed
+            mask = None
+            if lower is not None:
+                mask = np.zeros(int(sc.lib.blamm_hip_mask_words(n)), np.uint64)
+                mask[:lower.size] = lower
+                mask = torch.from_numpy(mask.view(np.int64)).to("cuda:0")
+            words = torch.from_numpy(words.view(np.int64)).to("cuda:0")
+            starts = torch.from_numpy(np.asarray(runs, np.uint64).view(np.int64)).to("cuda:0")
+            hits = torch.zeros(1 << 23, dtype=torch.int64, device="cuda:0")
+            torch.cuda.synchronize()
+            sc.scan_device(words, mask, n, starts, len(runs), hits, 1 << 22, None)
+            assert sc.scan_finish() > 200_000
+            records = sc.stats().candidates
