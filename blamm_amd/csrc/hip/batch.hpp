@@ -807,13 +807,13 @@ int blamm_hip_batch_submit(blamm_hip_batch* b, const blamm_request* reqs, uint32
         HIP_TRY(hipStreamSynchronize(b->stream));
         HIP_TRY(b->off_h.reserve((size_t)nreq + 1 + nreq / 8));
     }
-    // room for the expected candidates and hits (records <= hits + rescored
-    // windows; 1.5x margin), so the batch rarely needs a second run
+    // room for the expected candidates and hits (1.5x margin), so the batch
+    // rarely needs a second run
     uint64_t expect = 0;
     for (uint32_t r = 0; r < nreq; ++r) expect += reqs[r].expected_hits;
     if (expect) {
         expect += expect / 2 + 4096;
-        BLAMM_TRY(batch_grow(b, b->cand, expect));
+        BLAMM_TRY(batch_grow(b, b->cand, c->precision == BLAMM_PREC_BF16X2 ? kRecordsPerHit * expect : expect));
         BLAMM_TRY(batch_grow(b, b->hits, expect));
         BLAMM_TRY(batch_grow(b, b->grouped, b->hits.n));
     }

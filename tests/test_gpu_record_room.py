@@ -22,6 +22,29 @@ def workload(lmin, lmax, lower_every, n=1_500_000):
 
 
 @pytest.mark.parametrize("lmin,lmax,lower_every", [(24, 60, 0), (6, 25, 400)])
+def test_batches_run_once_with_exact_expectations(lmin, lmax, lower_every):
+    """Batches whose request states the number of its hits do not grow their
+    buffers and run again, and have the scan's hits: one of 81 % of a stream,
+    then one of the whole (which has 1.5 times its hits of room from the first)."""
+    P, lengths, thr, packed, lower, n, runs = workload(lmin, lmax, lower_every)
+    with ba.HipScanner(0) as sc:
+        sc.set_library(P, lengths, thr, ba.PREC_BF16X2)
+        b = ba.Batch(sc, max_bases=n + 64, max_requests=1)
+        try:
+            for m in (81 * n // 100, n):
+                starts = [r for r in runs if r < m]
+                want = np.sort(sc.scan(packed, m, starts, lower), order=["pos", "col"])
+                assert len(want) > 200_000
+                b.submit([ba.ScanRequest(packed, m, starts, lower, None, len(want))])
+                before = b.device_bytes()
+                assert b.wait() == len(want)
+                assert b.device_bytes() == before
+                assert np.array_equal(np.sort(b.hits(0), order=["pos", "col"]), want)
+        finally:
+            b.close()
+
+
+@pytest.mark.parametrize("lmin,lmax,lower_every", [(24, 60, 0), (6, 25, 400)])
 def test_reserve_holds_a_record_per_score(lmin, lmax, lower_every):
     """Room reserved for the records of a filter by scores (those of the
     split-BF16 form, and a tenth more) is enough for the default form's first
