@@ -76,9 +76,11 @@ namespace {
 
 // Device bytes a request occupies inside a batch: its stream, mask, run
 // starts and run-start bits; its column blocks (fragments and per-slot
-// tables); its work items; and per expected hit a filter record (16 B, about
-// one per hit), a finalize output (16 B) and a grouped read-back record.
-uint64_t request_bytes(const blamm_hip_ctx* c, const blamm_request& q)
+// tables); its work items; and per expected hit a filter record (16 B), a
+// finalize output (16 B) and a grouped read-back record.  *room: what a batch
+// may take beyond that, a second record per hit and items of fewer tiles than
+// the tuned window tile (16 at least, and 2^17 items, where there are many).
+uint64_t request_bytes(const blamm_hip_ctx* c, const blamm_request& q, uint64_t* room)
 {
     const uint64_t n = q.nbases + kReqAlign;
     uint64_t active = 0;
@@ -88,8 +90,10 @@ uint64_t request_bytes(const blamm_hip_ctx* c, const blamm_request& q)
     const uint64_t tiles = n / kBf16Tile + 1;
     const uint64_t cpb = (uint64_t)std::max(1, c->cols_per_blk);
     const uint64_t blocks = (active + cpb - 1) / cpb;
-    return n / 4 + (q.lcmask ? n / 8 : 0) + 8 * (q.nruns + 1) + n / 8 + blocks * batch_block_bytes(c) +
-           8 * (tiles / std::max<uint32_t>(1, c->tuning.chunk_tiles) + 1) * c->groups.size() +
+    const uint64_t items = (tiles / std::max<uint32_t>(1, c->tuning.chunk_tiles) + 1) * c->groups.size();
+    const uint64_t fine = std::min<uint64_t>((tiles / 16 + 1) * c->groups.size(), 1ull << 17);
+    *room = 16 * hits + 8 * (std::max(items, fine) - items);
+    return n / 4 + (q.lcmask ? n / 8 : 0) + 8 * (q.nruns + 1) + n / 8 + blocks * batch_block_bytes(c) + 8 * items +
            (32 + sizeof(GroupedHit)) * hits;
 }
 
@@ -308,10 +312,12 @@ int blamm_hip_server_submit(blamm_hip_server* S, const blamm_request* q, uint64_
             if (std::isnan(q->thresholds[j])) return fail(BLAMM_ERR_ARG, "server_submit: NaN threshold");
         r.thr.assign(q->thresholds, q->thresholds + c->ncols);
     }
-    r.bytes = request_bytes(c, *q);
+    uint64_t room = 0;
+    r.bytes = request_bytes(c, *q, &room);
     if (r.bytes > S->slot_budget)
         return fail(BLAMM_ERR_ARG, "server_submit: request needs ~" + std::to_string(r.bytes) +
                                        " device bytes; the per-batch budget is " + std::to_string(S->slot_budget));
+    r.bytes += room;    // counts against company in a batch, not against the request alone
     r.t_submit = now_ns();
     {
         std::lock_guard<std::mutex> g(S->mu);

@@ -73,3 +73,19 @@ def test_reserve_holds_a_record_per_score(lmin, lmax, lower_every):
             sc.scan_device(words, mask, n, starts, len(runs), hits, 1 << 22, None)
             assert sc.scan_finish() > 200_000
             records = sc.stats().candidates
+
+
+def test_server_counts_the_second_record():
+    """Two requests that would fill a slot's budget with one record per
+    expected hit are not put into one batch; each alone is accepted."""
+    P, lengths, thr, packed, lower, n, runs = workload(6, 25, 0, n=200_000)
+    with ba.HipScanner(0) as sc:
+        sc.set_library(P, lengths, thr, ba.PREC_BF16X2)
+        srv = ba.Server(sc, hbm_budget_bytes=100_000_000, slots=1)
+        try:
+            ids = [srv.submit(ba.ScanRequest(packed, n, runs, lower, None, 1_000_000)) for _ in range(6)]
+            for i in ids:
+                assert srv.wait(i, 60_000)
+                assert srv.release(i).batch_requests == 1
+        finally:
+            srv.close()
