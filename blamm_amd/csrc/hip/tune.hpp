@@ -9,6 +9,11 @@
 
 namespace {
 
+// What a setting means and which kernels it was timed on, as part of the cache's
+// keys: a change of either takes another number, and entries of others (or of
+// none, from before there was one) are not used.
+constexpr int kTuneVersion = 2;
+
 std::string tune_key(const blamm_hip_ctx* c, uint64_t nbases, bool mask)
 {
     // FNV-1a over the column length histogram
@@ -22,7 +27,7 @@ std::string tune_key(const blamm_hip_ctx* c, uint64_t nbases, bool mask)
     int lg = 0;
     while ((1ull << (lg + 1)) <= std::max<uint64_t>(nbases, 1)) ++lg;
     std::ostringstream os;
-    os << c->arch << "/cu" << c->num_cu << "/" << (c->precision == BLAMM_PREC_BF16X2 ? "bf16x2" : c->precision == BLAMM_PREC_BF16X2_LO ? "bf16x2lo" : "fp32") << "/cols"
+    os << "t" << kTuneVersion << "/" << c->arch << "/cu" << c->num_cu << "/" << (c->precision == BLAMM_PREC_BF16X2 ? "bf16x2" : c->precision == BLAMM_PREC_BF16X2_LO ? "bf16x2lo" : "fp32") << "/cols"
        << c->ncols << "/len" << std::hex << h << std::dec << "/n2^" << lg << (mask ? "/mask" : "");
     return os.str();
 }
