@@ -93,12 +93,15 @@ int blamm_hip_autotune(blamm_hip_ctx* c, const uint64_t* d_packed, uint64_t pack
     if (tune_lookup(cache_path, key, &best, &best_ms)) {
         BLAMM_TRY(blamm_hip_set_tuning(c, &best));
     } else {
-        const uint32_t nbmax = prec_bf(c->precision) ? kNbMaxBf16 : kNbMaxFp32;
         const uint32_t ntiles = (uint32_t)((nbases + kBf16Tile - 1) / kBf16Tile);
         best_ms = 1e300;
-        // layouts at the default window tile, then window tiles for the best layout
-        for (uint32_t kp : {4u, 8u})
-            for (uint32_t nb = nbmax; nb >= 1; nb /= 2) {
+        // layouts at the default window tile, then window tiles for the best
+        // layout.  Scans of the bf16 forms pad to 16 positions whatever the
+        // setting is (8 would only add empty chunks to histograms), and the
+        // fp32 form's motif tiles 2 and 4 are the same (fp32_blocks).
+        const std::vector<uint32_t> kpads = prec_bf(c->precision) ? std::vector<uint32_t>{4u} : std::vector<uint32_t>{4u, 8u};
+        for (uint32_t kp : kpads)
+            for (uint32_t nb = 2; nb >= 1; nb /= 2) {
                 blamm_tuning t{512, nb, kp};
                 BLAMM_TRY(blamm_hip_set_tuning(c, &t));
                 double ms;
