@@ -1106,7 +1106,8 @@ void in_parts(uint64_t n, Part part)
 }
 
 // Upload a host stream into the context's staging buffers (c->packed,
-// c->lcmask, c->runs), on the context's stream.
+// c->lcmask, c->runs), on the context's stream.  Callers' arrays end with the
+// word of the last base: nothing behind it is read.
 int stage_stream(blamm_hip_ctx* c, const uint64_t* packed, const uint64_t* lcmask, uint64_t nbases,
                  const uint64_t* run_starts, uint64_t nruns)
 {

@@ -121,22 +121,23 @@ int blamm_hip_set_library(blamm_hip_ctx *ctx, const float *P, int ldp, int ncols
 int blamm_hip_library_bounds(blamm_hip_ctx *ctx, double *max_filter_band,
                              double *max_score_error);
 
-/* Words a packed-stream / lowercase-mask buffer must hold for nbases (the
- * engine reads a few words of zero padding past the end). */
+/* Words a packed-stream / lowercase-mask buffer in device memory must hold for
+ * nbases (the kernels read a few words of zero padding past the end).  Buffers
+ * in host memory need (nbases+31)/32 and (nbases+63)/64 words; the engine reads
+ * no more of them. */
 uint64_t blamm_hip_packed_words(uint64_t nbases);
 uint64_t blamm_hip_mask_words(uint64_t nbases);
 
-/* Reserve room for n filter candidates (device scratch) and, for the
- * host-buffer scans, n hits in the context's device hit buffer (16 bytes
- * each, both).  Scans grow them on demand; reserving up front keeps device
+/* Reserve room for the filter records of n hits (device scratch; 32 bytes
+ * each, 16 where there is not so much memory) and, for the host-buffer scans,
+ * n hits in the context's device hit buffer (16 bytes each).  Scans grow them on demand; reserving up front keeps device
  * allocation out of later calls and lets a first scan that fits run once.
  * BLAMM_ERR_STATE while a scan_device is in flight. */
 int blamm_hip_reserve(blamm_hip_ctx *ctx, uint64_t n);
 
-/* Scan host buffers.  packed has blamm_hip_packed_words(nbases) words; lcmask
- * is NULL when the stream has no lowercase base, else it has
- * blamm_hip_mask_words(nbases) words; run_starts are sorted.  Hits (unordered)
- * go to hits[0..cap); *nhits receives their number.  If cap is too small the
+/* Scan host buffers.  packed has (nbases+31)/32 words; lcmask is NULL when the
+ * stream has no lowercase base, else it has (nbases+63)/64 words; run_starts
+ * are sorted.  Hits (unordered) go to hits[0..cap); *nhits receives their number.  If cap is too small the
  * call returns BLAMM_ERR_OVERFLOW with *nhits = required capacity.
  * nbases < 2^32 - 512 per call. */
 int blamm_hip_scan(blamm_hip_ctx *ctx, const uint64_t *packed, const uint64_t *lcmask,

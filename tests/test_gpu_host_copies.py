@@ -3,6 +3,7 @@ array, and hits split over threads are the hits of one."""
 from __future__ import annotations
 
 import ctypes
+import mmap
 
 import numpy as np
 import pytest
@@ -91,3 +92,33 @@ def test_fetch_follows_keep():
         assert sc.lib.blamm_hip_scan_fetch(sc.ctx, room.ctypes.data, n.value) == 0
         sc.reserve(1 << 20)
         assert sc.lib.blamm_hip_scan_fetch(sc.ctx, room.ctypes.data, n.value) == ba.BLAMM_ERR_STATE
+
+
+def before_guard(a):
+    """A copy of the words `a` (whole pages) that ends where a page which cannot
+    be read begins."""
+    m = mmap.mmap(-1, a.nbytes + mmap.PAGESIZE)
+    room = np.frombuffer(m, np.uint64)
+    at = room.ctypes.data
+    room[:a.size] = a
+    assert a.nbytes % mmap.PAGESIZE == 0
+    libc = ctypes.CDLL(None, use_errno=True)
+    assert libc.mprotect(ctypes.c_void_p(at + a.nbytes), ctypes.c_size_t(mmap.PAGESIZE), 0) == 0
+    return room[:a.size]
+
+
+@pytest.mark.parametrize("n", [1 << 15, 1 << 21])
+def test_nothing_behind_the_last_base_is_read(n):
+    """Host arrays of (n + 31) / 32 and (n + 63) / 64 words are enough for
+    scans and histograms."""
+    rng = np.random.default_rng(n)
+    text, runs = stream(rng, n, 0.2)
+    codes, lower = ba.pack(text)
+    c, low = before_guard(codes[:n // 32]), before_guard(lower[:n // 64])
+    with scanner(rng, 0.01) as sc:
+        want = by_place(sc.scan(codes, n, runs, lower))
+        for scan in (sc.scan, sc.scan_pinned):
+            assert np.array_equal(by_place(scan(c, n, runs, low)), want)
+        ncols = 40
+        lo, hi = np.full(ncols, -10, np.float32), np.full(ncols, 10, np.float32)
+        assert np.array_equal(sc.hist(c, n, lo, hi, 50, runs, low), sc.hist(codes, n, lo, hi, 50, runs, lower))
