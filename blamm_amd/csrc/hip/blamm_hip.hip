@@ -53,9 +53,9 @@ int fail(int code, const std::string& msg)
 constexpr int kNbMaxBf16 = 2;
 constexpr int kNbMaxFp32 = 4;
 
-// Filter records that the default form may leave per hit: 1.1 for motifs of 5-30
-// positions, 1.2 to 1.4 with lowercase bases, 1.6 for 24-60 positions (p = 1e-3
-// to 1e-6), with some room.
+// Filter records that the default form may leave per hit, with some room: 1.05 to
+// 1.2 for motifs of 5-30 positions, 1.6 for 24-60, 1.5 to 1.75 with lowercase
+// bases (4 Mbp x 300 columns, p = 1e-3 to 1e-6; a filter by scores 1.0).
 constexpr uint64_t kRecordsPerHit = 2;
 
 template <typename T>
@@ -129,9 +129,9 @@ struct GroupInfo {
 // Scratch of blamm_hip_scan_device_noalloc: two sets of scan counters (16,896
 // bytes) and filter records of 16 bytes, 90 MiB in all.  The records are 1.4
 // times BLAMM_NOALLOC_MAX_RECORDS, so that most scans with that many records by
-// scores fit at once: the screen leaves up to 1.25 times as many for motifs of
-// 5-25 positions and 1.4 to 1.6 times as many for 24-60 (1 Mbp x 300 columns,
-// p = 1e-2 to 1e-5); the others are filtered a second time (enqueue_scan).
+// scores fit at once: the screen leaves 1.05 to 1.2 times as many for motifs of
+// 5-30 positions, 1.5 to 1.75 times for 24-60 or with lowercase bases; those
+// that do not fit are filtered a second time (enqueue_scan).
 // Every GPU the library runs on holds its own copy until the process ends; all
 // contexts on one GPU share it, so no-alloc scans that overlap on one GPU race.
 // Host code never uses the array's name as an address: the device address of
@@ -904,8 +904,8 @@ int enqueue_scan(blamm_hip_ctx* c, const uint64_t* d_packed, const uint64_t* d_l
     const bool mask = d_lcmask != nullptr;
     if (nruns == 0) run_bits = nullptr;   // nothing to search
     // How many records the screen leaves is up to its rounding, which has no
-    // bound in terms of hits (1.1 to 1.6 per hit for 5-60 positions, 3 where a
-    // pseudocount near zero makes one position's weights huge).  Where they
+    // bound in terms of hits (1.05 to 1.75 per hit, 3 where a pseudocount near
+    // zero makes one position's weights huge).  Where they
     // must fit and might not, the split-BF16 filter is launched after it and
     // runs if they did not: its records are the windows within their band of
     // the threshold.  If all is well that is a launch that ends at once.

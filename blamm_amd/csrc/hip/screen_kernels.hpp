@@ -432,7 +432,13 @@ __global__ __launch_bounds__(kThreads, LO ? 3 : 4) void screen_kernel(ScreenArgs
 // smallest expected slack s + y - alpha w under the motif's own base
 // frequencies (~2^w), which is where the slack costs candidates.  In set 1 a
 // lowercase base adds 0 to both sides, which a shift would break: weights are
-// scaled by their largest magnitude and s >= 0 covers the rounding.
+// scaled by their largest magnitude and s >= 0 covers the rounding.  s is then
+// all slack where the base is lowercase, which counts as much as the uppercase
+// bases' (rounding up has none): without that every lowercase window of a
+// 24-60 position column passes up to some bits above 0 (1 Mbp x 300 columns
+// half lowercase, p = 1e-7: 1.6 times the windows of the BF16 filter, 1.49 ms;
+// 1.0 times, 0.88 ms with it), for more records where hits are few and cost
+// nothing (5-30 positions, p = 1e-5: 1.5 for 1.24 times, 0.06 ms both).
 // ---------------------------------------------------------------------------
 struct ScreenLayoutArgs {
     const float* slot_w;      // [slot][kMaxLen][4]
@@ -517,6 +523,7 @@ static __global__ __launch_bounds__(kThreads) void screen_layout_kernel(ScreenLa
                 }
                 float slack = 0.f;
                 for (int b = 0; b < 4; ++b) slack += pi[b] * (float)(s + y[b] - x[b]);
+                if (set) slack += (pi[0] + pi[1] + pi[2] + pi[3]) * (float)s;
                 if (slack < best) {
                     best = slack;
                     best_s = s;

@@ -89,3 +89,44 @@ def test_server_counts_the_second_record():
                 assert srv.release(i).batch_requests == 1
         finally:
             srv.close()
+
+
+def lowercase_bound(w, weight):
+    """What the screen's bound of an all lowercase window of column w is above 0,
+    in weights: its layout for masked streams restated, with the slack of a
+    lowercase base counted `weight` times that of an uppercase one."""
+    def fp6(x, rounded):
+        m = np.abs(x)
+        step = np.where(m < 2, 0.125, np.where(m < 4, 0.25, 0.5))
+        return np.clip(rounded(x / step) * step, -7.5, 7.5)
+
+    w = w.astype(np.float64)
+    alpha = 7.5 / np.abs(w).max()
+    pi = 2.0 ** np.maximum(w - w.max(1, keepdims=True), -60)
+    pi /= pi.sum(1, keepdims=True)
+    slack, excess = [], []
+    for rounded in (np.rint, np.ceil):
+        y = fp6(alpha * w, rounded)
+        e = np.maximum(0.0, (alpha * w - y).max(1))
+        excess.append(e)
+        slack.append((pi * (e[:, None] + y - alpha * w)).sum(1) + weight * e)
+    return np.where(slack[1] < slack[0], excess[1], excess[0]).sum() / alpha
+
+
+def test_lowercase_windows_above_their_bound_leave_no_records():
+    """Lowercase windows score 0.  A long column's threshold need be 0.3 to 1.2
+    bits above that for the default form to rule them out, and 0.5 to 1 bit more
+    if the slack of lowercase bases did not count where weights are rounded."""
+    text, runs, bg = stream_case(8, 20_000)
+    pwms, _ = library(synth.motifs(60, 50, 60, 0.4, seed=8), bg, pvalue=1e-4)
+    thr = np.array([lowercase_bound(w, 1.0) for w in pwms]) + 0.15
+    assert np.min([lowercase_bound(w, 0.0) for w in pwms] - thr) > 0.2
+    text = (np.frombuffer(text, np.uint8) | 0x20).tobytes()
+    packed, lower = ba.pack(text)
+    P, lengths, _ = ba.build_pattern_matrix(pwms)
+    with ba.HipScanner(0) as sc:
+        sc.set_library(P, lengths, thr.astype(np.float32), ba.PREC_BF16X2)
+        sc.scan(packed, len(text), runs, lower)
+        # two records at most of each of the tiles whose windows reach the
+        # padding, which is not lowercase: 59 windows and the last tile's rest
+        assert sc.stats().candidates <= 2 * 4 * len(pwms)
