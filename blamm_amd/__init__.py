@@ -486,12 +486,21 @@ class Batch:
         _check(self.lib.blamm_hip_batch_wait(self.b, ctypes.byref(n)))
         return int(n.value)
 
+    # hits that a first call makes room for, so that requests of few (a batch
+    # has hundreds) take one call each
+    _FEW = 512
+    _few_t = ctypes.c_char * (_FEW * HIT_DTYPE.itemsize)
+
     def hits(self, req: int) -> np.ndarray:
         n = ctypes.c_uint64()
-        _check(self.lib.blamm_hip_batch_read(self.b, req, None, 0, ctypes.byref(n)))
-        hits = np.empty(n.value, dtype=HIT_DTYPE)
-        _check(self.lib.blamm_hip_batch_read(self.b, req, hits.ctypes.data, n.value, ctypes.byref(n)))
-        return hits
+        few = self._few_t()
+        rc = self.lib.blamm_hip_batch_read(self.b, req, few, self._FEW, ctypes.byref(n))
+        if rc == BLAMM_ERR_OVERFLOW:
+            hits = np.empty(n.value, dtype=HIT_DTYPE)
+            _check(self.lib.blamm_hip_batch_read(self.b, req, hits.ctypes.data, n.value, ctypes.byref(n)))
+            return hits
+        _check(rc)
+        return np.frombuffer(few, HIT_DTYPE, n.value).copy()
 
     def stats(self) -> ScanStats:
         st = ScanStats()
