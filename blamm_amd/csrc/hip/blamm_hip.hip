@@ -537,21 +537,6 @@ int relayout(blamm_hip_ctx* c)
                 }
         fb.assign(16, 0);
     }
-    std::vector<float> f3;
-    if (!bf) {
-        // [block][MFMA][lane]: lane l holds entry f = 4 i + l/16 of column
-        // l%16, the FP32 difference w[f/3][f%3] - w[f/3][T]
-        f3.assign((size_t)nblk * kFp32Rows3 * 64, 0.f);
-        for (int bi = 0; bi < nblk; ++bi)
-            for (int i = 0; i < kFp32Rows3; ++i)
-                for (int l = 0; l < 64; ++l) {
-                    const int f = 4 * i + (l >> 4);
-                    const int slot = bi * kFp32Cols + (l & 15);
-                    if (!std::isfinite(s_off3[slot])) continue;
-                    const float* w = &s_w[((size_t)slot * kMaxLen + f / 3) * 4];
-                    f3[((size_t)bi * kFp32Rows3 + i) * 64 + l] = (float)((double)w[f % 3] - (double)w[3]);
-                }
-    }
     std::vector<uint32_t> gpk(scan_groups.size());
     for (size_t g = 0; g < scan_groups.size(); ++g)
         gpk[g] = group_pack(scan_groups[g].blk0, scan_groups[g].nch, scan_groups[g].nb);
@@ -561,9 +546,8 @@ int relayout(blamm_hip_ctx* c)
     HIP_TRY(c->frag_a.reserve(fa.size()));
     HIP_TRY(c->frag_b.reserve(fb.size()));
     if (!bf) {
-        HIP_TRY(c->frag3.reserve(f3.size()));
+        HIP_TRY(c->frag3.reserve((size_t)nblk * kFp32Rows3 * 64));
         HIP_TRY(c->slot_off3.reserve(nslots));
-        HIP_TRY(hipMemcpy(c->frag3.p, f3.data(), f3.size() * sizeof(float), hipMemcpyHostToDevice));
         HIP_TRY(hipMemcpy(c->slot_off3.p, s_off3.data(), nslots * sizeof(double), hipMemcpyHostToDevice));
     }
     HIP_TRY(c->slot_thr.reserve(nslots));
@@ -610,6 +594,13 @@ int relayout(blamm_hip_ctx* c)
                            0, c->stream, a);
         HIP_TRY(hipGetLastError());
         HIP_TRY(hipStreamSynchronize(c->stream));   // scans may run on other streams
+    }
+    if (!bf) {
+        hipLaunchKernelGGL(fp32_layout_kernel, dim3((nblk * kFp32Rows3 + kWavesPerBlock - 1) / kWavesPerBlock),
+                           dim3(kThreads), 0, c->stream, c->slot_w.p, c->slot_off3.p, c->frag3.p,
+                           (uint32_t)nblk * kFp32Rows3);
+        HIP_TRY(hipGetLastError());
+        HIP_TRY(hipStreamSynchronize(c->stream));
     }
     c->nslots = nslots;
     c->cols_per_blk = cols_per_blk;

@@ -944,6 +944,21 @@ __device__ __forceinline__ void zero_counters(unsigned long long* c)
 // One block per set of counters.
 static __global__ void zero_counters_kernel(unsigned long long* c) { zero_counters(c + blockIdx.x * kCntSet); }
 
+// The FP32 form's three entries per position, one wave per MFMA of a block
+// ([block][MFMA][lane]): lane l holds entry f = 4 i + l/16 of column l%16, the
+// FP32 difference w[f/3][f%3] - w[f/3][T] (0 in a column without them: off
+// infinite).  On the host this and the upload took 0.9 ms of 4,000 columns'
+// 5.5 ms in set_library.
+static __global__ __launch_bounds__(kThreads) void fp32_layout_kernel(const float* slot_w, const double* off,
+                                                                      float* frag, uint32_t rows)
+{
+    const uint32_t row = blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6), l = threadIdx.x & 63;
+    if (row >= rows) return;
+    const uint32_t slot = row / kFp32Rows3 * kFp32Cols + (l & 15), f = 4 * (row % kFp32Rows3) + (l >> 4);
+    const float* w = slot_w + ((size_t)slot * kMaxLen + f / 3) * 4;
+    frag[(size_t)row * 64 + l] = __builtin_isfinite(off[slot]) ? (float)((double)w[f % 3] - (double)w[3]) : 0.f;
+}
+
 // Run-start bits for finalize_kernel: bit i is set when a run starts at base
 // i (0 < i < nbases).  The clear kernel zeroes words [0, nbases / 64 + 2)
 // (what load_bits64 may read below q + 1 <= nbases), and what else a scan
