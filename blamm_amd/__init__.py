@@ -500,7 +500,7 @@ class Batch:
             _check(self.lib.blamm_hip_batch_read(self.b, req, hits.ctypes.data, n.value, ctypes.byref(n)))
             return hits
         _check(rc)
-        return np.frombuffer(few, HIT_DTYPE, n.value).copy()
+        return np.frombuffer(few, HIT_DTYPE, n.value).copy() if n.value else np.zeros(0, HIT_DTYPE)
 
     def stats(self) -> ScanStats:
         st = ScanStats()

@@ -1080,6 +1080,10 @@ template <typename Part>
 void in_parts(uint64_t n, Part part)
 {
     constexpr uint64_t per = 1ull << 15;
+    if (n <= per) {
+        if (n > 0) part(0, n);
+        return;
+    }
     const uint64_t nt = std::min<uint64_t>({(n + per - 1) / per, 16ull,
                                             std::max(1u, std::thread::hardware_concurrency())});
     std::thread pool[16];
@@ -1091,7 +1095,7 @@ void in_parts(uint64_t n, Part part)
             part(b, e);
         }
     }
-    if (n > 0) part(0, n / nt);
+    part(0, n / nt);
     for (auto& th : pool)
         if (th.joinable()) th.join();
 }
