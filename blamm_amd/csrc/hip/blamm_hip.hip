@@ -127,18 +127,18 @@ struct GroupInfo {
 }  // namespace
 
 // Scratch of blamm_hip_scan_device_noalloc: two sets of scan counters (16,896
-// bytes) and filter records of 16 bytes, 90 MiB in all.  The records are 1.4
-// times BLAMM_NOALLOC_MAX_RECORDS, so that most scans with that many records by
-// scores fit at once: the screen leaves 1.05 to 1.2 times as many for motifs of
-// 5-30 positions, 1.5 to 1.75 times for 24-60 or with lowercase bases; those
-// that do not fit are filtered a second time (enqueue_scan).
+// bytes) and BLAMM_NOALLOC_MAX_RECORDS filter records of 16 bytes, 64 MiB in
+// all.  (The screen leaves 1.05 to 1.75 times as many records as a filter by
+// scores; those that do not fit are filtered a second time, enqueue_scan.  Room
+// for 1.4 times the records instead cost every process 11 ms of its 51 in
+// blamm_hip_create: the loader clears the array at 2.4 GB/s.)
 // Every GPU the library runs on holds its own copy until the process ends; all
 // contexts on one GPU share it, so no-alloc scans that overlap on one GPU race.
 // Host code never uses the array's name as an address: the device address of
 // each GPU's copy comes from hipGetSymbolAddress, taken once per device in
 // blamm_hip_create with that device current.
 constexpr uint64_t kNoAllocHeader = 2 * kCntSet * sizeof(unsigned long long);
-constexpr uint64_t kNoAllocRecords = (uint64_t)BLAMM_NOALLOC_MAX_RECORDS / 5 * 7;
+constexpr uint64_t kNoAllocRecords = BLAMM_NOALLOC_MAX_RECORDS;
 static_assert(kCntSlots <= kCntSet && kNoAllocHeader % 256 == 0, "counters exceed the scratch header");
 static __device__ __align__(256) uint8_t scratch[kNoAllocHeader + kNoAllocRecords * 16];
 
@@ -1048,9 +1048,8 @@ int blamm_hip_scan_finish(blamm_hip_ctx* c, uint64_t* nhits)
         if (c->pending_noalloc)
             return fail(BLAMM_ERR_OVERFLOW, "scan_noalloc: " + std::to_string(cnt[kCntCand]) +
                                                 " filter records, more than the no-alloc scratch holds (" +
-                                                std::to_string(kNoAllocRecords) + "; up to " +
-                                                std::to_string(BLAMM_NOALLOC_MAX_RECORDS) +
-                                                " always fit); scan a shorter stream or fewer columns per call");
+                                                std::to_string(kNoAllocRecords) +
+                                                "); scan a shorter stream or fewer columns per call");
         // Grow the scratch so that a retry holds every candidate.
         HIP_TRY(c->cand.reserve((size_t)(cnt[kCntCand] + cnt[kCntCand] / 4 + 1024)));
         return fail(BLAMM_ERR_OVERFLOW, "scan: candidate scratch overflowed (grown; retry the scan)");

@@ -184,7 +184,7 @@ int blamm_hip_scan_finish(blamm_hip_ctx *ctx, uint64_t *nhits);
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc): blamm_hip_scan_device with its scratch -- the scan
  * counters and the filter records -- in a static device array of the library
- * (90 MiB per GPU, held until the process ends) instead of context buffers.
+ * (64 MiB per GPU, held until the process ends) instead of context buffers.
  * It calls no hipMalloc/hipFree, nor does blamm_hip_scan_finish after it.
  * Arguments, result and completion (blamm_hip_scan_finish) are those of
  * blamm_hip_scan_device.  A scan fits if at most BLAMM_NOALLOC_MAX_RECORDS

@@ -160,9 +160,9 @@ def coarse_library(ncols, seed):
 @pytest.mark.parametrize("lower", [0, 7])
 @pytest.mark.parametrize("n", [800_000, 2_000_003])
 def test_noalloc_takes_scans_that_the_bound_leaves_too_many_records_of(n, lower):
-    """Records between the stated maximum and the scratch's size (800,000
-    bases), and more than fit: as long as few windows are near their
-    threshold, both scans succeed, with the hits of scan_device."""
+    """The default form leaves more records than the scratch holds, but few
+    windows are near their threshold: the scans succeed, twice in a row, with
+    the hits of scan_device."""
     import torch
     rng = np.random.default_rng(n + lower)
     text = synth.CODE2BASE[rng.integers(0, 4, n)].copy()
@@ -181,9 +181,9 @@ def test_noalloc_takes_scans_that_the_bound_leaves_too_many_records_of(n, lower)
         assert sc.scan_finish() > 1000
         records = sc.stats().candidates
         say(f"noalloc: {n} bases, {records} records of the default form")
-        assert records > MAX_RECORDS and (n < 1_000_000) == (records <= MAX_RECORDS // 5 * 7)
+        assert records > MAX_RECORDS
         for _ in range(2):
             a, b = run_both(sc, text, runs, cap)
             assert np.array_equal(a["pos"], b["pos"]) and np.array_equal(a["col"], b["col"])
             assert np.array_equal(a["score"].view(np.uint32), b["score"].view(np.uint32))
-        assert sc.stats().candidates < MAX_RECORDS or n < 1_000_000
+            assert sc.stats().candidates < MAX_RECORDS
