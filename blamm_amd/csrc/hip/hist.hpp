@@ -174,7 +174,7 @@ int blamm_hip_hist_device(blamm_hip_ctx* c, const uint64_t* d_packed, uint64_t p
     for (int pass = 0; pass < 2; ++pass)
         for (const GroupInfo& g : c->groups)
             if ((g.nch > (uint32_t)kWideChunks) == (pass == 1))
-                for (uint32_t i = 0; i < g.nb; ++i) groups.push_back(group_pack(g.blk0 + i, g.nch, clamp[g.blk0 + i] ? 2 : 1));
+                for (uint32_t i = 0; i < g.nb; ++i) groups.push_back(group_pack(g.blk0 + i, g.nch, lds && clamp[g.blk0 + i] ? 2 : 1));
     uint32_t nnarrow = 0;
     for (const GroupInfo& g : c->groups)
         if (g.nch <= (uint32_t)kWideChunks) nnarrow += g.nb;

@@ -52,7 +52,7 @@ struct HistArgs {
     const HistSlot* hs;
     const float* slot_w;           // [slot][kMaxLen][4] FP32 weights
     const uint64_t* run_starts;
-    const uint32_t* groups;        // group_pack(blk0, nch, 1 or 2): one column block per item, 2 = clamp
+    const uint32_t* groups;        // group_pack(blk0, nch, 1 or 2): one column block per item, 2 = clamp (LDS variant)
     unsigned long long* counts;    // [slot][nbins]
     unsigned long long* counters;  // kCntBand: windows binned exactly; kCntQueue: work item head
     uint32_t nbases, nruns, qend, nbins;
@@ -320,7 +320,7 @@ __global__ __launch_bounds__(kThreads, WIDE ? 2 : 4) void hist_filter_kernel(His
         __syncthreads();
 #define BLAMM_H(N) \
     case N * 8 + 1: exact += hist_range<N, MASK, LDS, false>(a, st, hist_lds, blk0, t0 + wave, t1, lane); break; \
-    case N * 8 + 2: exact += hist_range<N, MASK, LDS, true>(a, st, hist_lds, blk0, t0 + wave, t1, lane); break;
+    case N * 8 + 2: if constexpr (LDS) exact += hist_range<N, MASK, LDS, true>(a, st, hist_lds, blk0, t0 + wave, t1, lane); break;
         if constexpr (WIDE) {
             switch (nch * 8 + nb) {
                 BLAMM_H(9) BLAMM_H(10) BLAMM_H(11) BLAMM_H(12)

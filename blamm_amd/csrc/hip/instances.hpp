@@ -1,7 +1,8 @@
 // The filter and histogram kernels are compiled in translation units of their
-// own (screen.hip, filter_fp32.hip, hist_filter.hip) so that the library builds
-// in parallel; the launching code sees these declarations and leaves
-// the instantiation to those units.
+// own (screen.hip, filter_fp32.hip, hist_filter.hip, hist_filter_hbm.hip) so that
+// the library builds in parallel and a process loads only the code of the units
+// it calls (about 2 ms per MB); the launching code sees these declarations and
+// leaves the instantiation to those units.
 #pragma once
 
 #include "scan_kernels.hpp"
@@ -12,9 +13,9 @@ namespace blamm {
 
 // (lowercase mask, list form)
 #define BLAMM_SCAN_INSTANCES(X) X(false, false) X(false, true) X(true, false) X(true, true)
-#define BLAMM_HIST_INSTANCES(X)                                                             \
-    X(false, false, false) X(false, true, false) X(true, false, false) X(true, true, false) \
-    X(false, false, true) X(false, true, true) X(true, false, true) X(true, true, true)
+// (mask, LDS histograms, motifs longer than 32 positions)
+#define BLAMM_HIST_LDS_INSTANCES(X) X(false, true, false) X(true, true, false) X(false, true, true) X(true, true, true)
+#define BLAMM_HIST_HBM_INSTANCES(X) X(false, false, false) X(true, false, false) X(false, false, true) X(true, false, true)
 
 #ifndef BLAMM_INSTANTIATE
 #define BLAMM_EXTERN_SCREEN(M, L) extern template __global__ void screen_kernel<M, L, false>(ScreenArgs, WorkQueue, ListArgs);
@@ -24,7 +25,8 @@ namespace blamm {
 BLAMM_SCAN_INSTANCES(BLAMM_EXTERN_SCREEN)
 BLAMM_SCAN_INSTANCES(BLAMM_EXTERN_FP32)
 BLAMM_SCAN_INSTANCES(BLAMM_EXTERN_LO)
-BLAMM_HIST_INSTANCES(BLAMM_EXTERN_HIST)
+BLAMM_HIST_LDS_INSTANCES(BLAMM_EXTERN_HIST)
+BLAMM_HIST_HBM_INSTANCES(BLAMM_EXTERN_HIST)
 #undef BLAMM_EXTERN_SCREEN
 #undef BLAMM_EXTERN_FP32
 #undef BLAMM_EXTERN_LO
