@@ -896,10 +896,10 @@ int enqueue_scan(blamm_hip_ctx* c, const uint64_t* d_packed, const uint64_t* d_l
     if (nruns == 0) run_bits = nullptr;   // nothing to search
     // How many records the screen leaves is up to its rounding, which has no
     // bound in terms of hits (1.05 to 1.75 per hit, 3 where a pseudocount near
-    // zero makes one position's weights huge).  Where they
-    // must fit and might not, the split-BF16 filter is launched after it and
-    // runs if they did not: its records are the windows within their band of
-    // the threshold.  If all is well that is a launch that ends at once.
+    // zero makes one position's weights huge).  Where they must fit and might
+    // not, the split-BF16 filter is launched after it and runs if they did not:
+    // its records are the windows within their band of the threshold.  If all
+    // is well that is a launch that ends at once (1.5 us).
     unsigned long long* again = nullptr;
     if (c->pending_noalloc && c->precision == BLAMM_PREC_BF16X2 && c->split_finite &&
         (nbases + kBf16Tile - 1) / kBf16Tile * 2 * (uint64_t)c->nslots > cand_cap)

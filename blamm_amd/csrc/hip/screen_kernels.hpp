@@ -21,7 +21,7 @@
 // positions instead of 4.  The integers lose little: at 62.5 Mbp x 4,000
 // columns, p = 1e-5, the screen records 13.95M lanes for 13.07M hits, a filter
 // on the weights' bf16 hi terms with its proven band 14.53M (soft-masked
-// streams, set 1 of the layout below: 416k against 315k for 259k hits).
+// streams, set 1 of the layout below: 465k against 315k for 259k hits).
 //
 // What bounds it: instruction issue beside the matrix cores.  Per 32 x 32 tile
 // block a wave issues one MFMA per 16 positions (32 cycles of matrix core, 16
