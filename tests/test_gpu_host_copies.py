@@ -115,8 +115,9 @@ def test_nothing_behind_the_last_base_is_read(n):
     text, runs = stream(rng, n, 0.2)
     codes, lower = ba.pack(text)
     c, low = before_guard(codes[:n // 32]), before_guard(lower[:n // 64])
-    with scanner(rng, 0.01) as sc:
+    with scanner(rng, 0.7) as sc:
         want = by_place(sc.scan(codes, n, runs, lower))
+        assert len(want) > 100
         for scan in (sc.scan, sc.scan_pinned):
             assert np.array_equal(by_place(scan(c, n, runs, low)), want)
         ncols = 40
